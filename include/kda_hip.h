@@ -295,7 +295,9 @@ size_t kda_layer_workspace_size(int which, int B, int T, int H, int D);
  * reduction), 11-13 the segmented forward at D = 128 (bf16): 11 segment maps,
  * 12 segment start states, 13 the forward of every segment; 14 the backward's
  * state recompute and reverse carry in one launch (bf16 D = 128 without
- * segments: then ids 3 and 4 record nothing).
+ * segments: then ids 3 and 4 record nothing).  Sequences of at most 16 tokens
+ * at D <= 64 that run in one launch per direction record ids 1 and 5 only, and
+ * use no workspace (its size does not change).
  * kda_profile_read must be called after the streams have completed. */
 #define KDA_PROF_NKERNELS 15
 int kda_profile_enable(int on);              /* 1: clear records and start; 0: stop */

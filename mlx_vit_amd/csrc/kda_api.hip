@@ -604,8 +604,19 @@ int fwd_launch(int pass, const void* q, const void* k, const void* v, const void
     const int nc = (T + kda::C - 1) / kda::C, BH = B * H;
     // g_dtype doubles as the launchers' g kind: 0 fp32, 1 bf16, 2 one fp32 decay per head
     const int in_bf16 = dtype == KDA_DTYPE_BF16, g_kind = g_dtype;
-    hipError_t e =
-        launch_prep_pass(pass, q, k, v, g, beta, ws, T, H, D, BH * nc, in_bf16, g_kind, st, prof, dio);
+    hipError_t e;
+    if (kda::short_sequences(T, D, in_bf16, BH)) {
+        kda::ShortArgs sa = {};
+        sa.q = q; sa.k = k; sa.v = v; sa.g = g; sa.beta = beta; sa.s0 = s0;
+        sa.o = o; sa.s_final = s_final;
+        sa.T = T; sa.H = H; sa.BH = BH;
+        if (epi) {
+            sa.z = epi->z; sa.ld_z = epi->ld_z; sa.nw = epi->w; sa.eps = epi->eps; sa.y = epi->y; sa.ld_y = epi->ld_y;
+        }
+        e = timed(PROF_RECUR_FWD, st, [&] { return kda::launch_short(sa, D, in_bf16, g_kind, false, st); }, prof);
+        return e == hipSuccess ? ok() : hip_fail(e, "kda_short_fwd_kernel");
+    }
+    e = launch_prep_pass(pass, q, k, v, g, beta, ws, T, H, D, BH * nc, in_bf16, g_kind, st, prof, dio);
     if (e != hipSuccess) return hip_fail(e, "kda_prep_kernel");
 
     int nseg, seg_len;
@@ -714,6 +725,14 @@ int bwd_launch(int pass, const void* q, const void* k, const void* v, const void
     const int nc = (T + kda::C - 1) / kda::C, BH = B * H;
     const int in_bf16 = dtype == KDA_DTYPE_BF16, g_kind = g_dtype;
     hipError_t e;
+    if (kda::short_sequences(T, D, in_bf16, BH)) {
+        kda::ShortArgs sa = {};
+        sa.q = q; sa.k = k; sa.v = v; sa.g = g; sa.beta = beta; sa.dout = dout; sa.s0 = s0; sa.dsf = ds_final;
+        sa.dq = dq; sa.dk = dk; sa.dv = dv; sa.dg = dg; sa.dbeta = dbeta; sa.ds0 = ds0;
+        sa.T = T; sa.H = H; sa.BH = BH;
+        e = timed(PROF_LOCAL, st, [&] { return kda::launch_short(sa, D, in_bf16, g_kind, true, st); });
+        return e == hipSuccess ? ok() : hip_fail(e, "kda_short_bwd_kernel");
+    }
     if (pass == KDA_PASS_BWD) {
         e = launch_prep_pass(pass, q, k, v, g, beta, ws, T, H, D, BH * nc, in_bf16, g_kind, st, true, dio);
         if (e != hipSuccess) return hip_fail(e, "kda_prep_kernel");

@@ -115,6 +115,25 @@ hipError_t launch_seg_states(const SegArgs& a, hipStream_t st);
 // all_maps, segX the reverse maps), written to segS[s].
 hipError_t launch_seg_rscan(const SegArgs& a, hipStream_t st);
 
+// Sequences of at most SHORT_MAX_T tokens (kda_short.hip), forward and adjoint,
+// from the op's inputs to its outputs with no workspace.  y set: the layer's
+// gated RMSNorm fused (as RecurArgs); s0, s_final, dsf, ds0 may be null.
+constexpr int SHORT_MAX_T = 16;
+struct ShortArgs {
+    const void *q, *k, *v, *g, *beta, *dout;
+    const float *s0, *dsf;
+    void *o, *dq, *dk, *dv, *dg, *dbeta;
+    float *s_final, *ds0;
+    const void* z;
+    const float* nw;
+    void* y;
+    int64_t ld_z, ld_y;
+    float eps;
+    int T, H, BH;
+};
+bool short_sequences(int T, int D, int in_bf16, int BH);
+hipError_t launch_short(const ShortArgs& a, int D, int in_bf16, int g_kind, bool bwd, hipStream_t st);
+
 // Compute-unit count of device `dev` (0 if it cannot be queried), looked up
 // once per device under std::call_once, so concurrent callers are safe.
 int device_cu_count(int dev);

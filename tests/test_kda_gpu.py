@@ -849,3 +849,57 @@ def test_random_sweep(case):
         if gr is not None and refb.get(n) is not None:
             errs["t_" + n] = R.rel_l2(gr.cpu(), refb[n])
     _assert_all(errs, TOL[dtype], f"random sweep {case}")
+
+
+# ---------------------------------------------------------------- short sequences
+
+SHORT_CASES = [(T, D, dtype, g, decay) for T, D in ((1, 64), (7, 64), (8, 32), (8, 64), (9, 64), (15, 32), (16, 64))
+               for dtype, g, decay in ((torch.bfloat16, torch.bfloat16, "mild"), (torch.bfloat16, torch.float32, "layer"),
+                                       (torch.float32, torch.float32, "layer"), (torch.float32, torch.float32, "mixed"),
+                                       (torch.bfloat16, "head", "mild"))]
+
+
+@pytest.mark.parametrize("T,D,dtype,g_kind,decay", SHORT_CASES)
+def test_short_sequences(T, D, dtype, g_kind, decay):
+    """Sequences of at most 16 tokens (one wave each, no workspace), forward and
+    backward, with and without a state and a final-state cotangent, at the edges
+    of the 8- and 16-row variants; 5 x 3 sequences (87 x 3 where bf16 at D = 64 runs
+    there only above 256) leave the last workgroup partly empty.  "mixed": decays of both signs, one of them below the kernel's
+    floor.  All arithmetic is fp32, so a bf16 result is off by its own rounding
+    (2^-8 an element at most) and an fp32 one by the rounding of the cumsums in
+    the exponents (at most 2^8 in log2 units at the layer's decay: 2^8 * 2^-24)."""
+    kda = _kda()
+    B, H = (5 if T <= 8 or D == 32 or dtype == torch.float32 else 87), 3
+    x = R.make_inputs(B, T, H, D, dtype=dtype, seed=T + D, with_state=True, with_grad=True)
+    gen = torch.Generator().manual_seed(T)
+    if decay == "layer":
+        x["g"] = -torch.linspace(1, 16, H).reshape(H, 1) * torch.nn.functional.softplus(
+            0.5 * torch.randn(B, T, H, D, generator=gen))
+    elif decay == "mixed":
+        x["g"] = 0.2 * torch.randn(B, T, H, D, generator=gen)
+        x["g"][:, T // 2, 0] = -1e30
+    if g_kind == "head":
+        gh = x["g"][..., 0].float().contiguous()
+        x["g"] = gh.unsqueeze(-1).expand(B, T, H, D).contiguous()
+    else:
+        x["g"] = x["g"].to(g_kind)
+    ga = gh if g_kind == "head" else x["g"]
+    dsf = torch.randn(B, H, D, D, generator=gen)
+    tol = 2.0 ** -8 if dtype == torch.bfloat16 else 2e-5
+    for s0, ds in ((None, None), (x["s0"], dsf), (x["s0"], None), (None, dsf)):
+        args = [x["q"].to(DEV), x["k"].to(DEV), x["v"].to(DEV), ga.to(DEV), x["beta"].to(DEV),
+                None if s0 is None else s0.to(DEV)]
+        o, sf, ws = kda.kda_forward_train(*args)
+        got = kda.kda_backward_train(*args, x["do"].to(DEV), None if ds is None else ds.to(DEV), ws)
+        torch.cuda.synchronize()
+        ref = cref.forward(x["q"], x["k"], x["v"], x["g"], x["beta"], s0)
+        refb = cref.backward(x["q"], x["k"], x["v"], x["g"], x["beta"], s0, x["do"], ds)
+        if g_kind == "head":
+            refb["dg"] = refb["dg"].sum(-1)
+        errs = {"o": R.rel_l2(o.cpu(), ref["o"]), "s_final": R.rel_l2(sf.cpu(), ref["s_final"])}
+        for n, a in zip(("dq", "dk", "dv", "dg", "dbeta", "ds0"), got):
+            if refb[n].abs().max() == 0:      # T = 1 without a state: no decay gradient
+                assert a.abs().max() == 0, n
+            else:
+                errs[n] = R.rel_l2(a.cpu(), refb[n])
+        _assert_all(errs, tol, f"short T={T} D={D} {dtype} g={g_kind} {decay} s0={s0 is not None} dsf={ds is not None}")
