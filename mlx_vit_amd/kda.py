@@ -193,17 +193,20 @@ def kda_forward_train(q, k, v, g, beta, initial_state=None, chunk_size: int = CH
 
 
 def kda_backward_train(q, k, v, g, beta, initial_state, do, ds_final, workspace: torch.Tensor,
-                       chunk_size: int = CHUNK):
+                       chunk_size: int = CHUNK, _need_ds0: bool = True):
     """VJP from the workspace of ``kda_forward_train`` (same inputs): returns
     (dq, dk, dv, dg, dbeta, d_initial_state).  A workspace of the pair's whole
     size also serves as the backward's scratch; a kept-part one gets a scratch
     buffer allocated for the call."""
-    return kda_backward(q, k, v, g, beta, initial_state, do, ds_final, chunk_size, workspace, _train=True)
+    return kda_backward(q, k, v, g, beta, initial_state, do, ds_final, chunk_size, workspace, _train=True,
+                        _need_ds0=_need_ds0)
 
 
 def kda_backward(q, k, v, g, beta, initial_state, do, ds_final=None, chunk_size: int = CHUNK,
-                 workspace: Optional[torch.Tensor] = None, _train: bool = False):
-    """VJP of ``kda_forward``: returns (dq, dk, dv, dg, dbeta, d_initial_state)."""
+                 workspace: Optional[torch.Tensor] = None, _train: bool = False, _need_ds0: bool = True):
+    """VJP of ``kda_forward``: returns (dq, dk, dv, dg, dbeta, d_initial_state).
+    ``_need_ds0=False`` (the autograd nodes without an initial state) leaves
+    the last one out."""
     _check_chunk(chunk_size)
     q, k, v, g, beta, s0 = _prepare(q, k, v, g, beta, initial_state)
     B, T, H, D = q.shape
@@ -224,7 +227,7 @@ def kda_backward(q, k, v, g, beta, initial_state, do, ds_final=None, chunk_size:
     dev = q.device
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     dg, dbeta = torch.empty_like(g), torch.empty_like(beta)
-    ds0 = torch.empty((B, H, D, D), dtype=torch.float32, device=dev)
+    ds0 = torch.empty((B, H, D, D), dtype=torch.float32, device=dev) if _need_ds0 else None
     if _train and workspace is None:
         raise ValueError("kda_backward_train needs the workspace returned by kda_forward_train")
     ws = _workspace(_lib.KDA_PASS_BWD, B, T, H, D, dev, q.dtype, workspace)
@@ -309,7 +312,9 @@ class ChunkKDAFunction(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, g, beta, initial_state)
         ctx.ws = ws
         ctx.chunk_size = chunk_size
-        ctx.has_state = initial_state is not None
+        ctx.need_ds0 = ctx.needs_input_grad[5]
+        # an unused output's cotangent comes as None, not as a (B, H, D, D) of zeros to fill and read
+        ctx.set_materialize_grads(False)
         return o, s_final
 
     @staticmethod
@@ -319,12 +324,12 @@ class ChunkKDAFunction(torch.autograd.Function):
             do = torch.zeros_like(q)
         if ctx.ws is not None:
             dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws,
-                                                            ctx.chunk_size)
+                                                            ctx.chunk_size, _need_ds0=ctx.need_ds0)
             ctx.ws = None
         else:
-            dq, dk, dv, dg, dbeta, ds0 = kda_backward(q, k, v, g, beta, s0, do, ds_final, ctx.chunk_size)
-        return (dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), dg.to(g.dtype), dbeta.to(beta.dtype),
-                ds0 if ctx.has_state else None, None)
+            dq, dk, dv, dg, dbeta, ds0 = kda_backward(q, k, v, g, beta, s0, do, ds_final, ctx.chunk_size,
+                                                      _need_ds0=ctx.need_ds0)
+        return (dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), dg.to(g.dtype), dbeta.to(beta.dtype), ds0, None)
 
 
 def chunk_kda(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, beta: torch.Tensor,

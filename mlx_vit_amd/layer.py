@@ -276,7 +276,8 @@ class ChunkKDAGatedFunction(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, g, beta, initial_state, o, gate, norm_weight)
         ctx.ws = ws if train else None
         ctx.eps = eps
-        ctx.has_state = initial_state is not None
+        ctx.need_ds0 = ctx.needs_input_grad[5]
+        ctx.set_materialize_grads(False)   # no zeros for an unused final state's cotangent
         return y, s_final
 
     @staticmethod
@@ -286,12 +287,13 @@ class ChunkKDAGatedFunction(torch.autograd.Function):
             dy = torch.zeros(gate.shape, dtype=o.dtype, device=o.device)
         do, dz, dw = gated_rmsnorm_backward(o, gate, w, ctx.eps, dy)
         if ctx.ws is not None:
-            dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws)
+            dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws,
+                                                            _need_ds0=ctx.need_ds0)
             ctx.ws = None
         else:
-            dq, dk, dv, dg, dbeta, ds0 = kda_backward(q, k, v, g, beta, s0, do, ds_final)
+            dq, dk, dv, dg, dbeta, ds0 = kda_backward(q, k, v, g, beta, s0, do, ds_final, _need_ds0=ctx.need_ds0)
         return (dq.to(q.dtype), dk.to(k.dtype), dv.to(v.dtype), dg.to(g.dtype), dbeta.to(beta.dtype),
-                ds0 if ctx.has_state else None, dz.to(gate.dtype), dw.to(w.dtype), None)
+                ds0, dz.to(gate.dtype), dw.to(w.dtype), None)
 
 
 class ShortCausalConv1d(nn.Module):
