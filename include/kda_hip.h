@@ -279,6 +279,42 @@ int kda_layer_gated_rmsnorm_bwd(const void* o, const void* z, int64_t ld_z, cons
                                 int rows, int H, int D, float eps, int dtype,
                                 void* workspace, size_t ws_bytes, void* stream);
 
+/* Weight gradients of linear maps y = x W^T (+ b), one launch for up to
+ * KDA_WGRAD_MAX_PROBLEMS of them over the same rows:
+ *   dw[i][j] = sum_r dy[r][i] x[r][j],  db[i] = sum_r dy[r][i] (db may be NULL)
+ * bf16 dy, x, dw and db, fp32 sums in a fixed order.  dy: rows of ld_dy, n
+ * columns; x: rows of ld_x, k columns; dw [n][k] and db [n] contiguous.  k a
+ * multiple of 8; ld_dy and ld_x multiples of 8 that cover n and k rounded up to
+ * 8; dy, x and dw 16-byte aligned.  rows >= 1; workspace: at least
+ * kda_weight_grad_workspace_size bytes (may be 0), 16-byte aligned.  No
+ * counterpart in the reference, whose framework forms them (the gradients of
+ * the nn.Linear maps of GatedDeltaLayer, nope_gdn_mlx.py:736-772). */
+#define KDA_WGRAD_MAX_PROBLEMS 8
+typedef struct kda_wgrad_problem {
+    const void* dy;
+    const void* x;
+    void* dw;
+    void* db;
+    int64_t ld_dy, ld_x;
+    int64_t n, k;
+} kda_wgrad_problem;
+size_t kda_weight_grad_workspace_size(const kda_wgrad_problem* problems, int count, int rows);
+int kda_weight_grad(const kda_wgrad_problem* problems, int count, int rows, void* workspace, size_t ws_bytes,
+                    void* stream);
+
+/* Copies with conversion, one launch: job j writes dst[i] = src[i], i < n, from
+ * dtype (dtypes & 255) to dtype (dtypes >> 8), 0 fp32 or 1 bf16.  At most
+ * KDA_PACK_MAX_JOBS jobs; they must not overlap.  It lays a layer's parameters
+ * out for its GEMMs and kernels, and their gradients back. */
+#define KDA_PACK_MAX_JOBS 24
+typedef struct kda_pack_job {
+    const void* src;
+    void* dst;
+    int64_t n;
+    int64_t dtypes;
+} kda_pack_job;
+int kda_layer_pack(const kda_pack_job* jobs, int count, void* stream);
+
 #define KDA_LAYER_PRODUCER 0
 #define KDA_LAYER_RMSNORM 1
 size_t kda_layer_workspace_size(int which, int B, int T, int H, int D);

@@ -55,6 +55,9 @@ SIGNATURES = {
                                + [_I] * 2 + [_P, _Z, _P], _I),
     "kda_layer_gated_rmsnorm_fwd": ([_P, _P, _L, _P, _P, _L] + [_I] * 3 + [_F, _I, _P], _I),
     "kda_layer_gated_rmsnorm_bwd": ([_P, _P, _L, _P, _P, _L, _P, _P, _L, _P] + [_I] * 3 + [_F, _I, _P, _Z, _P], _I),
+    "kda_weight_grad_workspace_size": ([_P, _I, _I], _Z),
+    "kda_weight_grad": ([_P, _I, _I, _P, _Z, _P], _I),
+    "kda_layer_pack": ([_P, _I, _P], _I),
     "kda_layer_workspace_size": ([_I] * 5, _Z),
     "kda_profile_enable": ([_I], _I),
     "kda_profile_name": ([_I], ctypes.c_char_p),

@@ -1221,6 +1221,62 @@ int kda_layer_gated_rmsnorm_bwd(const void* o, const void* z, int64_t ld_z, cons
     return e == hipSuccess ? ok() : hip_fail(e, "kda_layer_gated_rmsnorm_bwd");
 }
 
+size_t kda_weight_grad_workspace_size(const kda_wgrad_problem* problems, int count, int rows) {
+    if (!problems || count < 1 || count > KDA_WGRAD_MAX_PROBLEMS || rows < 1) return 0;
+    for (int j = 0; j < count; ++j)
+        if (problems[j].n < 1 || problems[j].k < 1 || problems[j].n > (1 << 20) || problems[j].k > (1 << 20)) return 0;
+    return kda::wgrad_ws_floats(reinterpret_cast<const kda::WgradProblem*>(problems), count, rows) * sizeof(float);
+}
+
+int kda_weight_grad(const kda_wgrad_problem* problems, int count, int rows, void* workspace, size_t ws_bytes,
+                    void* stream) {
+    static_assert(sizeof(kda_wgrad_problem) == sizeof(kda::WgradProblem), "one layout");
+    static_assert(KDA_WGRAD_MAX_PROBLEMS == kda::WGRAD_MAX_PROBLEMS, "one limit");
+    if (!problems) return fail(KDA_E_INVALID, "problems is NULL");
+    if (count < 1 || count > KDA_WGRAD_MAX_PROBLEMS)
+        return fail(KDA_E_INVALID, "count=%d: expected 1 to %d problems", count, KDA_WGRAD_MAX_PROBLEMS);
+    if (rows < 1) return fail(KDA_E_INVALID, "rows=%d", rows);
+    for (int j = 0; j < count; ++j) {
+        const kda_wgrad_problem& p = problems[j];
+        if (!p.dy || !p.x || !p.dw) return fail(KDA_E_INVALID, "problem %d: dy, x and dw must be non-NULL", j);
+        if (!aligned(p.dy, 16) || !aligned(p.x, 16) || !aligned(p.dw, 16))
+            return fail(KDA_E_INVALID, "problem %d: dy, x and dw must be 16-byte aligned", j);
+        if (p.n < 1 || p.n > (1 << 20) || p.k < 8 || p.k > (1 << 20) || p.k % 8 != 0)
+            return fail(KDA_E_UNSUPPORTED, "problem %d: n=%lld, k=%lld (k must be a multiple of 8)", j, (long long)p.n,
+                        (long long)p.k);
+        // a step's 32 rows are addressed with 32-bit byte offsets
+        if (p.ld_dy % 8 != 0 || p.ld_x % 8 != 0 || p.ld_dy < ((p.n + 7) & ~(int64_t)7) || p.ld_x < p.k ||
+            p.ld_dy > (1 << 24) || p.ld_x > (1 << 24))
+            return fail(KDA_E_INVALID, "problem %d: ld_dy=%lld, ld_x=%lld", j, (long long)p.ld_dy, (long long)p.ld_x);
+    }
+    const size_t need = kda_weight_grad_workspace_size(problems, count, rows);
+    if (need > 0) {
+        if (!workspace) return fail(KDA_E_INVALID, "workspace is NULL");
+        if (!aligned(workspace, 16)) return fail(KDA_E_INVALID, "workspace is not 16-byte aligned");
+        if (ws_bytes < need) return fail(KDA_E_WORKSPACE, "workspace has %zu bytes, needs %zu", ws_bytes, need);
+    }
+    const hipError_t e = kda::launch_wgrad(reinterpret_cast<const kda::WgradProblem*>(problems), count, rows,
+                                           static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? ok() : hip_fail(e, "kda_weight_grad");
+}
+
+int kda_layer_pack(const kda_pack_job* jobs, int count, void* stream) {
+    static_assert(sizeof(kda_pack_job) == sizeof(kda::PackJob), "one layout");
+    static_assert(KDA_PACK_MAX_JOBS == kda::PACK_MAX_JOBS, "one limit");
+    if (count < 0 || count > KDA_PACK_MAX_JOBS || (count > 0 && !jobs))
+        return fail(KDA_E_INVALID, "count=%d: expected 0 to %d jobs", count, KDA_PACK_MAX_JOBS);
+    for (int j = 0; j < count; ++j) {
+        const int64_t sd = jobs[j].dtypes & 255, dd = jobs[j].dtypes >> 8;
+        if (sd > 1 || dd < 0 || dd > 1) return fail(KDA_E_UNSUPPORTED, "job %d: dtypes=%lld", j, (long long)jobs[j].dtypes);
+        if (jobs[j].n < 0 || jobs[j].n > ((int64_t)1 << 32)) return fail(KDA_E_INVALID, "job %d: n=%lld", j, (long long)jobs[j].n);
+        if (jobs[j].n == 0) continue;
+        if (!jobs[j].src || !jobs[j].dst || !aligned(jobs[j].src, sd ? 2 : 4) || !aligned(jobs[j].dst, dd ? 2 : 4))
+            return fail(KDA_E_INVALID, "job %d: src or dst is NULL or misaligned", j);
+    }
+    const hipError_t e = kda::launch_pack(reinterpret_cast<const kda::PackJob*>(jobs), count, static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? ok() : hip_fail(e, "kda_layer_pack");
+}
+
 size_t kda_layer_workspace_size(int which, int B, int T, int H, int D) {
     if (B < 0 || T < 0 || H < 1 || D < 1) return 0;
     if (which == KDA_LAYER_PRODUCER) return kda::producer_ws_floats(B, T, H, D) * sizeof(float);

@@ -181,6 +181,24 @@ int api_fwd_on_workspace(const void* q, const void* k, const void* v, const void
                          const float* s0, void* o, float* s_final, int B, int T, int H, int D, int chunk, int dtype,
                          int g_dtype, void* workspace, size_t ws_bytes, void* stream);
 
+// Weight gradients and the batched conversion copy (kda_wgrad.hip); the
+// fields of kda_wgrad_problem and kda_pack_job
+constexpr int WGRAD_MAX_PROBLEMS = 8;
+struct WgradProblem {
+    const void *dy, *x;
+    void *dw, *db;
+    int64_t ld_dy, ld_x, n, k;
+};
+size_t wgrad_ws_floats(const WgradProblem* q, int count, int rows);
+hipError_t launch_wgrad(const WgradProblem* q, int count, int rows, float* part, hipStream_t st);
+constexpr int PACK_MAX_JOBS = 24;
+struct PackJob {
+    const void* src;
+    void* dst;
+    int64_t n, dtypes;
+};
+hipError_t launch_pack(const PackJob* jobs, int count, hipStream_t st);
+
 // GatedDeltaLayer producer (projection outputs -> q, k, v, g, beta) and its
 // adjoint.  Row strides are in elements; q, k, v, g, dq, dk, dv, dg are
 // contiguous [B, T, H*D], beta and dbeta contiguous [B, T, H].

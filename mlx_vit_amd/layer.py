@@ -26,6 +26,7 @@ adjoint; there is no CPU path.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Optional, Tuple
 
@@ -123,9 +124,11 @@ def producer_forward(qkv: torch.Tensor, xf: torch.Tensor, xb: torch.Tensor, conv
 
 
 def producer_backward(qkv, xf, xb, conv_w, conv_b, dt_bias, A_log, dq, dk, dv, dg, dbeta,
-                      num_heads: int, head_dim: int, scale: float, beta_mult: float = 1.0):
+                      num_heads: int, head_dim: int, scale: float, beta_mult: float = 1.0,
+                      _dqkv: Optional[torch.Tensor] = None, _dxb: Optional[torch.Tensor] = None):
     """VJP of ``producer_forward``: returns (dqkv, dxf, dxb, dconv_w, dconv_b,
-    ddt_bias, dA_log); the parameter gradients are fp32."""
+    ddt_bias, dA_log); the parameter gradients are fp32.  ``_dqkv`` and ``_dxb``:
+    where to write dqkv and dxb, column slices of one (B, T, *) buffer."""
     H, D = num_heads, head_dim
     HD = H * D
     dt = qkv.dtype
@@ -154,8 +157,8 @@ def producer_backward(qkv, xf, xb, conv_w, conv_b, dt_bias, A_log, dq, dk, dv, d
         dA = torch.empty((H,), **f32)
     else:
         dg = dt_bias = A_log = dxf = ddt = dA = None
-    dqkv = torch.empty((B, T, 3 * HD), dtype=dt, device=dev)
-    dxb = torch.empty((B, T, H), dtype=dt, device=dev)
+    dqkv = torch.empty((B, T, 3 * HD), dtype=dt, device=dev) if _dqkv is None else _dqkv
+    dxb = torch.empty((B, T, H), dtype=dt, device=dev) if _dxb is None else _dxb
     dconv_w = torch.empty((3, HD, CONV_TAPS), **f32)
     dconv_b = None if conv_b is None else torch.empty((3, HD), **f32)
     lib = _lib.load()
@@ -167,7 +170,8 @@ def producer_backward(qkv, xf, xb, conv_w, conv_b, dt_bias, A_log, dq, dk, dv, d
         base, base + HD * es, base + 2 * HD * es, _ptr(xf), _ptr(xb), ld_x, ld_f, ld_b,
         _ptr(conv_w), _ptr(conv_b), _ptr(dt_bias), _ptr(A_log),
         _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dg), _ptr(dbeta),
-        dbase, dbase + HD * es, dbase + 2 * HD * es, _ptr(dxf), _ptr(dxb), 3 * HD, HD if gate else 0, H,
+        dbase, dbase + HD * es, dbase + 2 * HD * es, _ptr(dxf), _ptr(dxb), _rows(dqkv, "dqkv"),
+        HD if gate else 0, _rows(dxb, "dxb"),
         _ptr(dconv_w), _ptr(dconv_b), _ptr(ddt), _ptr(dA),
         B, T, H, D, float(scale), float(beta_mult), _DTYPE_CODE[dt], _DTYPE_CODE[g_dtype],
         _ptr(ws), ws.numel(), _stream(dev))
@@ -211,6 +215,37 @@ def gated_rmsnorm_backward(o, z, weight, eps, dy):
                                          _DTYPE_CODE[o.dtype], _ptr(ws), ws.numel(), _stream(dev))
     _lib.check(rc, "kda_layer_gated_rmsnorm_bwd")
     return do, dz, dw
+
+
+def _i64(rows) -> ctypes.Array:
+    """The rows' integers (addresses, sizes) as one C array of 64-bit fields."""
+    flat = [v for r in rows for v in r]
+    return (ctypes.c_int64 * len(flat))(*flat)
+
+
+def weight_grads(problems, rows: int):
+    """Weight gradients of linear maps over the same ``rows`` rows, in one
+    launch: for each (dy, x, bias) with dy (rows, n) and x (rows, k) bf16, rows
+    at even strides, dw = dy^T x (n, k) and, with ``bias``, db = sum of dy's rows
+    (n,).  Returns [(dw, db or None), ...]."""
+    out, fields = [], []
+    dev = problems[0][0].device
+    for dy, x, bias in problems:
+        for name, t in (("dy", dy), ("x", x)):
+            if t.dim() != 2 or t.shape[0] != rows or t.dtype != torch.bfloat16 or t.stride(1) != 1 or t.device != dev:
+                raise ValueError(f"{name} must be a ({rows}, n) bfloat16 matrix with unit column stride on {dev}")
+        n, k = dy.shape[1], x.shape[1]
+        dw = torch.empty((n, k), dtype=torch.bfloat16, device=dev)
+        db = torch.empty((n,), dtype=torch.bfloat16, device=dev) if bias else None
+        out.append((dw, db))
+        fields.append((dy.data_ptr(), x.data_ptr(), dw.data_ptr(), 0 if db is None else db.data_ptr(),
+                       dy.stride(0), x.stride(0), n, k))
+    lib = _lib.load()
+    arr = _i64(fields)
+    nws = lib.kda_weight_grad_workspace_size(arr, len(fields), rows)
+    ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dev)
+    _lib.check(lib.kda_weight_grad(arr, len(fields), rows, _ptr(ws), ws.numel(), _stream(dev)), "kda_weight_grad")
+    return out
 
 
 class ProducerFunction(torch.autograd.Function):
@@ -414,9 +449,9 @@ class GatedDeltaLayer(nn.Module):
                 compute_path: Optional[str] = None) -> Tuple[torch.Tensor, torch.Tensor]:
         if x.dim() != 3 or x.shape[-1] != self.hidden_size:
             raise ValueError(f"x must be (B, L, {self.hidden_size}); got {tuple(x.shape)}")
+        path = compute_path or self.compute_path
         q, k, v, g, beta = self.produce(x)
         gate = self.g_proj_2(self.g_proj_1(x))
-        path = compute_path or self.compute_path
         if (self.fused_output_norm and path == HIP_PATH and self.channel_wise_decay and gate.dtype == q.dtype
                 and gated_supported(self.head_dim, q.dtype)):
             y, new_state = ChunkKDAGatedFunction.apply(q, k, v, g, beta, state, gate, self.o_norm.weight,

@@ -412,3 +412,28 @@ def test_layer_parity_scalar_alpha():
     for n, p in layer.named_parameters():
         errs["d" + n] = _rel(p.grad, rp[n].grad)
     _check(errs, TOL[torch.float32], "layer scalar alpha")
+
+
+@pytest.mark.parametrize("rows,shapes", [
+    (1, [(8, 8, True)]), (31, [(12, 64, True)]), (33, [(64, 72, False), (12, 8, True)]),
+    (224, [(130, 192, True)]), (257, [(128, 128, False), (200, 64, True), (300, 136, True)]),
+    (3000, [(140, 128, True), (64, 256, False)])])
+def test_weight_grads_parity(rows, shapes):
+    """weight_grads against the fp32 products: one and several problems, tails of
+    the 32-row steps, of the 128 and 64 wide tiles and of the row splits (one
+    split below 512 rows).  fp32 sums of bf16 operands rounded once: 2^-8 an
+    element at most.  dy as a column slice of a wider matrix."""
+    from mlx_vit_amd.layer import weight_grads
+    gen = torch.Generator().manual_seed(rows)
+    probs = []
+    for n, k, bias in shapes:
+        wide = torch.randn(rows, -(-n // 8) * 8 + 16, generator=gen).to(torch.bfloat16).to(DEV)
+        probs.append((wide[:, 8:8 + n], torch.randn(rows, k, generator=gen).to(torch.bfloat16).to(DEV), bias))
+    got = weight_grads(probs, rows)
+    torch.cuda.synchronize()
+    for (dy, x, bias), (dw, db) in zip(probs, got):
+        ref = {"dw": dy.double().cpu().T @ x.double().cpu(), "db": dy.double().cpu().sum(0)}
+        errs = {"dw": _rel(dw, ref["dw"])}
+        if bias:
+            errs["db"] = _rel(db, ref["db"])
+        _check(errs, 2.0 ** -8, f"weight_grads rows={rows} n={dy.shape[1]} k={x.shape[1]}")
