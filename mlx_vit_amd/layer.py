@@ -37,6 +37,7 @@ import torch.nn.functional as F
 from . import _lib
 from .kda import (BWD_HEAD_DIMS, CHUNK, FWD_HEAD_DIMS, _DTYPE_CODE, _ptr, _stream, gated_supported,
                   kda_backward, kda_backward_train, kda_forward_gated)
+from .layer_fused import fused_layer, fused_params
 from .recurrence import GDN_HIP_PATH, HIP_PATH, KDARecurrence
 
 CONV_TAPS = 4
@@ -450,6 +451,13 @@ class GatedDeltaLayer(nn.Module):
         if x.dim() != 3 or x.shape[-1] != self.hidden_size:
             raise ValueError(f"x must be (B, L, {self.hidden_size}); got {tuple(x.shape)}")
         path = compute_path or self.compute_path
+        if (self.channel_wise_decay and path == HIP_PATH and not self.fused_output_norm
+                and type(self.recurrence) is KDARecurrence):
+            params = fused_params(self, x, state)
+            if params is not None:
+                spec = (self.num_heads, self.head_dim, self.scale, 2.0 if self.allow_neg_eigval else 1.0,
+                        self.o_norm.eps, self.chunk_size)
+                return fused_layer(x, state, spec, params)
         q, k, v, g, beta = self.produce(x)
         gate = self.g_proj_2(self.g_proj_1(x))
         if (self.fused_output_norm and path == HIP_PATH and self.channel_wise_decay and gate.dtype == q.dtype

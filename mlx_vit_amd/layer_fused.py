@@ -1,0 +1,209 @@
+"""The bf16 channel-wise ``GatedDeltaLayer`` as one autograd node.
+
+The layer is launch-bound between its kernels: as separate torch modules it is
+about 80 launches and 20 autograd nodes forward and backward, 1.0 to 1.5 ms of
+host time, as long as its GPU work at 8 clips.  Here
+
+* the six maps that read x (q, k, v, f_proj_1, g_proj_1, b_proj) are one GEMM on
+  their stacked weights, and one GEMM returns dx (no per-map dx sums);
+* the stacking and the fp32 copies of the small parameters are one launch
+  (``kda_layer_pack``), as are the bf16 roundings of their gradients;
+* every weight gradient is formed by one launch (``weight_grads``).
+
+``GatedDeltaLayer.forward`` runs this only where it is what the separate modules
+compute (``fused_params``); everything else keeps the general path.
+"""
+from __future__ import annotations
+
+from typing import List, Optional, Tuple
+
+import torch
+import torch.nn as nn
+from torch.nn.modules import module as _nn_module
+
+from . import _lib
+from .kda import _DTYPE_CODE, _stream, kda_backward_train, kda_forward, kda_forward_train
+
+_PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
+
+
+def _plain_module(m: nn.Module, cls: type) -> bool:
+    """m is exactly a cls whose call is its forward: no subclass (a
+    parametrization makes one), hooks or instance override."""
+    return (type(m) is cls and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
+            and not m._backward_hooks and not m._backward_pre_hooks)
+
+
+def fused_params(layer, x: torch.Tensor, state: Optional[torch.Tensor]) -> Optional[Tuple[torch.Tensor, ...]]:
+    """The layer's parameters in ``fused_layer``'s order, or None where the
+    general path has to run: other dtypes than bf16 activations and weights,
+    autocast or tracing, module hooks, replaced modules, tensor subclasses."""
+    from .layer import GatedDeltaLayer, RMSNormGated, ShortCausalConv1d
+    if x.dtype != torch.bfloat16 or x.device.type != "cuda" or x.numel() == 0 or type(x) not in _PLAIN_TENSORS:
+        return None
+    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling():
+        return None
+    if (_nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks
+            or _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks):
+        return None
+    if type(layer).produce is not GatedDeltaLayer.produce or "produce" in layer.__dict__:
+        return None
+    linears = (layer.q_proj, layer.k_proj, layer.v_proj, layer.f_proj_1, layer.g_proj_1, layer.b_proj,
+               layer.f_proj_2, layer.g_proj_2, layer.o_proj)
+    convs = (layer.q_conv1d, layer.k_conv1d, layer.v_conv1d)
+    if not (all(_plain_module(m, nn.Linear) for m in linears) and all(type(c) is ShortCausalConv1d for c in convs)
+            and _plain_module(layer.o_norm, RMSNormGated)):
+        return None
+    if any(m.bias is not None for m in linears if m is not layer.g_proj_2) or layer.g_proj_2.bias is None:
+        return None
+    if any(c.bias is None for c in convs):
+        return None
+    weights = [m.weight for m in linears] + [layer.g_proj_2.bias]
+    small = [c.weight for c in convs] + [c.bias for c in convs] + [layer.o_norm.weight, layer.dt_bias, layer.A_log]
+    dev = x.device
+    for p in weights:
+        if p.dtype != torch.bfloat16 or type(p) not in _PLAIN_TENSORS or p.device != dev or not p.is_contiguous():
+            return None
+    for p in small:
+        if p.dtype not in _DTYPE_CODE or type(p) not in _PLAIN_TENSORS or p.device != dev or not p.is_contiguous():
+            return None
+    hidden, total, D, H = layer.hidden_size, layer.total_dim, layer.head_dim, layer.num_heads
+    rank = layer.f_proj_1.weight.shape[0]
+    shapes = [(total, hidden)] * 3 + [(rank, hidden), (D, hidden), (H, hidden), (total, rank), (total, D),
+                                      (hidden, total), (total,)]
+    if any(tuple(p.shape) != s for p, s in zip(weights, shapes)):
+        return None
+    # the weight-gradient kernel reads 8 columns at a time and forms rows of 8
+    if hidden % 8 or rank % 8 or total % 8 or D % 8:
+        return None
+    if state is not None and (type(state) not in _PLAIN_TENSORS or state.device != dev):
+        return None
+    return (*weights, *small)
+
+
+def _pack(jobs: List[Tuple[torch.Tensor, int, int]]) -> None:
+    """One launch of copies with conversion: (source, destination address,
+    destination dtype code)."""
+    from .layer import _i64
+    arr = _i64([(s.data_ptr(), dst, s.numel(), _DTYPE_CODE[s.dtype] | dd << 8) for s, dst, dd in jobs])
+    _lib.check(_lib.load().kda_layer_pack(arr, len(jobs), _stream(jobs[0][0].device)), "kda_layer_pack")
+
+
+def _views(fp: torch.Tensor, HD: int, D: int):
+    """(conv_w, conv_b, norm weight, dt_bias, A_log) of the packed fp32 parameters."""
+    from .layer import CONV_TAPS
+    return (fp[:12 * HD].view(3, HD, CONV_TAPS), fp[12 * HD:15 * HD].view(3, HD), fp[15 * HD:15 * HD + D],
+            fp[15 * HD + D:16 * HD + D], fp[16 * HD + D:])
+
+
+def _forward(x, state, spec, params, train: bool):
+    """(out, new_state, what the backward reads, the training pair's workspace)."""
+    from .layer import gated_rmsnorm_forward, producer_forward
+    H, D, scale, mult, eps, chunk = spec
+    wq, wk, wv, wf1, wg1, wb, wf2, wg2, wo, bg2 = params[:10]
+    B, L, hidden = x.shape
+    M, HD, rank = B * L, H * D, wf1.shape[0]
+    N = 3 * HD + rank + D + H
+    NP = -(-N // 8) * 8
+    dev, bf = x.device, torch.bfloat16
+    x2 = x.contiguous().view(M, hidden)
+    # rows past N of the stacked weight are not written: the columns they give
+    # are not read
+    wcat = torch.empty((NP, hidden), dtype=bf, device=dev)
+    fp = torch.empty(16 * HD + D + H, dtype=torch.float32, device=dev)
+    jobs, at = [], wcat.data_ptr()
+    for w in (wq, wk, wv, wf1, wg1, wb):
+        jobs.append((w, at, 1))
+        at += 2 * w.numel()
+    at = fp.data_ptr()
+    for p in params[10:]:   # conv weights, conv biases, norm weight, dt_bias, A_log
+        jobs.append((p, at, 0))
+        at += 4 * p.numel()
+    _pack(jobs)
+    conv_w, conv_b, nw, dt_bias, A_log = _views(fp, HD, D)
+
+    P = torch.mm(x2, wcat.t())
+    P3 = P.view(B, L, NP)
+    xf = torch.mm(P[:, 3 * HD:3 * HD + rank], wf2.t()).view(B, L, HD)
+    z = torch.addmm(bg2, P[:, 3 * HD + rank:3 * HD + rank + D], wg2.t()).view(B, L, HD)
+    q, k, v, g, beta = producer_forward(P3[..., :3 * HD], xf, P3[..., N - H:N], conv_w, conv_b, dt_bias, A_log,
+                                        H, D, scale, mult, torch.float32)
+    ws = None
+    if train:
+        o, s_final, ws = kda_forward_train(q, k, v, g, beta, state, chunk)
+    else:
+        o, s_final = kda_forward(q, k, v, g, beta, state, chunk)
+    y = gated_rmsnorm_forward(o, z, nw, eps)
+    out = torch.mm(y.view(M, HD), wo.t()).view(B, L, hidden)
+    return out, s_final, (x2, P, xf, z, q, k, v, g, beta, state, o, y, wcat, fp, wf2, wg2, wo), ws
+
+
+def fused_layer(x, state, spec, params):
+    """(out, new_state) of the layer for x (B, L, hidden).  ``spec`` = (H, D, scale,
+    beta_mult, eps, chunk_size); ``params`` as ``fused_params`` orders them."""
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, state, *params)):
+        return FusedLayerFunction.apply(x, state, spec, *params)
+    out, s_final, _, _ = _forward(x, state, spec, params, False)
+    return out, s_final
+
+
+class FusedLayerFunction(torch.autograd.Function):
+    """``fused_layer`` with a gradient for every input."""
+
+    @staticmethod
+    def forward(ctx, x, state, spec, *params):
+        out, s_final, saved, ctx.ws = _forward(x, state, spec, params, True)
+        ctx.save_for_backward(*saved)
+        ctx.spec, ctx.shape = spec, (*x.shape, params[3].shape[0])
+        ctx.small = [(p.dtype, p.shape) for p in params[10:]]
+        ctx.set_materialize_grads(False)
+        return out, s_final
+
+    @staticmethod
+    @torch.no_grad()
+    def backward(ctx, dout, ds_final):
+        from .layer import gated_rmsnorm_backward, producer_backward, weight_grads
+        x2, P, xf, z, q, k, v, g, beta, s0, o, y, wcat, fp, wf2, wg2, wo = ctx.saved_tensors
+        H, D, scale, mult, eps, chunk = ctx.spec
+        B, L, hidden, rank = ctx.shape
+        M, HD, NP = B * L, H * D, wcat.shape[0]
+        N = 3 * HD + rank + D + H
+        f1, g1 = slice(3 * HD, 3 * HD + rank), slice(3 * HD + rank, 3 * HD + rank + D)
+        dev = x2.device
+        if dout is None:
+            dout = torch.zeros((B, L, hidden), dtype=x2.dtype, device=dev)
+        dout2 = dout.to(x2.dtype).contiguous().view(M, hidden)
+        conv_w, conv_b, nw, dt_bias, A_log = _views(fp, HD, D)
+        dy = torch.mm(dout2, wo).view(B, L, HD)
+        do, dz, dnw = gated_rmsnorm_backward(o, z, nw, eps, dy)
+        dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws, chunk,
+                                                        _need_ds0=ctx.needs_input_grad[1])
+        ctx.ws = None
+        dP = torch.empty((M, NP), dtype=x2.dtype, device=dev)
+        P3, dP3 = P.view(B, L, NP), dP.view(B, L, NP)
+        _, dxf, _, dcw, dcb, ddt, dA = producer_backward(
+            P3[..., :3 * HD], xf, P3[..., N - H:N], conv_w, conv_b, dt_bias, A_log, dq, dk, dv, dg, dbeta, H, D, scale,
+            mult, _dqkv=dP3[..., :3 * HD], _dxb=dP3[..., N - H:N])
+        dxf2, dz2 = dxf.view(M, HD), dz.view(M, HD)
+        torch.mm(dxf2, wf2, out=dP[:, f1])
+        torch.mm(dz2, wg2, out=dP[:, g1])
+        need = ctx.needs_input_grad
+        dx = torch.mm(dP[:, :N], wcat[:N]).view(B, L, hidden) if need[0] else None
+        grads: List[Optional[torch.Tensor]] = [None] * 19
+        if any(need[3:13]):
+            (dwcat, _), (dwo, _), (dwf2, _), (dwg2, dbg2) = weight_grads(
+                [(dP[:, :N], x2, False), (dout2, y.view(M, HD), False), (dxf2, P[:, f1], False),
+                 (dz2, P[:, g1], True)], M)
+            grads[:10] = [*dwcat.split([HD, HD, HD, rank, D, H]), dwf2, dwg2, dwo, dbg2]
+        if any(need[13:]):
+            sources = [*dcw, *dcb, dnw, ddt, dA]
+            jobs = []
+            for i, (t, (dt, shape)) in enumerate(zip(sources, ctx.small)):
+                if dt == torch.float32:
+                    grads[10 + i] = t.view(shape)
+                else:
+                    grads[10 + i] = torch.empty(shape, dtype=dt, device=dev)
+                    jobs.append((t, grads[10 + i].data_ptr(), _DTYPE_CODE[dt]))
+            if jobs:
+                _pack(jobs)
+        return (dx, ds0, None, *(t if n else None for t, n in zip(grads, need[3:])))

@@ -437,3 +437,57 @@ def test_weight_grads_parity(rows, shapes):
         if bias:
             errs["db"] = _rel(db, ref["db"])
         _check(errs, 2.0 ** -8, f"weight_grads rows={rows} n={dy.shape[1]} k={x.shape[1]}")
+
+
+@pytest.mark.parametrize("H,D,L,frozen,contiguous", [(3, 64, 100, False, True), (2, 32, 8, True, True),
+                                                     (8, 96, 70, False, False)])
+def test_layer_one_node_matches_modules(H, D, L, frozen, contiguous):
+    """The layer as one autograd node against the same layer run module by module
+    (a forward hook on one of its maps sends it there, and is called): outputs
+    and every gradient to the bf16 bar, with a state, frozen parameters, a
+    non-contiguous input, and with only the new state used."""
+    from mlx_vit_amd import GatedDeltaLayer
+    from mlx_vit_amd.layer_fused import fused_params
+    from mlx_vit_amd.model import to_bf16
+    torch.manual_seed(7)
+    layer = to_bf16(GatedDeltaLayer(H * D, H, D)).to(DEV)
+    if frozen:
+        for n, p in layer.named_parameters():
+            p.requires_grad_(n.startswith("g_proj") or n == "A_log" or n == "k_conv1d.weight")
+    gen = torch.Generator().manual_seed(L)
+    x = torch.randn(2, L, H * D, generator=gen).to(torch.bfloat16).to(DEV)
+    if not contiguous:
+        x = x.transpose(0, 1).contiguous().transpose(0, 1)
+    s0 = (0.1 * torch.randn(2, H, D, D, generator=gen)).to(DEV).requires_grad_()
+    dout = torch.randn(2, L, H * D, generator=gen).to(torch.bfloat16).to(DEV)
+    ds = torch.randn(2, H, D, D, generator=gen).to(DEV)
+    x.requires_grad_()
+    leaves = [("x", x), ("s0", s0)] + [(n, p) for n, p in layer.named_parameters() if p.requires_grad]
+
+    def grads(outs, cots):
+        got = torch.autograd.grad(outs, [t for _, t in leaves], cots, allow_unused=True)
+        return {n: g for (n, _), g in zip(leaves, got) if g is not None}
+
+    assert fused_params(layer, x, s0) is not None
+    out, s = layer(x, s0)
+    one = grads([out, s], [dout, ds])
+    only_state = grads([layer(x, s0)[1]], [ds])
+    with torch.no_grad():
+        out_ng, s_ng = layer(x, s0)
+    calls = []
+    handle = layer.b_proj.register_forward_hook(lambda *a: calls.append(1))
+    assert fused_params(layer, x, s0) is None
+    out_m, s_m = layer(x, s0)
+    mods = grads([out_m, s_m], [dout, ds])
+    mods_state = grads([layer(x, s0)[1]], [ds])
+    handle.remove()
+    torch.cuda.synchronize()
+    assert len(calls) == 2 and set(one) == set(mods)
+    errs = {"out": _rel(out, out_m), "s": _rel(s, s_m), "out_ng": _rel(out_ng, out_m), "s_ng": _rel(s_ng, s_m)}
+    errs.update({n: _rel(g, mods[n]) for n, g in one.items()})
+    # the maps behind the output only (gate, norm, o_proj) get zeros or no gradient here
+    errs.update({"state:" + n: _rel(g, mods_state[n]) for n, g in only_state.items()
+                 if n in mods_state and mods_state[n].abs().max() > 0})
+    for n, g in one.items():
+        assert g.dtype == mods[n].dtype and g.shape == mods[n].shape, n
+    _check(errs, 1e-2, f"one node H={H} D={D} L={L}")
