@@ -34,9 +34,9 @@ namespace {
 constexpr int KC = 4;        // conv taps (ShortCausalConv1d(kernel_size=4))
 constexpr int CPW = 256;     // channels per wave
 constexpr int MAXW = 8;      // H*D <= 2048
-constexpr int PR = 2;        // producer forward: rows per workgroup
-constexpr int BR = 8;        // producer backward: rows per strip
-constexpr int BNS = 4;       // producer backward: strips per workgroup
+constexpr int PR = 3;        // producer forward: rows per workgroup
+constexpr int BR = 4;        // producer backward: rows per strip
+constexpr int BNS = 8;       // producer backward: strips per workgroup
 constexpr int NR = 4;        // norm forward: rows per workgroup
 constexpr int NRB = 4;       // norm backward: rows per strip
 constexpr int NNS = 2;       // norm backward: strips per workgroup
@@ -78,6 +78,21 @@ __device__ __forceinline__ float wave_sum(float v) {
     for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
     return v;
 }
+// Sum over the wave by DPP adds (row shifts, then the row broadcasts): the total
+// is in lane 63.  Six VALU adds; a shuffle butterfly is six LDS-pipe permutes.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_add(float x) {
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROWS, 0xf, ROWS == 0xf));
+}
+__device__ __forceinline__ float wave_sum63(float x) {
+    x = dpp_add<0x111, 0xf>(x);   // row_shr 1, 2, 4, 8: lane 15 of each row of 16 has the row's sum
+    x = dpp_add<0x112, 0xf>(x);
+    x = dpp_add<0x114, 0xf>(x);
+    x = dpp_add<0x118, 0xf>(x);
+    x = dpp_add<0x142, 0xa>(x);   // row_bcast 15 into rows 1 and 3, row_bcast 31 into rows 2 and 3
+    return dpp_add<0x143, 0xc>(x);
+}
+
 // Sum over aligned groups of n lanes (n a power of two <= 64).
 __device__ __forceinline__ float lanes_sum(float v, int n) {
     for (int m = n >> 1; m >= 1; m >>= 1) v += __shfl_xor(v, m);
@@ -157,10 +172,11 @@ __device__ __forceinline__ void conv_silu_rows(const ProdArgs& a, const Lanes& L
 
 // Workgroup = (batch row b, strip of PR tokens).  q and k need the norm of the
 // whole H*D row: a first pass forms the per-row sums of squares (reduced
-// across the workgroup through LDS), and after the barrier q and k are
-// scaled by their inverse norms and stored, held in registers across the
-// barrier (70 VGPRs at PR = 2; at 4 rows recomputing them after the barrier
-// was 15% slower than holding them).
+// across the workgroup through LDS), and after the barrier, which leaves the
+// stores of v, g and beta in flight, q and k are scaled by their inverse norms
+// and stored, held in registers across it (80 VGPRs).  HBM-bound: 12544 x 768
+// bf16 with fp32 g, 173 MB, 45.6 us on warm inputs (3.8 TB/s) against 47.8 and
+// 49.8 us at 2 and 4 rows (a strip reads PR + 3 rows of each conv input).
 template <typename ST, typename GT>
 __global__ __launch_bounds__(512) void producer_fwd_kernel(const ProdArgs a) {
     __shared__ float red[2][MAXW][PR];
@@ -178,8 +194,8 @@ __global__ __launch_bounds__(512) void producer_fwd_kernel(const ProdArgs a) {
             if (L.live)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) ss = fmaf(sv[j][e], sv[j][e], ss);
-            ss = wave_sum(ss);
-            if (L.lane == 0) red[i][L.w][j] = ss;
+            ss = wave_sum63(ss);
+            if (L.lane == 63) red[i][L.w][j] = ss;
         }
     };
     float sq[PR][4], sk[PR][4];
@@ -225,7 +241,7 @@ __global__ __launch_bounds__(512) void producer_fwd_kernel(const ProdArgs a) {
             if (t0 + j < T) st1<ST>(beta + (rb + t0 + j) * a.H + L.h, sigm(xv[j]) * a.beta_mult);
     }
 
-    __syncthreads();
+    lds_barrier();   // leaves the stores above in flight
     auto finish = [&](const float (&sv)[PR][4], int i, ST* out, float mult) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < PR; ++j) {
@@ -243,33 +259,32 @@ __global__ __launch_bounds__(512) void producer_fwd_kernel(const ProdArgs a) {
 }
 
 // ---------------------------------------------------------------- producer, backward
-// dy (the adjoint of the conv output) of tensor i for NRW rows from t0; the
-// x rows t0-3 .. t0+NRW-1 come back in xr for the tap gradients.  For q and k
-// the row norms reduce across the workgroup through red (one barrier).
-template <typename ST, int NRW, int I>
-__device__ __forceinline__ void prod_dy_rows(const ProdArgs& a, const Lanes& L, int t0, size_t rb,
-                                             const float (&wt)[4][KC], const float (&bias)[4],
-                                             float (*red)[2][BR], float (&dy)[NRW][4],
-                                             float (&xr)[NRW + KC - 1][4]) {
-    const int T = a.T;
-    constexpr int i = I;
-    const ST* x = static_cast<const ST*>(I == 0 ? a.xq : I == 1 ? a.xk : a.xv);
-    const ST* d = static_cast<const ST*>(I == 0 ? a.dq : I == 1 ? a.dk : a.dv);
-#pragma unroll
-    for (int r = 0; r < NRW + KC - 1; ++r) {
-        const int t = t0 - (KC - 1) + r;
-        Vec4<ST>::ld(x + (rb + min(max(t, 0), T - 1)) * a.ld_x + L.cc, xr[r]);
-        if (t < 0) xr[r][0] = xr[r][1] = xr[r][2] = xr[r][3] = 0.f;
+// four channels of a row as loaded
+template <typename ST> struct Raw4;
+template <> struct Raw4<float> {
+    float4 v;
+    __device__ __forceinline__ void ld(const float* p) { v = *reinterpret_cast<const float4*>(p); }
+    __device__ __forceinline__ void get(float* x) const { x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w; }
+};
+template <> struct Raw4<uint16_t> {
+    uint2 v;
+    __device__ __forceinline__ void ld(const uint16_t* p) { v = *reinterpret_cast<const uint2*>(p); }
+    __device__ __forceinline__ void get(float* x) const {
+        x[0] = bf_lo(v.x); x[1] = bf_hi(v.x); x[2] = bf_lo(v.y); x[3] = bf_hi(v.y);
     }
-    float dd[NRW][4];
+};
+
+// dy (the adjoint of the conv output) of N rows from the x rows N + 3 and the
+// cotangents dd (zero for rows past T and idle lanes).  For q and k (NORM) the
+// row norms reduce across the workgroup through red (one barrier that leaves
+// the loads and stores in flight).
+template <int N, bool NORM>
+__device__ __forceinline__ void conv_dy_rows(const Lanes& L, float mult, const float (&wt)[4][KC],
+                                             const float (&bias)[4], const float (&xr)[N + KC - 1][4],
+                                             const float (&dd)[N][4], float (*red)[2 * BR], float (&dy)[N][4]) {
+    float y[N][4], sg[N][4];
 #pragma unroll
-    for (int j = 0; j < NRW; ++j) {
-        Vec4<ST>::ld(d + (rb + min(t0 + j, T - 1)) * L.HD + L.cc, dd[j]);
-        if (t0 + j >= T || !L.live) dd[j][0] = dd[j][1] = dd[j][2] = dd[j][3] = 0.f;
-    }
-    float y[NRW][4], sg[NRW][4];
-#pragma unroll
-    for (int j = 0; j < NRW; ++j)
+    for (int j = 0; j < N; ++j)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float v = bias[e];
@@ -278,160 +293,242 @@ __device__ __forceinline__ void prod_dy_rows(const ProdArgs& a, const Lanes& L, 
             y[j][e] = v;
             sg[j][e] = sigm(v);
         }
-    float ds[NRW][4];
-    if (i < 2) {
+    float inv[N], corr[N];
+    if constexpr (NORM) {
 #pragma unroll
-        for (int j = 0; j < NRW; ++j) {
+        for (int j = 0; j < N; ++j) {
             float ss = 0.f, dot = 0.f;
-            if (L.live)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float sv = y[j][e] * sg[j][e];
-                    ss = fmaf(sv, sv, ss);
-                    dot = fmaf(sv, dd[j][e], dot);
-                }
-            ss = wave_sum(ss);
-            dot = wave_sum(dot);
-            if (L.lane == 0) { red[L.w][0][j] = ss; red[L.w][1][j] = dot; }
+            for (int e = 0; e < 4; ++e) {
+                const float sv = L.live ? y[j][e] * sg[j][e] : 0.f;
+                ss = fmaf(sv, sv, ss);
+                dot = fmaf(sv, dd[j][e], dot);
+            }
+            ss = wave_sum63(ss);
+            dot = wave_sum63(dot);
+            if (L.lane == 63) {
+                red[L.w][2 * j] = ss;
+                red[L.w][2 * j + 1] = dot;
+            }
         }
-        __syncthreads();
-        const float mult = i == 0 ? a.scale : 1.f;
+        lds_barrier();
+        float tot[2 * BR];
 #pragma unroll
-        for (int j = 0; j < NRW; ++j) {
-            float ss = 0.f, dot = 0.f;
-            for (int u = 0; u < L.NW; ++u) { ss += red[u][0][j]; dot += red[u][1][j]; }
-            const float n = sqrtf(ss);
-            // d(s / max(n, eps)) = ds / n - s (s . ds) / n^3 while n > eps, ds / eps below
-            const float inv = n > L2_EPS ? 1.f / n : 1.f / L2_EPS;
-            const float corr = n > L2_EPS ? dot * inv * inv : 0.f;
+        for (int j = 0; j < 2 * BR; ++j) tot[j] = 0.f;
+        for (int u = 0; u < L.NW; ++u)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) ds[j][e] = mult * inv * (dd[j][e] - y[j][e] * sg[j][e] * corr);
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < NRW; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ds[j][e] = dd[j][e];
-    }
-#pragma unroll
-    for (int j = 0; j < NRW; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            dy[j][e] = (t0 + j < T && L.live)
-                           ? ds[j][e] * sg[j][e] * (1.f + y[j][e] * (1.f - sg[j][e]))
-                           : 0.f;
-}
-
-// One conv input's backward over a segment [tlo, thi) of batch row rb / T.
-template <typename ST, int I>
-__device__ __forceinline__ void prod_bwd_conv(const ProdArgs& a, const Lanes& L, int tlo, int thi, size_t rb,
-                                              float (*red)[MAXW][2][BR], float* part) {
-    constexpr int i = I;
-    const int T = a.T;
-    const int nst = (thi - tlo + BR - 1) / BR;
-    int par = 0;
-        float wt[4][KC], bias[4];
-        load_taps<I>(a, L, wt, bias);
-        ST* dx = static_cast<ST*>(I == 0 ? a.dxq : I == 1 ? a.dxk : a.dxv);
-        float acc[KC + 1][4];
-#pragma unroll
-        for (int k = 0; k <= KC; ++k) acc[k][0] = acc[k][1] = acc[k][2] = acc[k][3] = 0.f;
-        float carry[KC - 1][4];
-        if (thi < T) {
-            float xh[2 * (KC - 1)][4];
-            prod_dy_rows<ST, KC - 1, I>(a, L, thi, rb, wt, bias, red[par], carry, xh);
-            par ^= 1;
-        } else {
-#pragma unroll
-            for (int r = 0; r < KC - 1; ++r) carry[r][0] = carry[r][1] = carry[r][2] = carry[r][3] = 0.f;
-        }
-        for (int si = nst - 1; si >= 0; --si) {
-            const int t0 = tlo + si * BR;
-            float dy[BR][4], xr[BR + KC - 1][4];
-            prod_dy_rows<ST, BR, I>(a, L, t0, rb, wt, bias, red[par], dy, xr);
-            par ^= 1;
-#pragma unroll
-            for (int j = 0; j < BR; ++j) {
-                float o[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float v = 0.f;
-#pragma unroll
-                    for (int k = 0; k < KC; ++k) {
-                        const int u = j + KC - 1 - k;   // x[t] feeds y[t + 3 - k] through tap k
-                        v = fmaf(wt[e][k], u < BR ? dy[u][e] : carry[u - BR][e], v);
-                    }
-                    o[e] = v;
-                }
-                if (t0 + j < T && L.live) Vec4<ST>::st(dx + (rb + t0 + j) * a.ld_dx + L.cc, o);
+            for (int j = 0; j < 2 * BR; j += 4) {
+                const float4 r = *reinterpret_cast<const float4*>(&red[u][j]);
+                tot[j] += r.x; tot[j + 1] += r.y; tot[j + 2] += r.z; tot[j + 3] += r.w;
             }
 #pragma unroll
-            for (int j = 0; j < BR; ++j)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-#pragma unroll
-                    for (int k = 0; k < KC; ++k) acc[k][e] = fmaf(dy[j][e], xr[j + k][e], acc[k][e]);
-                    acc[KC][e] += dy[j][e];
-                }
-#pragma unroll
-            for (int r = 0; r < KC - 1; ++r)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) carry[r][e] = dy[r][e];
+        for (int j = 0; j < N; ++j) {
+            // d(s / max(n, eps)) = ds / n - s (s . ds) / n^3 while n > eps, ds / eps below
+            const float n = sqrtf(tot[2 * j]);
+            const float i = n > L2_EPS ? 1.f / n : 1.f / L2_EPS;
+            corr[j] = n > L2_EPS ? tot[2 * j + 1] * i * i : 0.f;
+            inv[j] = mult * i;
         }
-        if (L.live)
-#pragma unroll
-            for (int k = 0; k <= KC; ++k) Vec4<float>::st(part + (size_t)(5 * i + k) * L.HD, acc[k]);
     }
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float ds = NORM ? inv[j] * (dd[j][e] - y[j][e] * sg[j][e] * corr[j]) : dd[j][e];
+            dy[j][e] = ds * sg[j][e] * (1.f + y[j][e] * (1.f - sg[j][e]));
+        }
+}
 
-// Workgroup = (batch row b, segment of BR*BNS tokens) x role: blockIdx.y 0-2
-// takes conv input q, k or v, 3 the decay and write gates, so four
-// independent workgroups share a segment.  A conv input runs its strips from
-// the last to the first so that the dy rows a strip needs beyond its end are
-// the previous strip's (carried in registers); the three rows past the
-// segment are recomputed once.  Partial sums of the parameter gradients go to
-// part[wg][NPV][H*D]:
+// One conv input's backward over a segment [tlo, thi) of batch row rb / T, in
+// strips of BR rows from the last to the first: the dy rows a strip needs
+// beyond its end are the previous strip's, and the x rows before its start the
+// next strip's, which are in registers a strip ahead (as is the next strip's
+// cotangent).
+template <typename ST, int I>
+__device__ __forceinline__ void prod_bwd_conv_rows(const ProdArgs& a, const Lanes& L, int tlo, int thi, size_t rb,
+                                                   const float (&wt)[4][KC], const float (&bias)[4],
+                                                   float (*red)[MAXW][2 * BR], int& par, float (&acc)[KC + 1][4]) {
+    constexpr bool NORM = I < 2;
+    const int T = a.T;
+    const float mult = I == 0 ? a.scale : 1.f;
+    const ST* x = static_cast<const ST*>(I == 0 ? a.xq : I == 1 ? a.xk : a.xv) + L.cc;
+    const ST* d = static_cast<const ST*>(I == 0 ? a.dq : I == 1 ? a.dk : a.dv) + L.cc;
+    ST* dx = static_cast<ST*>(I == 0 ? a.dxq : I == 1 ? a.dxk : a.dxv) + L.cc;
+    const int nst = (thi - tlo + BR - 1) / BR;
+    int t0 = tlo + (nst - 1) * BR;
+    // rows outside [0, T) are read at its ends and zeroed where they are used
+    auto ld_x = [&](Raw4<ST>& r, int t) __attribute__((always_inline)) {
+        r.ld(x + (rb + min(max(t, 0), T - 1)) * a.ld_x);
+    };
+    auto ld_d = [&](Raw4<ST>& r, int t) __attribute__((always_inline)) {
+        r.ld(d + (rb + min(max(t, 0), T - 1)) * L.HD);
+    };
+    auto get_x = [&](const Raw4<ST>& r, int t, float* o) __attribute__((always_inline)) {
+        r.get(o);
+        if (t < 0) o[0] = o[1] = o[2] = o[3] = 0.f;
+    };
+    auto get_d = [&](const Raw4<ST>& r, int t, float* o) __attribute__((always_inline)) {
+        r.get(o);
+        if (t >= T || !L.live) o[0] = o[1] = o[2] = o[3] = 0.f;
+    };
+    Raw4<ST> xc[BR], xp[BR], dc[BR];   // x rows t0.., x rows t0 - BR.., d rows t0..
+#pragma unroll
+    for (int j = 0; j < BR; ++j) ld_x(xc[j], t0 + j);
+#pragma unroll
+    for (int j = 0; j < BR; ++j) ld_d(dc[j], t0 + j);
+#pragma unroll
+    for (int j = 0; j < BR; ++j) ld_x(xp[j], t0 - BR + j);
+    float carry[KC - 1][4];
+    if (thi < T) {
+        Raw4<ST> hx[2 * (KC - 1)], hd[KC - 1];
+#pragma unroll
+        for (int r = 0; r < 2 * (KC - 1); ++r) ld_x(hx[r], thi - (KC - 1) + r);
+#pragma unroll
+        for (int r = 0; r < KC - 1; ++r) ld_d(hd[r], thi + r);
+        float xr[2 * (KC - 1)][4], dd[KC - 1][4];
+#pragma unroll
+        for (int r = 0; r < 2 * (KC - 1); ++r) get_x(hx[r], thi - (KC - 1) + r, xr[r]);
+#pragma unroll
+        for (int r = 0; r < KC - 1; ++r) get_d(hd[r], thi + r, dd[r]);
+        conv_dy_rows<KC - 1, NORM>(L, mult, wt, bias, xr, dd, red[par], carry);
+        par ^= 1;
+    } else {
+#pragma unroll
+        for (int r = 0; r < KC - 1; ++r) carry[r][0] = carry[r][1] = carry[r][2] = carry[r][3] = 0.f;
+    }
+    for (; t0 >= tlo; t0 -= BR) {
+        Raw4<ST> xn[BR], dn[BR];
+#pragma unroll
+        for (int j = 0; j < BR; ++j) ld_d(dn[j], t0 - BR + j);
+#pragma unroll
+        for (int j = 0; j < BR; ++j) ld_x(xn[j], t0 - 2 * BR + j);
+        float xr[BR + KC - 1][4], dd[BR][4], dy[BR][4];
+#pragma unroll
+        for (int r = 0; r < KC - 1; ++r) get_x(xp[BR - (KC - 1) + r], t0 - (KC - 1) + r, xr[r]);
+#pragma unroll
+        for (int j = 0; j < BR; ++j) {
+            xc[j].get(xr[KC - 1 + j]);
+            get_d(dc[j], t0 + j, dd[j]);
+        }
+        conv_dy_rows<BR, NORM>(L, mult, wt, bias, xr, dd, red[par], dy);
+        par ^= 1;
+#pragma unroll
+        for (int j = 0; j < BR; ++j) {
+            float o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = 0.f;
+#pragma unroll
+                for (int k = 0; k < KC; ++k) {
+                    const int u = j + KC - 1 - k;   // x[t] feeds y[t + 3 - k] through tap k
+                    v = fmaf(wt[e][k], u < BR ? dy[u][e] : carry[u - BR][e], v);
+                }
+                o[e] = v;
+            }
+            if (t0 + j < T && L.live) Vec4<ST>::st(dx + (rb + t0 + j) * a.ld_dx, o);
+        }
+#pragma unroll
+        for (int j = 0; j < BR; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int k = 0; k < KC; ++k) acc[k][e] = fmaf(dy[j][e], xr[j + k][e], acc[k][e]);
+                acc[KC][e] += dy[j][e];
+            }
+#pragma unroll
+        for (int r = 0; r < KC - 1; ++r)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) carry[r][e] = dy[r][e];
+#pragma unroll
+        for (int j = 0; j < BR; ++j) {
+            xc[j] = xp[j];
+            xp[j] = xn[j];
+            dc[j] = dn[j];
+        }
+    }
+}
+
+// conv input I over the segments [tlo, thi) of the batch rows b0 .. b1 - 1; par
+// alternates the two reduction buffers across all of them
+template <typename ST, int I>
+__device__ __forceinline__ void prod_bwd_conv(const ProdArgs& a, const Lanes& L, int tlo, int thi, int b0, int b1,
+                                              float (*red)[MAXW][2 * BR], float* part) {
+    float wt[4][KC], bias[4], acc[KC + 1][4];
+    load_taps<I>(a, L, wt, bias);
+#pragma unroll
+    for (int k = 0; k <= KC; ++k) acc[k][0] = acc[k][1] = acc[k][2] = acc[k][3] = 0.f;
+    int par = 0;
+    for (int b = b0; b < b1; ++b)
+        prod_bwd_conv_rows<ST, I>(a, L, tlo, thi, (size_t)b * a.T, wt, bias, red, par, acc);
+    if (L.live)
+#pragma unroll
+        for (int k = 0; k <= KC; ++k) Vec4<float>::st(part + (size_t)(5 * I + k) * L.HD, acc[k]);
+}
+
+// Sequences shorter than a segment: as many of them per workgroup as fill one,
+// so that the parameter-gradient partials (17 H*D floats a workgroup) stay a
+// small part of the traffic (1568 sequences of 8 tokens: 82 MB written and
+// read with one each)
+__host__ __device__ __forceinline__ int prod_seqs(int T) { return T * 2 > BR * BNS ? 1 : BR * BNS / (T > 0 ? T : 1); }
+
+
+// Workgroup = (batch row b, segment of BR*BNS tokens; or prod_seqs short
+// sequences) x role: blockIdx.y 0-2 takes conv input q, k or v, 3 the decay and
+// write gates, so four independent workgroups share a segment.  What bounds it:
+// VALU (about 45 operations and two transcendentals an element) and latency at
+// two waves a SIMD (226 VGPRs).  Strips of 4 rows with the next strip's rows
+// loaded a strip ahead, the row norms by DPP adds, and barriers that leave
+// loads and stores in flight: at 12544 x 768 bf16 159 -> 103 us with the
+// reductions, against 8-row strips (256 VGPRs) with shuffle butterflies, whose
+// loads each strip waited for.  Three waves a SIMD (168 VGPRs, 70 spilled) take
+// 117 us; 12 or 16 strips a workgroup 107 and 112 us.  The segment's last
+// strip needs the three dy rows past its end: recomputed once.  Partial sums
+// of the parameter gradients go to part[wg][NPV][H*D]:
 //   v = 5 i + k  tap k of conv i     v = 5 i + 4  bias of conv i
 //   v = 15       dt_bias             v = 16       dg * g (summed per head -> dA_log)
 template <typename ST, typename GT>
 __global__ __launch_bounds__(512) void producer_bwd_kernel(const ProdArgs a) {
-    __shared__ float red[2][MAXW][2][BR];
+    __shared__ __attribute__((aligned(16))) float red[2][MAXW][2 * BR];
     const Lanes L(a.H, a.D);
     const int T = a.T;
     constexpr int SEG = BR * BNS;
-    const int nseg = (T + SEG - 1) / SEG;
+    const int nseg = (T + SEG - 1) / SEG, nb = prod_seqs(T);
     const int wg = xcd_remap(blockIdx.x, gridDim.x);
-    const int b = wg / nseg, tlo = (wg % nseg) * SEG;
+    const int b0 = wg / nseg * nb, b1 = min(a.B, b0 + nb), tlo = (wg % nseg) * SEG;
     const int thi = min(tlo + SEG, T);
-    const size_t rb = (size_t)b * T;
     float* part = a.part + (size_t)wg * NPV * L.HD + L.cc;
 
     const int role = blockIdx.y;
-    if (role == 0) prod_bwd_conv<ST, 0>(a, L, tlo, thi, rb, red, part);
-    else if (role == 1) prod_bwd_conv<ST, 1>(a, L, tlo, thi, rb, red, part);
-    else if (role == 2) prod_bwd_conv<ST, 2>(a, L, tlo, thi, rb, red, part);
-    // decay gate (when present) and write gate over rows [tlo, thi)
+    if (role == 0) prod_bwd_conv<ST, 0>(a, L, tlo, thi, b0, b1, red, part);
+    else if (role == 1) prod_bwd_conv<ST, 1>(a, L, tlo, thi, b0, b1, red, part);
+    else if (role == 2) prod_bwd_conv<ST, 2>(a, L, tlo, thi, b0, b1, red, part);
+    // decay gate (when present) and write gate over the rows: a segment's, or
+    // those of the whole short sequences, which follow one another
     else {
+        const size_t lo = (size_t)b0 * T + tlo;
+        const int rows = nseg > 1 ? thi - tlo : (b1 - b0) * T;
         if (a.dg) {
-            const ST* xf = static_cast<const ST*>(a.xf);
-            const GT* dg = static_cast<const GT*>(a.dg);
-            ST* dxf = static_cast<ST*>(a.dxf);
+            const ST* xf = static_cast<const ST*>(a.xf) + lo * a.ld_f + L.cc;
+            const GT* dg = static_cast<const GT*>(a.dg) + lo * L.HD + L.cc;
+            ST* dxf = static_cast<ST*>(a.dxf) + lo * a.ld_df + L.cc;
             const float4 dtv = *reinterpret_cast<const float4*>(a.dt_bias + L.cc);
             const float dt[4] = {dtv.x, dtv.y, dtv.z, dtv.w};
             const float eA = __expf(a.A_log[L.h]);
             float adt[4] = {0.f, 0.f, 0.f, 0.f}, aA[4] = {0.f, 0.f, 0.f, 0.f};
-            for (int t0 = tlo; t0 < thi; t0 += BR) {
-                float z[BR][4], dgv[BR][4];
-    #pragma unroll
-                for (int j = 0; j < BR; ++j) {
-                    const size_t r = rb + min(t0 + j, T - 1);
-                    Vec4<ST>::ld(xf + r * a.ld_f + L.cc, z[j]);
-                    Vec4<GT>::ld(dg + r * L.HD + L.cc, dgv[j]);
+            constexpr int GR = 8;   // rows in flight
+            for (int t0 = 0; t0 < rows; t0 += GR) {
+                float z[GR][4], dgv[GR][4];
+#pragma unroll
+                for (int j = 0; j < GR; ++j) {
+                    const size_t r = min(t0 + j, rows - 1);
+                    Vec4<ST>::ld(xf + r * a.ld_f, z[j]);
+                    Vec4<GT>::ld(dg + r * L.HD, dgv[j]);
                 }
-    #pragma unroll
-                for (int j = 0; j < BR; ++j) {
-                    const bool ok = t0 + j < thi && L.live;
+#pragma unroll
+                for (int j = 0; j < GR; ++j) {
+                    const bool ok = t0 + j < rows && L.live;
                     float o[4];
-    #pragma unroll
+#pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float zz = z[j][e] + dt[e];
                         const float gd = ok ? dgv[j][e] : 0.f;
@@ -439,7 +536,7 @@ __global__ __launch_bounds__(512) void producer_bwd_kernel(const ProdArgs a) {
                         adt[e] += o[e];
                         aA[e] = fmaf(gd, -eA * softplus(zz), aA[e]);
                     }
-                    if (ok) Vec4<ST>::st(dxf + (rb + t0 + j) * a.ld_df + L.cc, o);
+                    if (ok) Vec4<ST>::st(dxf + (size_t)(t0 + j) * a.ld_df, o);
                 }
             }
             if (L.live) {
@@ -451,25 +548,14 @@ __global__ __launch_bounds__(512) void producer_bwd_kernel(const ProdArgs a) {
             Vec4<float>::st(part + (size_t)15 * L.HD, zero);
             Vec4<float>::st(part + (size_t)16 * L.HD, zero);
         }
-        if (L.live && L.cc % a.D == 0) {
-            const ST* xb = static_cast<const ST*>(a.xb);
-            const ST* dbeta = static_cast<const ST*>(a.dbeta);
-            ST* dxb = static_cast<ST*>(a.dxb);
-            for (int t0 = tlo; t0 < thi; t0 += BR) {
-                float xv[BR], dv[BR];   // all loads of the strip first
-#pragma unroll
-                for (int j = 0; j < BR; ++j) {
-                    const size_t r = rb + min(t0 + j, T - 1);
-                    xv[j] = ld1<ST>(xb + r * a.ld_b + L.h);
-                    dv[j] = ld1<ST>(dbeta + r * a.H + L.h);
-                }
-#pragma unroll
-                for (int j = 0; j < BR; ++j) {
-                    const float sb = sigm(xv[j]);
-                    if (t0 + j < thi)
-                        st1<ST>(dxb + (rb + t0 + j) * a.ld_db + L.h, dv[j] * a.beta_mult * sb * (1.f - sb));
-                }
-            }
+        // write gate: (row, head) pairs over the threads
+        const ST* xb = static_cast<const ST*>(a.xb) + lo * a.ld_b;
+        const ST* dbeta = static_cast<const ST*>(a.dbeta) + lo * a.H;
+        ST* dxb = static_cast<ST*>(a.dxb) + lo * a.ld_db;
+        for (int i = threadIdx.x; i < rows * a.H; i += blockDim.x) {
+            const int r = i / a.H, h = i - r * a.H;
+            const float sb = sigm(ld1<ST>(xb + (size_t)r * a.ld_b + h));
+            st1<ST>(dxb + (size_t)r * a.ld_db + h, ld1<ST>(dbeta + i) * a.beta_mult * sb * (1.f - sb));
         }
     }
 }
@@ -684,7 +770,10 @@ int norm_waves(int H, int D) {
     return (H + hpw - 1) / hpw;
 }
 
-int producer_partials(int B, int T) { return B * ((T + BR * BNS - 1) / (BR * BNS)); }
+int producer_partials(int B, int T) {
+    const int nb = prod_seqs(T);
+    return (B + nb - 1) / nb * ((T + BR * BNS - 1) / (BR * BNS));
+}
 size_t producer_ws_floats(int B, int T, int H, int D) {
     const int P = producer_partials(B, T), N = NPV * H * D;
     return ((size_t)P + 1 + colsum_splits(P, N)) * N;
