@@ -62,51 +62,77 @@ __device__ __forceinline__ float sum4gw(float x) {
     return x;
 }
 
-// The diagonal tile of block m, pair by pair, for the lane's rows t = 16 m +
-// 4 g4 + e of channel d: everything from LDS -- gamma g (row stride ldg), the
-// staged raw k / q rows sk / sq (row stride ldq), dP sp and dA sda (row stride
-// lda) -- and the sums (dk, dq, dgamma terms) to res[3][16][D].  Not inlined:
-// its loops stay out of the register allocation of the kernel's common path.
-template <int D, typename TI, int PREC>
-__device__ __noinline__ void wide_pair_block(const float* __restrict__ g, int ldg, const TI* __restrict__ sk,
-                                             const TI* __restrict__ sq, int ldq, const float* __restrict__ sp,
-                                             const float* __restrict__ sda, int lda, float* __restrict__ res, int m,
-                                             int g4, int d) {
-    // the lane's four rows advance together: four independent sums per step
-    float gt[4], kt[4], qt[4], ak[4], aq[4], ag[4];
+// Layout of a wave's private LDS for its diagonal tiles: the raw k and q rows of
+// its 16 channels ([64][DT_K] bf16 each), then over them two planes of sums
+// ([64][DT_P] fp32); strides that put the four blocks' rows on distinct banks
+constexpr int DT_K = 18, DT_P = 17, DT_BYTES = 2 * C * DT_P * 4;
+static_assert(2 * C * DT_K * 2 <= DT_BYTES, "k and q fit under the planes");
+
+// The four diagonal tiles of a wave's channel tile, pair by pair with the exact
+// weight e^{gamma_t - gamma_s} (s < t): lane (r16, g4) takes block g4 of channel
+// d = its r16's, all 120 pairs of it, the block's rows in registers.  wp: the
+// wave's private area (above); gamma s.g (row stride ldg, own channels only),
+// dP sp and dA sda (row stride lda).  The sums (rows of dk, dq) go to the two
+// planes and those of dgamma over the gamma column itself, which nothing reads
+// afterwards: everything is the wave's own, so no barrier.  Each pair's dgamma
+// term is one value, added to row t and taken from row s.
+// Not inlined: its registers stay out of the kernel's common path.
+typedef __attribute__((address_space(3))) float lds_f32;
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+typedef __attribute__((address_space(3))) unsigned char lds_u8;
+
+template <int PREC>
+__device__ __noinline__ void wide_diag_tiles(lds_f32* g, int ldg, lds_u8* wp, const lds_f32* sp, const lds_f32* sda,
+                                             int lda, int g4, int r16) {
+    const lds_u16* sk = reinterpret_cast<const lds_u16*>(wp) + BS * g4 * DT_K + r16;
+    const lds_u16* sq = sk + C * DT_K;
+    g += BS * g4 * ldg;
+    float gt[BS], kt[BS], qt[BS], ak[BS], aq[BS], ag[BS];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int t = BS * m + 4 * g4 + e;
-        gt[e] = g[t * ldg + d];
-        kt[e] = ld1<TI>(sk + t * ldq + d);
-        qt[e] = ld1<TI>(sq + t * ldq + d);
-        ak[e] = aq[e] = ag[e] = 0.f;
+    for (int t = 0; t < BS; ++t) {
+        gt[t] = g[t * ldg];
+        kt[t] = bf2f(sk[t * DT_K]);
+        qt[t] = bf2f(sq[t * DT_K]);
+        ak[t] = aq[t] = ag[t] = 0.f;
     }
-#pragma unroll 1
-    for (int r = 0; r < BS; ++r) {
-        const int sx = BS * m + r;
-        const float gs = g[sx * ldg + d], ks_raw = ld1<TI>(sk + sx * ldq + d), qs_raw = ld1<TI>(sq + sx * ldq + d);
+    const lds_f32* pr = sp + BS * g4 * lda + BS * g4;
+    const lds_f32* ar = sda + BS * g4 * lda + BS * g4;
+    typedef __attribute__((address_space(3))) const f32x4 lds_f32x4;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int rt = 4 * g4 + e, t = BS * m + rt;
-            // row side: pair (t, s), s < t; column side: pair (s, t), s > t
-            const bool row = r < rt, col = r > rt;
-            const float ex = kexp<PREC>(row ? gt[e] - gs : gs - gt[e]);
-            const float pp = sp[row ? t * lda + sx : sx * lda + t], pa = sda[row ? t * lda + sx : sx * lda + t];
-            const float ks = ks_raw * ex;
-            const float c = (pp * ks_raw + pa * qs_raw) * ex;
-            ak[e] += row ? pp * ks : col ? c : 0.f;
-            aq[e] += row ? pa * ks : 0.f;
-            ag[e] += row ? (pp * kt[e] + pa * qt[e]) * ks : col ? -c * kt[e] : 0.f;
+    for (int t = 1; t < BS; ++t) {
+#pragma unroll
+        for (int s0 = 0; s0 < t; s0 += 4) {
+            const f32x4 pp = *reinterpret_cast<lds_f32x4*>(pr + t * lda + s0);
+            const f32x4 pa = *reinterpret_cast<lds_f32x4*>(ar + t * lda + s0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int s = s0 + u;
+                if (s >= t) continue;
+                const float ex = kexp<PREC>(gt[t] - gt[s]), ks = kt[s] * ex;
+                ak[t] = fmaf(pp[u], ks, ak[t]);
+                aq[t] = fmaf(pa[u], ks, aq[t]);
+                const float z = ex * fmaf(pp[u], kt[t], pa[u] * qt[t]);
+                ak[s] += z;
+                const float c = z * kt[s];
+                ag[t] += c;
+                ag[s] -= c;
+            }
         }
-    }
+        // one row's pairs at a time: left alone, the compiler loads every row's
+        // coefficients first and spills 230 registers
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int rt = 4 * g4 + e;
-        res[(0 * BS + rt) * D + d] = ak[e];
-        res[(1 * BS + rt) * D + d] = aq[e];
-        res[(2 * BS + rt) * D + d] = ag[e];
+        for (int s = 0; s <= t; ++s) asm volatile("" : "+v"(ak[s]), "+v"(ag[s]));
+        asm volatile("" : "+v"(aq[t])::"memory");
     }
+    lds_f32* res = reinterpret_cast<lds_f32*>(wp) + BS * g4 * DT_P + r16;
+    wave_sync();   // every lane has read its k and q: the planes take their place
+#pragma unroll
+    for (int t = 0; t < BS; ++t) {
+        res[t * DT_P] = ak[t];
+        res[(C + t) * DT_P] = aq[t];
+        g[t * ldg] = ag[t];
+    }
+    wave_sync();
 }
 
 }  // namespace
@@ -117,7 +143,7 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
     static_assert(NW == NT && NB == 4, "one wave per channel tile, one thread per (channel, row block)");
     __shared__ WideLds<D> s;
     __shared__ __align__(16) float sp[C][C + 4];   // Akk, then dP = diag(beta) dL
-    __shared__ float sda[C][C + 4];         // dAqk (lower, with the diagonal)
+    __shared__ __align__(16) float sda[C][C + 4];   // dAqk (lower, with the diagonal)
     __shared__ __align__(16) float tii[NB][BS][BS + 4];
     __shared__ float sdb[NB + NT][C];       // dbeta partials: [j] from dL tiles of column block j, [NB + nt] channel tile nt
     __shared__ __align__(16) char pfbuf[256];   // landing bytes of the L2 prefetch
@@ -254,6 +280,35 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
     const int unsafe = __syncthreads_or(flag);
     const int strong = __syncthreads_or(sflag);
 
+    // L2 prefetch of the chunk this XCD starts next (chunk ids a CU count apart
+    // go to one XCD and start about when this one ends): its phase-0 inputs --
+    // the rows of q, k and g (two 128-byte lines a row) and A_kk and the
+    // inverses -- one 4-byte DMA per line, the landing bytes scratch.  Waves 0-1
+    // take q, 2-3 k, 4-5 g, 6-7 A_kk, and 32 lanes of wave 0 the inverses.  The
+    // addresses are formed here: a pick among the argument block's fields inside
+    // the instantiated phases put the block in scratch memory (224 -> 278 us).
+    const char *pfp = nullptr, *pfi = nullptr;
+    if (a.pf_ahead > 0 && ch + a.pf_ahead < (int)gridDim.x) {
+        const int pc = ch + a.pf_ahead, pbh = pc / a.nc, pn = pc - pbh * a.nc;
+        const int pb = pbh / a.H, ph = pbh - pb * a.H, pvalid = min(C, a.T - pn * C);
+        const size_t pbase = ((size_t)pb * a.T + (size_t)pn * C) * rs + (size_t)ph * dio;
+        const int grp = w >> 1, li = tid & 127, r = li >> 1;
+        if (grp == 3) {
+            pfp = reinterpret_cast<const char*>(a.Akk + (size_t)pc * C * C) + 128 * li;
+        } else if (r < pvalid) {
+            const char* tp = static_cast<const char*>(grp == 0 ? a.q : grp == 1 ? a.k : a.g);
+            const size_t es = (grp == 2) ? sizeof(TG) : sizeof(TI);
+            pfp = tp + (pbase + (size_t)r * rs) * es + 128 * (li & 1);
+        }
+        if (w == 0 && l < 32) pfi = reinterpret_cast<const char*>(a.Tii + (size_t)pc * NB * BS * BS) + 128 * l;
+    }
+    // The phases after the cumsum are instantiated twice, apart from here on: with
+    // the copies parting only at phase 4 the strong copy's diagonal tiles spilled
+    // the common one's registers.  SSv2 shape (8 x 1568 x 8 x 96): 224 -> 211 us
+    // within the guard, 417 -> 258 us at the layer's initial decay.  (Two
+    // kernels by a flag from the prep: 201 and 273 us, but fp32 551 -> 622.)
+    auto tail = [&](auto mode_c) __attribute__((always_inline)) {
+    constexpr int MODE = decltype(mode_c)::value;
     // wave w owns channel tile w: rows t = 16 m + 4 g4 + e, channel d
     const int nt = w, d = nt * BS + r16;
     // raw k, q of the lane's rows; el = e^{gamma_t - gamma_r} (r = 16 m), eb =
@@ -463,30 +518,10 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
     if constexpr (STG) tw.store(swu, LDQ);
     __syncthreads();
 
-    // L2 prefetch of the chunk this XCD starts next (chunk ids a CU count apart
-    // go to one XCD and start about when this one ends): its phase-0 inputs --
-    // the rows of q, k and g (two 128-byte lines a row) and A_kk and the
-    // inverses -- one 4-byte DMA per line, the landing bytes scratch.  Issued
-    // after this chunk's last global load, so that no wait of this chunk covers
-    // it, and waited for at the end.  Waves 0-1 take q, 2-3 k, 4-5 g, 6-7 A_kk,
-    // and 32 lanes of wave 0 the inverses (the pointer is picked per wave).
-    if (a.pf_ahead > 0 && ch + a.pf_ahead < (int)gridDim.x) {
-        const int pc = ch + a.pf_ahead, pbh = pc / a.nc, pn = pc - pbh * a.nc;
-        const int pb = pbh / a.H, ph = pbh - pb * a.H, pvalid = min(C, a.T - pn * C);
-        const size_t pbase = ((size_t)pb * a.T + (size_t)pn * C) * rs + (size_t)ph * dio;
-        const uint32_t m = lds_addr(pfbuf);
-        const int grp = w >> 1, li = tid & 127, r = li >> 1;
-        const char* p = nullptr;
-        if (grp == 3) {
-            p = reinterpret_cast<const char*>(a.Akk + (size_t)pc * C * C) + 128 * li;
-        } else if (r < pvalid) {
-            const char* tp = static_cast<const char*>(grp == 0 ? a.q : grp == 1 ? a.k : a.g);
-            const size_t es = (grp == 2) ? sizeof(TG) : sizeof(TI);
-            p = tp + (pbase + (size_t)r * rs) * es + 128 * (li & 1);
-        }
-        if (p) dma4(p, m);
-        if (w == 0 && l < 32) dma4(reinterpret_cast<const char*>(a.Tii + (size_t)pc * NB * BS * BS) + 128 * l, m);
-    }
+    // the L2 prefetch (pfp below): after this chunk's last global load, so that
+    // no wait of this chunk covers it; waited for at the end
+    if (pfp) dma4(pfp, lds_addr(pfbuf));
+    if (pfi) dma4(pfi, lds_addr(pfbuf));
 
     // ---------------- phase 3: dL = -tril(dR [W | U]^T, -1), one half of dR at a time ----------------
     // bf16: W and U are exact in bf16, so splitting only dR (PREC 2) keeps the
@@ -623,48 +658,42 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
             }
         }
         if constexpr (STRONG) {
-            // The diagonal tiles pair by pair within each block, with the exact
-            // weight e^{gamma_t - gamma_s} (s < t) from LDS gamma.  Everything the
-            // pair loops read comes from LDS -- the raw k and q rows (exact in
-            // bf16) staged in the free staging area -- and their sums go back
-            // there (per block: 16 rows x 3 planes, fp32), so the loops hold no
-            // per-lane arrays; each lane then adds its own rows' sums.
-            TI* const sk = st0;
-            TI* const sq = st1p;
-            float* const res = reinterpret_cast<float*>(stg + 2 * T_BYTES);   // [3][BS][D]
-            static_assert(2 * T_BYTES + 3 * BS * D * 4 <= STG_BYTES, "pair sums fit the staging area");
+            // The diagonal tiles pair by pair, in the wave's private part of the
+            // (then free) staging area; each lane then adds its own rows' sums.
+            unsigned char* const wp = stg + w * DT_BYTES;
+            static_assert(!STRONG || NW * DT_BYTES <= STG_BYTES, "the waves' private areas fit the staging area");
+            TI* const sk = reinterpret_cast<TI*>(wp) + r16;
 #pragma unroll
             for (int m = 0; m < NB; ++m)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int t = BS * m + 4 * g4 + e;
-                    st1<TI>(sk + t * LDQ + d, kx[m][e]);
-                    st1<TI>(sq + t * LDQ + d, qx[m][e]);
+                    st1<TI>(sk + t * DT_K, kx[m][e]);
+                    st1<TI>(sk + (C + t) * DT_K, qx[m][e]);
                 }
+            wave_sync();
+            wide_diag_tiles<PREC>((lds_f32*)&s.g[0][d], D + 4, (lds_u8*)wp, (const lds_f32*)&sp[0][0],
+                                  (const lds_f32*)&sda[0][0], C + 4, g4, r16);
+            const float* res = reinterpret_cast<const float*>(wp) + r16;
 #pragma unroll
-            for (int m = 0; m < NB; ++m) {
-                __syncthreads();   // staged rows visible; the previous block's sums read
-                wide_pair_block<D, TI, PREC>(&s.g[0][0], D + 4, sk, sq, LDQ, &sp[0][0], &sda[0][0], C + 4, res, m, g4,
-                                             d);
-                // the lane's own rows: written by itself above, no barrier needed
+            for (int m = 0; m < NB; ++m)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int rt = 4 * g4 + e;
-                    dka[m][e] += res[(0 * BS + rt) * D + d];
-                    dqa[m][e] += res[(1 * BS + rt) * D + d];
-                    dga[m][e] += res[(2 * BS + rt) * D + d];
+                    const int t = BS * m + 4 * g4 + e;
+                    dka[m][e] += res[t * DT_P];
+                    dqa[m][e] += res[(C + t) * DT_P];
+                    dga[m][e] += s.g[t][d];
                 }
-            }
         }
     };
-    // (fp32 operands: no room to stage k and q, so a chunk past the span guard
-    // takes the pair-by-pair path below)
-    if (!unsafe && !(strong && !STG)) {
-        if (STG && strong)
-            anchored(std::integral_constant<bool, STG>{});
-        else
-            anchored(std::false_type{});
-    } else {
+    // MODE 0: every block within the guard (the condition always holds: the
+    // branch keeps phase 4's loads and factors from being scheduled into its
+    // neighbours, 120 -> 30 spill accesses).  MODE 1: bf16 strong blocks, unless
+    // g > 0 or a NaN; everything else (fp32 operands have no room to stage k and
+    // q) takes the pair-by-pair path below
+    if (MODE == 0 ? valid > 0 : (STG && !unsafe)) {
+        anchored(std::integral_constant<bool, MODE == 1 && STG>{});
+    } else if constexpr (MODE == 1) {
         // pair by pair with the exact weight e^{gamma_t - gamma_s}: raw k and q of
         // the other rows from global memory, gamma from LDS
 #pragma unroll
@@ -752,6 +781,11 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
         for (int j = 0; j < NB + NT; ++j) db += sdb[j][tid];
         st1<TI>(static_cast<TI*>(a.dbeta) + bbase + (size_t)tid * a.H, db);
     }
+    };
+    if (__builtin_expect(!(unsafe | strong), 1))
+        tail(std::integral_constant<int, 0>{});
+    else
+        tail(std::integral_constant<int, 1>{});
     dma_wait<0>();   // the prefetch has landed before the workgroup's LDS is released
 }
 

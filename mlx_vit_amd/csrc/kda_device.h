@@ -739,6 +739,13 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// Order the wave's own LDS traffic: its DS operations execute in order, so
+// only the compiler has to be kept from moving them.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Swizzled LDS tiles: rows of RB bytes (a multiple of 16); the 16-byte chunk c
 // of row r is stored at chunk c ^ (r & M), M = min(RB / 16, 8) - 1, so that
 // the 16 rows an MFMA fragment read touches spread over the banks.

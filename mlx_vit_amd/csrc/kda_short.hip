@@ -27,13 +27,6 @@ namespace kda {
 
 namespace {
 
-// Order the wave's own LDS traffic: its DS operations execute in order, so
-// only the compiler has to be kept from moving them.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 __device__ __forceinline__ float uniform(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
