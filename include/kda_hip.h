@@ -330,8 +330,8 @@ size_t kda_layer_workspace_size(int which, int B, int T, int H, int D);
  * reduction), 9 gated RMSNorm (forward), 10 gated RMSNorm (backward, with its
  * reduction), 11-13 the segmented forward at D = 128 (bf16): 11 segment maps,
  * 12 segment start states, 13 the forward of every segment; 14 the backward's
- * state recompute and reverse carry in one launch (bf16 D = 128 without
- * segments: then ids 3 and 4 record nothing).  Sequences of at most 16 tokens
+ * state recompute and reverse carry in one launch (fp32, and bf16 D = 128
+ * without segments: then ids 3 and 4 record nothing).  Sequences of at most 16 tokens
  * at D <= 64 that run in one launch per direction record ids 1 and 5 only, and
  * use no workspace (its size does not change).
  * kda_profile_read must be called after the streams have completed. */

@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD_DIR = os.path.join(HERE, "_build")
 LIB_PATH = os.path.join(HERE, "libkda_hip.so")
 SOURCES = ["kda_fwd.hip", "kda_recur.hip", "kda_bwd.hip", "kda_layer.hip", "kda_api.hip", "kda_noalloc.hip", "kda_seg.hip", "kda_bwdw.hip", "kda_pad.hip", "kda_short.hip",
-           "kda_wgrad.hip"]
+           "kda_wgrad.hip", "kda_recur_f32.hip"]
 ARCH = os.environ.get("KDA_OFFLOAD_ARCH", "gfx950")
 
 # Packed-fp32 VALU ops are disabled for device code; the host pass warns that

@@ -664,7 +664,9 @@ int fwd_launch(int pass, const void* q, const void* k, const void* v, const void
     if (epi) {
         ra.z = epi->z; ra.ld_z = epi->ld_z; ra.nw = epi->w; ra.eps = epi->eps; ra.y = epi->y; ra.ld_y = epi->ld_y;
     }
-    e = timed(PROF_RECUR_FWD, st, [&] { return kda::launch_recur(ra, D, in_bf16, 0, st); }, prof);
+    e = timed(PROF_RECUR_FWD, st, [&] {
+        return in_bf16 ? kda::launch_recur(ra, D, 0, st) : kda::launch_recur_f32(ra, D, st);
+    }, prof);
     if (e != hipSuccess) return hip_fail(e, "kda_recur_kernel");
     return ok();
 }
@@ -766,16 +768,16 @@ int bwd_launch(int pass, const void* q, const void* k, const void* v, const void
         });
         if (e != hipSuccess) return hip_fail(e, "kda_segchain_kernel(states)");
     }
-    // bf16 D = 128 without segments: the state recompute shares one launch with
-    // the reverse carry below (kda_states_dh_kernel)
-    const bool merged = nseg == 1 && in_bf16 && D == 128;
+    // fp32, and bf16 D = 128 without segments: the state recompute shares one
+    // launch with the reverse carry below
+    const bool merged = nseg == 1 && (!in_bf16 || D == 128);
     kda::RecurArgs ra = {};
     if (nseg == 1) {
         ra.W = W; ra.U = U; ra.KbT = KbT; ra.eG = eG; ra.s0 = s0; ra.h = hS; ra.Vp = Vp;
         ra.Kb = region(ws, KDA_WS_KB);
         ra.T = T; ra.H = H; ra.nc = nc; ra.BH = BH;
         if (!merged) {
-            e = timed(PROF_RECUR_H, st, [&] { return kda::launch_recur(ra, D, in_bf16, 1, st); });
+            e = timed(PROF_RECUR_H, st, [&] { return kda::launch_recur(ra, D, 1, st); });
             if (e != hipSuccess) return hip_fail(e, "kda_recur_kernel");
         }
     }
@@ -812,9 +814,11 @@ int bwd_launch(int pass, const void* q, const void* k, const void* v, const void
             return r;
         });
     } else if (merged) {
-        e = timed(PROF_STATES_DH, st, [&] { return kda::launch_states_dh(ra, da, st); });
+        e = timed(PROF_STATES_DH, st, [&] {
+            return in_bf16 ? kda::launch_states_dh(ra, da, st) : kda::launch_states_dh_f32(ra, da, D, st);
+        });
     } else {
-        e = timed(PROF_DH, st, [&] { return kda::launch_dh(da, D, in_bf16, st); });
+        e = timed(PROF_DH, st, [&] { return kda::launch_dh(da, D, st); });
     }
     if (e != hipSuccess) return hip_fail(e, "kda_dh_kernel");
 

@@ -141,11 +141,16 @@ int device_cu_count(int dev);
 // g_kind: 0 fp32 g [B, T, H, D], 1 bf16 g, 2 one fp32 decay per (b, t, h),
 // g and dg [B, T, H] (GHead; bf16 inputs at D <= 64 only)
 hipError_t launch_prep(const PrepArgs& a, int D, int in_bf16, int g_kind, int nchunks, hipStream_t st);
-// mode 0: O and the final state (and y when a.y is set); 1: the chunk-start states h
-hipError_t launch_recur(const RecurArgs& a, int D, int in_bf16, int mode, hipStream_t st);
+// bf16; mode 0: O and the final state (and y when a.y is set); 1: the chunk-start
+// states h (D <= 64)
+hipError_t launch_recur(const RecurArgs& a, int D, int mode, hipStream_t st);
+// fp32 (kda_recur_f32.hip): the forward; the state recompute and the reverse carry in one launch
+hipError_t launch_recur_f32(const RecurArgs& a, int D, hipStream_t st);
+hipError_t launch_states_dh_f32(const RecurArgs& ra, const DhArgs& da, int D, hipStream_t st);
 // whether launch_recur can fuse the gated RMSNorm for this head size and dtype
 bool recur_epilogue_supported(int D, int in_bf16);
-hipError_t launch_dh(const DhArgs& a, int D, int in_bf16, hipStream_t st);
+// bf16, D <= 64
+hipError_t launch_dh(const DhArgs& a, int D, hipStream_t st);
 hipError_t launch_dh_seg_maps(const DhArgs& a, hipStream_t st);
 // bf16 D = 128: the state recompute (MODE 1) and the reverse carry in one launch
 hipError_t launch_states_dh(const RecurArgs& ra, const DhArgs& da, hipStream_t st);

@@ -25,8 +25,11 @@
 //   kda_recur3_kernel  bf16, D = 128 forward: four 4-wave workgroups per
 //       (batch, head), 32 dv columns each
 //   kda_recur2_kernel / kda_dh2_kernel  bf16, D = 32
-//   kda_recur_kernel / kda_dh_kernel    fp32 inputs (the first, generic design:
-//       one 256-thread workgroup per (batch, head), register-staged double buffer)
+//   kda_states_dh_kernel, kda_dh_kernel  bf16, D = 128: the backward's two
+//       recurrences in one launch, and the reverse carry over segments (the
+//       first, generic design: 256-thread workgroups on column slices of the
+//       state, register-staged double buffer)
+// fp32 inputs run the kernels of kda_recur_f32.hip.
 #include "kda_internal.h"
 
 namespace kda {
@@ -50,22 +53,20 @@ __device__ __forceinline__ Frag8 negfrag(Frag8 f) {
 // LDS geometry: NBUF operand sets (one chunk's slabs each) followed by NBUF
 // output staging tiles.  Rows are padded by 16 bytes against bank conflicts.
 // A workgroup owns DC = D / CS state columns; U and the outputs are DC wide.
-template <int D, typename ST, int MODE, int CS>
+template <int D, typename ST, int CS>
 struct RecurLayout {
     static constexpr int DC = D / CS;
     static constexpr int PS = 16 / (int)sizeof(ST);
     static constexpr int LDR = D + PS;               // rows of [C][D] / [D][D] tiles
     static constexpr int LDU = DC + PS;              // rows of [C][DC] tiles (U, outputs)
-    static constexpr int LDC = C + PS;               // rows of [D][C] / [C][C] tiles
+    static constexpr int LDC = C + PS;               // rows of [D][C] tiles
     static constexpr int W_OFF = 0;
     static constexpr int U_OFF = W_OFF + C * LDR;
-    static constexpr int QP_OFF = U_OFF + C * LDU;
-    static constexpr int KBT_OFF = QP_OFF + (MODE == 0 ? C * LDR : 0);
-    static constexpr int AQK_OFF = KBT_OFF + D * LDC;
-    static constexpr int SET_ELEMS = AQK_OFF + (MODE == 0 ? C * LDC : 0);
+    static constexpr int KBT_OFF = U_OFF + C * LDU;
+    static constexpr int SET_ELEMS = KBT_OFF + D * LDC;
     static constexpr int EG_BYTE = SET_ELEMS * (int)sizeof(ST);
     static constexpr int SET_BYTES = (EG_BYTE + D * 4 + 15) & ~15;
-    static constexpr int STG_ELEMS = (MODE == 0) ? C * LDU : D * LDU + C * LDU;   // O | h, V'
+    static constexpr int STG_ELEMS = D * LDU + C * LDU;   // h, V'
     static constexpr int STG_BYTES = (STG_ELEMS * (int)sizeof(ST) + 15) & ~15;
     static constexpr int NBUF = (2 * SET_BYTES + 2 * STG_BYTES <= 160 * 1024) ? 2 : 1;
     static constexpr int STG_OFF = NBUF * SET_BYTES;
@@ -105,22 +106,19 @@ struct DhLayout {
 //   wait for the loads, write them to LDS set (n+1)&1; barrier.
 // With NBUF = 1 an extra barrier separates the compute from the overwrite.
 // ----------------------------------------------------------------------------
-// The kernel body (kda_recur_kernel, kda_states_dh_kernel): workgroup wgi of
+// The state recompute's body (kda_states_dh_kernel): workgroup wgi of
 // the launch's recurrence workgroups, Lay::BYTES of LDS at smem.
-template <int D, typename ST, int PREC, int MODE, int CS, bool EPI = false>
+template <int D, typename ST, int PREC, int CS>
 __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* smem, const int wgi) {
-    using Lay = RecurLayout<D, ST, MODE, CS>;
+    using Lay = RecurLayout<D, ST, CS>;
     constexpr int NT = D / BS, DC = Lay::DC, NTW = DC / BS, TPW = (NTW + 3) / 4;
     constexpr int LDR = Lay::LDR, LDU = Lay::LDU, LDC = Lay::LDC;
 
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, r16 = l & 15, g4 = l >> 4;
     const int bh = wgi / CS, c0 = (wgi - bh * CS) * DC;
-    const int b = bh / a.H, h = bh - b * a.H;
     const ST* gW = static_cast<const ST*>(a.W);
     const ST* gU = static_cast<const ST*>(a.U);
-    const ST* gQp = static_cast<const ST*>(a.Qp);
     const ST* gKbT = static_cast<const ST*>(a.KbT);
-    const ST* gAqk = static_cast<const ST*>(a.Aqk);
 
     auto set = [&](int buf) __attribute__((always_inline)) { return reinterpret_cast<ST*>(smem + buf * Lay::SET_BYTES); };
     auto seg = [&](int buf) __attribute__((always_inline)) { return reinterpret_cast<float*>(smem + buf * Lay::SET_BYTES + Lay::EG_BYTE); };
@@ -150,10 +148,9 @@ __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* sm
             }
         }
 
-    Tile<ST, C, D> pW, pQp;
+    Tile<ST, C, D> pW;
     Tile<ST, C, DC> pU;
     Tile<ST, D, C> pKbT;
-    Tile<ST, C, C> pAqk;
     Tile<float, 1, D> pEg;
 
     auto issue = [&](int n) __attribute__((always_inline)) {
@@ -162,42 +159,18 @@ __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* sm
         pU.load(gU + ch * C * D + c0, D);
         pKbT.load(gKbT + ch * C * D, C);
         pEg.load(a.eG + ch * D, D);
-        if constexpr (MODE == 0) {
-            pQp.load(gQp + ch * C * D, D);
-            pAqk.load(gAqk + ch * C * C, C);
-        }
     };
     auto commit = [&](int buf) __attribute__((always_inline)) {
         pW.store(set(buf) + Lay::W_OFF, LDR);
         pU.store(set(buf) + Lay::U_OFF, LDU);
         pKbT.store(set(buf) + Lay::KBT_OFF, LDC);
         pEg.store(seg(buf), D);
-        if constexpr (MODE == 0) {
-            pQp.store(set(buf) + Lay::QP_OFF, LDR);
-            pAqk.store(set(buf) + Lay::AQK_OFF, LDC);
-        }
     };
     auto flush = [&](int n) __attribute__((always_inline)) {   // stores of chunk n's staged outputs
         const ST* sst = stg((Lay::NBUF == 2) ? (n & 1) : 0);
-        if constexpr (MODE == 0) {
-            const int t0 = n * C, valid = min(C, a.T - t0);
-            ST* go = static_cast<ST*>(a.o) + (((size_t)b * a.T + t0) * a.H + h) * D + c0;
-            if constexpr (EPI) {
-                // whole rows (CS = 1): the gated RMSNorm on the staged tile, z read here
-                static_assert(CS == 1, "the fused epilogue needs whole output rows");
-                const size_t rb = (size_t)b * a.T + t0;
-                tile_out_gated<ST, C, D>((int)threadIdx.x, sst, LDU, go, (size_t)a.H * D,
-                                         static_cast<ST*>(a.y) + rb * a.ld_y + (size_t)h * D, (size_t)a.ld_y,
-                                         static_cast<const ST*>(a.z) + rb * a.ld_z + (size_t)h * D,
-                                         (size_t)a.ld_z, a.nw, a.eps, valid);
-            } else {
-                tile_out<ST, C, DC>(sst, LDU, go, (size_t)a.H * D, valid);
-            }
-        } else {
-            const size_t ch = (size_t)bh * a.nc + n;
-            tile_out<ST, D, DC>(sst, LDU, static_cast<ST*>(a.h) + ch * D * D + c0, D, D);
-            tile_out<ST, C, DC>(sst + D * LDU, LDU, static_cast<ST*>(a.Vp) + ch * C * D + c0, D, C);
-        }
+        const size_t ch = (size_t)bh * a.nc + n;
+        tile_out<ST, D, DC>(sst, LDU, static_cast<ST*>(a.h) + ch * D * D + c0, D, D);
+        tile_out<ST, C, DC>(sst + D * LDU, LDU, static_cast<ST*>(a.Vp) + ch * C * D + c0, D, C);
     };
 
     issue(0);
@@ -218,7 +191,7 @@ __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* sm
 
         // All A fragments of this chunk are read from LDS first (one wait),
         // then the MFMA chain runs without LDS round trips in between.
-        Frag8 Aw[NB][D / 32], Akb[NT][C / 32], Aq[NB][D / 32], Aa[NB][C / 32];
+        Frag8 Aw[NB][D / 32], Akb[NT][C / 32];
 #pragma unroll
         for (int m = 0; m < NB; ++m)
 #pragma unroll
@@ -227,19 +200,8 @@ __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* sm
         for (int mt = 0; mt < NT; ++mt)
 #pragma unroll
             for (int ks = 0; ks < C / 32; ++ks) Akb[mt][ks] = ldfrag<PREC, ST>(sKbT, LDC, BS * mt, 32 * ks);
-        if constexpr (MODE == 0) {
-            const ST* sQp = set(buf) + Lay::QP_OFF;
-            const ST* sAqk = set(buf) + Lay::AQK_OFF;
-#pragma unroll
-            for (int m = 0; m < NB; ++m) {
-#pragma unroll
-                for (int ks = 0; ks < D / 32; ++ks) Aq[m][ks] = ldfrag<PREC, ST>(sQp, LDR, BS * m, 32 * ks);
-#pragma unroll
-                for (int ks = 0; ks <= m / 2; ++ks) Aa[m][ks] = ldfrag<PREC, ST>(sAqk, LDC, BS * m, 32 * ks);
-            }
-        }
         f32x4 Vp[TPW][NB];
-        Frag8 Bs[TPW][D / 32], Bn[TPW][D / 32];
+        Frag8 Bn[TPW][D / 32];
 #pragma unroll
         for (int j = 0; j < TPW; ++j) {
 #pragma unroll
@@ -247,10 +209,8 @@ __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* sm
 #pragma unroll
                 for (int e = 0; e < 4; ++e) Vp[j][m][e] = ld1<ST>(sU + (BS * m + 4 * g4 + e) * LDU + lcol[j]);
 #pragma unroll
-            for (int ks = 0; ks < D / 32; ++ks) {
-                Bs[j][ks] = accfrag<PREC>(S[j][2 * ks], S[j][2 * ks + 1]);
+            for (int ks = 0; ks < D / 32; ++ks)
                 Bn[j][ks] = accfrag<PREC>(negacc(S[j][2 * ks]), negacc(S[j][2 * ks + 1]));
-            }
         }
         __builtin_amdgcn_sched_barrier(0);
 
@@ -268,7 +228,7 @@ __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* sm
 #pragma unroll
             for (int ks = 0; ks < C / 32; ++ks) Bv[j][ks] = accfrag<PREC>(Vp[j][2 * ks], Vp[j][2 * ks + 1]);
 
-        // S <- diag(e^G) S + Kb^T V'  (issued before O: it is on the critical path)
+        // S <- diag(e^G) S + Kb^T V'
         f32x4 Snew[TPW][NT];
 #pragma unroll
         for (int mt = 0; mt < NT; ++mt) {
@@ -282,40 +242,20 @@ __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* sm
             }
         }
 
-        if constexpr (MODE == 0) {
-            // O = Qp S + Aqk V'
+        ST* hst = sst;
+        ST* vst = sst + D * LDU;
 #pragma unroll
-            for (int m = 0; m < NB; ++m) {
-                f32x4 O[TPW];
+        for (int j = 0; j < TPW; ++j)
+            if (has[j]) {
 #pragma unroll
-                for (int j = 0; j < TPW; ++j) {
-                    O[j] = zero4();
-                    if (has[j]) {
+                for (int mt = 0; mt < NT; ++mt)
 #pragma unroll
-                        for (int ks = 0; ks < D / 32; ++ks) O[j] = mma<PREC>(Aq[m][ks], Bs[j][ks], O[j]);
+                    for (int e = 0; e < 4; ++e) st1<ST>(hst + (BS * mt + 4 * g4 + e) * LDU + lcol[j], S[j][mt][e]);
 #pragma unroll
-                        for (int ks = 0; ks <= m / 2; ++ks) O[j] = mma<PREC>(Aa[m][ks], Bv[j][ks], O[j]);
+                for (int m = 0; m < NB; ++m)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) st1<ST>(sst + (BS * m + 4 * g4 + e) * LDU + lcol[j], O[j][e]);
-                    }
-                }
+                    for (int e = 0; e < 4; ++e) st1<ST>(vst + (BS * m + 4 * g4 + e) * LDU + lcol[j], Vp[j][m][e]);
             }
-        } else {
-            ST* hst = sst;
-            ST* vst = sst + D * LDU;
-#pragma unroll
-            for (int j = 0; j < TPW; ++j)
-                if (has[j]) {
-#pragma unroll
-                    for (int mt = 0; mt < NT; ++mt)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) st1<ST>(hst + (BS * mt + 4 * g4 + e) * LDU + lcol[j], S[j][mt][e]);
-#pragma unroll
-                    for (int m = 0; m < NB; ++m)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) st1<ST>(vst + (BS * m + 4 * g4 + e) * LDU + lcol[j], Vp[j][m][e]);
-                }
-        }
 #pragma unroll
         for (int j = 0; j < TPW; ++j)
 #pragma unroll
@@ -336,27 +276,11 @@ __device__ __forceinline__ void recur_body(const RecurArgs& a, unsigned char* sm
         }
     }
     if (Lay::NBUF == 2) flush(a.nc - 1);
-
-    if (MODE == 0 && a.s_final) {
-#pragma unroll
-        for (int j = 0; j < TPW; ++j)
-            if (has[j])
-#pragma unroll
-                for (int mt = 0; mt < NT; ++mt)
-                    *reinterpret_cast<float4*>(a.s_final + ((size_t)bh * D + col[j]) * D + BS * mt + 4 * g4) =
-                        make_float4(S[j][mt][0], S[j][mt][1], S[j][mt][2], S[j][mt][3]);
-    }
 }
 
 // ----------------------------------------------------------------------------
 // reverse state recurrence (same pipeline, chunks in reverse order)
 // ----------------------------------------------------------------------------
-template <int D, typename ST, int PREC, int MODE, int CS, bool EPI = false>
-__global__ __launch_bounds__(256) void kda_recur_kernel(const RecurArgs a) {
-    __shared__ __align__(16) unsigned char smem[RecurLayout<D, ST, MODE, CS>::BYTES];
-    recur_body<D, ST, PREC, MODE, CS, EPI>(a, smem, blockIdx.x);
-}
-
 // CS > 1: CS workgroups per (batch, head), DC = D / CS columns each; every A
 // fragment is then used by one column tile of a wave, so fragments are read
 // from LDS where they are used instead of being held for the whole chunk (at
@@ -621,11 +545,11 @@ __global__ __launch_bounds__(256) void kda_dh_kernel(const DhArgs a) {
 // run the reverse carry (two per (b, h), as kda_dh_kernel), side by side on
 // 4 BH CUs instead of one kernel after the other.
 __global__ __launch_bounds__(256) void kda_states_dh_kernel(const RecurArgs ra, const DhArgs da) {
-    constexpr int B1 = RecurLayout<128, uint16_t, 1, 2>::BYTES, B2 = DhLayout<128, uint16_t, 2>::BYTES;
+    constexpr int B1 = RecurLayout<128, uint16_t, 2>::BYTES, B2 = DhLayout<128, uint16_t, 2>::BYTES;
     __shared__ __align__(16) unsigned char smem[B1 > B2 ? B1 : B2];
     const int n1 = 2 * ra.BH;
     if ((int)blockIdx.x < n1)
-        recur_body<128, uint16_t, 1, 1, 2>(ra, smem, blockIdx.x);
+        recur_body<128, uint16_t, 1, 2>(ra, smem, blockIdx.x);
     else
         dh_body<128, uint16_t, 1, 2, 0>(da, smem, (int)blockIdx.x - n1);
 }
@@ -2337,79 +2261,36 @@ __global__ __launch_bounds__(512) void kda_dh4_kernel(const DhArgs a) {
 // ----------------------------------------------------------------------------
 // launchers
 // ----------------------------------------------------------------------------
-// D = 128 splits the state's dv columns over two workgroups per (batch, head)
-// bf16: row-split kernels with CS2 workgroups per (batch, head); fp32: one
-// workgroup per (batch, head), D = 128 split over two.
+// row-split kernels with CS2 workgroups per (batch, head)
 template <int D> struct RowSplit { static constexpr int CS = (D >= 128) ? 4 : 2; };
 
-template <int D, typename ST, int MODE>
+template <int D, int MODE>
 static hipError_t launch_recur_t(const RecurArgs& a, hipStream_t st) {
+    constexpr int CS2 = RowSplit<D>::CS;
     if (a.y != nullptr) {
-        // the forward with the gated RMSNorm fused into the O store: kernels whose
+        // the forward with the gated RMSNorm fused into the O store: a kernel whose
         // workgroup holds whole output rows
-        if constexpr (MODE == 0 && std::is_same<ST, uint16_t>::value && D == 64)
+        if constexpr (MODE == 0 && D == 64)
             hipLaunchKernelGGL((kda_recur5_kernel<D, true>), dim3(a.BH), dim3(1024), 0, st, a);
-        else if constexpr (MODE == 0 && std::is_same<ST, float>::value && D <= 64)
-            hipLaunchKernelGGL((kda_recur_kernel<D, ST, 3, 0, 1, true>), dim3(a.BH), dim3(256), 0, st, a);
         else
             return hipErrorInvalidValue;
         return hipGetLastError();
     }
-    if constexpr (std::is_same<ST, uint16_t>::value && D == 64) {
+    if constexpr (D == 64) {
         if (a.Kb == nullptr) return hipErrorInvalidValue;
-        constexpr int CS2 = RowSplit<D>::CS;
         hipLaunchKernelGGL((kda_recur4_kernel<D, MODE, CS2>), dim3(a.BH * CS2), dim3(512), 0, st, a);
-    } else if constexpr (std::is_same<ST, uint16_t>::value && D >= 64) {
-        constexpr int CS2 = RowSplit<D>::CS;
+    } else if constexpr (D > 64) {
         hipLaunchKernelGGL((kda_recur3_kernel<D, MODE, CS2>), dim3(a.BH * CS2), dim3(256), 0, st, a);
-    } else if constexpr (std::is_same<ST, uint16_t>::value) {
-        constexpr int CS2 = RowSplit<D>::CS;
+    } else {
         hipLaunchKernelGGL((kda_recur2_kernel<D, MODE, CS2>), dim3(a.BH * CS2), dim3(512), 0, st, a);
-    } else {
-        constexpr int CS = (D >= 128) ? 2 : 1;
-        hipLaunchKernelGGL((kda_recur_kernel<D, ST, 3, MODE, CS>), dim3(a.BH * CS), dim3(256), 0, st, a);
     }
     return hipGetLastError();
 }
 
-template <int D, typename ST>
-static hipError_t launch_dh_t(const DhArgs& a, hipStream_t st) {
-    if constexpr (std::is_same<ST, uint16_t>::value && D >= 64) {
-        if (!a.Aqk || !a.Qp || !a.W || !a.Kb) return hipErrorInvalidValue;
-        constexpr int CS2 = RowSplit<D>::CS;
-        hipLaunchKernelGGL((kda_dh4_kernel<D, CS2>), dim3(a.BH * CS2), dim3(512), 0, st, a);
-    } else if constexpr (std::is_same<ST, uint16_t>::value) {
-        constexpr int CS2 = RowSplit<D>::CS;
-        hipLaunchKernelGGL((kda_dh2_kernel<D, CS2>), dim3(a.BH * CS2), dim3(512), 0, st, a);
-    } else {
-        hipLaunchKernelGGL((kda_dh_kernel<D, ST, 3>), dim3(a.BH), dim3(256), 0, st, a);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_recur(const RecurArgs& a, int D, int in_bf16, int mode, hipStream_t st) {
-#define KDA_RECUR_CASE(DD)                                                                        \
-    if (D == DD) {                                                                                \
-        if (mode == 0) return in_bf16 ? launch_recur_t<DD, uint16_t, 0>(a, st)                    \
-                                      : launch_recur_t<DD, float, 0>(a, st);                      \
-        return in_bf16 ? launch_recur_t<DD, uint16_t, 1>(a, st) : launch_recur_t<DD, float, 1>(a, st); \
-    }
-    KDA_RECUR_CASE(32)
-    KDA_RECUR_CASE(64)
-#undef KDA_RECUR_CASE
-    if (D == 128 && mode == 0)
-        return in_bf16 ? launch_recur_t<128, uint16_t, 0>(a, st) : launch_recur_t<128, float, 0>(a, st);
-    // the backward's state recompute at D = 128: the generic kernel, which also
-    // writes V' for the D = 128 local-adjoint kernel; two workgroups per
-    // (batch, head), 64 dv columns each
-    if (D == 128 && mode == 1) {
-        if (a.Vp == nullptr || a.KbT == nullptr) return hipErrorInvalidValue;
-        if (in_bf16)
-            hipLaunchKernelGGL((kda_recur_kernel<128, uint16_t, 1, 1, 2>), dim3(a.BH * 2), dim3(256), 0, st, a);
-        else
-            hipLaunchKernelGGL((kda_recur_kernel<128, float, 3, 1, 2>), dim3(a.BH * 2), dim3(256), 0, st, a);
-        return hipGetLastError();
-    }
+hipError_t launch_recur(const RecurArgs& a, int D, int mode, hipStream_t st) {
+    if (D == 32) return mode == 0 ? launch_recur_t<32, 0>(a, st) : launch_recur_t<32, 1>(a, st);
+    if (D == 64) return mode == 0 ? launch_recur_t<64, 0>(a, st) : launch_recur_t<64, 1>(a, st);
+    if (D == 128 && mode == 0) return launch_recur_t<128, 0>(a, st);
     return hipErrorInvalidValue;
 }
 
@@ -2436,19 +2317,14 @@ hipError_t launch_states_dh(const RecurArgs& ra, const DhArgs& da, hipStream_t s
     return hipGetLastError();
 }
 
-hipError_t launch_dh(const DhArgs& a, int D, int in_bf16, hipStream_t st) {
-    if (D == 32) return in_bf16 ? launch_dh_t<32, uint16_t>(a, st) : launch_dh_t<32, float>(a, st);
-    if (D == 64) return in_bf16 ? launch_dh_t<64, uint16_t>(a, st) : launch_dh_t<64, float>(a, st);
-    // D = 128: the generic kernel on the transposed slabs; bf16: two workgroups
-    // per (batch, head), 64 dS columns each (one column tile per wave); fp32:
-    // four, 32 dS columns each (one operand set and its staging fit the LDS
-    // only at that width)
-    if (D == 128) {
-        if (!a.AqkT || !a.QpT || !a.WT || !a.Kb) return hipErrorInvalidValue;
-        if (in_bf16)
-            hipLaunchKernelGGL((kda_dh_kernel<128, uint16_t, 1, 2>), dim3(a.BH * 2), dim3(256), 0, st, a);
-        else
-            hipLaunchKernelGGL((kda_dh_kernel<128, float, 3, 4>), dim3(a.BH * 4), dim3(256), 0, st, a);
+hipError_t launch_dh(const DhArgs& a, int D, hipStream_t st) {
+    if (D == 32) {
+        hipLaunchKernelGGL((kda_dh2_kernel<32, RowSplit<32>::CS>), dim3(a.BH * RowSplit<32>::CS), dim3(512), 0, st, a);
+        return hipGetLastError();
+    }
+    if (D == 64) {
+        if (!a.Aqk || !a.Qp || !a.W || !a.Kb) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((kda_dh4_kernel<64, RowSplit<64>::CS>), dim3(a.BH * RowSplit<64>::CS), dim3(512), 0, st, a);
         return hipGetLastError();
     }
     return hipErrorInvalidValue;
