@@ -315,6 +315,14 @@ typedef struct kda_pack_job {
 } kda_pack_job;
 int kda_layer_pack(const kda_pack_job* jobs, int count, void* stream);
 
+/* The scalar-alpha decay as the kernels take it: g[i] = max(log(alpha[i]), g_min),
+ * fp32, for n values alpha of dtype; and its adjoint dalpha[i] = dg[i] /
+ * alpha[i] where log(alpha[i]) >= g_min, else 0 (nope_gdn_mlx.py:641-650 applies
+ * alpha itself). */
+int kda_log_decay_fwd(const void* alpha, float* g, int64_t n, float g_min, int dtype, void* stream);
+int kda_log_decay_bwd(const void* alpha, const float* dg, void* dalpha, int64_t n, float g_min, int dtype,
+                      void* stream);
+
 #define KDA_LAYER_PRODUCER 0
 #define KDA_LAYER_RMSNORM 1
 size_t kda_layer_workspace_size(int which, int B, int T, int H, int D);

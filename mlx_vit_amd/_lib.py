@@ -58,6 +58,8 @@ SIGNATURES = {
     "kda_weight_grad_workspace_size": ([_P, _I, _I], _Z),
     "kda_weight_grad": ([_P, _I, _I, _P, _Z, _P], _I),
     "kda_layer_pack": ([_P, _I, _P], _I),
+    "kda_log_decay_fwd": ([_P, _P, _L, _F, _I, _P], _I),
+    "kda_log_decay_bwd": ([_P, _P, _P, _L, _F, _I, _P], _I),
     "kda_layer_workspace_size": ([_I] * 5, _Z),
     "kda_profile_enable": ([_I], _I),
     "kda_profile_name": ([_I], ctypes.c_char_p),

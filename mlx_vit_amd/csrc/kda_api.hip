@@ -1281,6 +1281,31 @@ int kda_layer_pack(const kda_pack_job* jobs, int count, void* stream) {
     return e == hipSuccess ? ok() : hip_fail(e, "kda_layer_pack");
 }
 
+static int log_decay(const void* alpha, float* g, const float* dg, void* dalpha, int64_t n, float g_min, int dtype,
+                     void* stream) {
+    if (dtype != KDA_DTYPE_F32 && dtype != KDA_DTYPE_BF16)
+        return fail(KDA_E_UNSUPPORTED, "dtype=%d: expected 0 (fp32) or 1 (bf16)", dtype);
+    if (n < 0) return fail(KDA_E_INVALID, "n=%lld", (long long)n);
+    if (n == 0) return ok();
+    KDA_TRY(check_scalar(alpha, "alpha", dtype));
+    if (dalpha) KDA_TRY(check_scalar(dalpha, "dalpha", dtype));
+    const hipError_t e = kda::launch_log_decay(alpha, g, dg, dalpha, (size_t)n, g_min, dtype == KDA_DTYPE_BF16,
+                                               static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? ok() : hip_fail(e, "kda_log_decay");
+}
+
+int kda_log_decay_fwd(const void* alpha, float* g, int64_t n, float g_min, int dtype, void* stream) {
+    if (n > 0) KDA_TRY(check_f32(g, "g", 4, false));
+    return log_decay(alpha, g, nullptr, nullptr, n, g_min, dtype, stream);
+}
+
+int kda_log_decay_bwd(const void* alpha, const float* dg, void* dalpha, int64_t n, float g_min, int dtype,
+                      void* stream) {
+    if (n > 0) KDA_TRY(check_f32(dg, "dg", 4, false));
+    if (n > 0 && !dalpha) return fail(KDA_E_INVALID, "dalpha is NULL");
+    return log_decay(alpha, nullptr, dg, dalpha, n, g_min, dtype, stream);
+}
+
 size_t kda_layer_workspace_size(int which, int B, int T, int H, int D) {
     if (B < 0 || T < 0 || H < 1 || D < 1) return 0;
     if (which == KDA_LAYER_PRODUCER) return kda::producer_ws_floats(B, T, H, D) * sizeof(float);

@@ -203,6 +203,9 @@ struct PackJob {
     int64_t n, dtypes;
 };
 hipError_t launch_pack(const PackJob* jobs, int count, hipStream_t st);
+// g = max(log alpha, g_min); dg non-null: dalpha instead
+hipError_t launch_log_decay(const void* alpha, float* g, const float* dg, void* dalpha, size_t n, float g_min,
+                            int in_bf16, hipStream_t st);
 
 // GatedDeltaLayer producer (projection outputs -> q, k, v, g, beta) and its
 // adjoint.  Row strides are in elements; q, k, v, g, dq, dk, dv, dg are

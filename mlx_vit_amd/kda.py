@@ -42,7 +42,9 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream(dev: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    """The current stream's handle (without building a Stream object)."""
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if dev.index is None else dev.index))
 
 
 def head_decay_supported(D: int, dtype: torch.dtype) -> bool:
@@ -345,6 +347,34 @@ def chunk_kda(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor
 GDN_LOG_ALPHA_MIN = -80.0
 
 
+class LogDecayFunction(torch.autograd.Function):
+    """g = max(log(alpha), GDN_LOG_ALPHA_MIN) in fp32, one launch each way."""
+
+    @staticmethod
+    def forward(ctx, alpha):
+        a = alpha.contiguous()
+        g = torch.empty(a.shape, dtype=torch.float32, device=a.device)
+        _lib.check(_lib.load().kda_log_decay_fwd(_ptr(a), _ptr(g), a.numel(), GDN_LOG_ALPHA_MIN, _DTYPE_CODE[a.dtype],
+                                                 _stream(a.device)), "kda_log_decay_fwd")
+        ctx.save_for_backward(a)
+        return g
+
+    @staticmethod
+    def backward(ctx, dg):
+        (a,) = ctx.saved_tensors
+        dg = dg.to(torch.float32).contiguous()
+        da = torch.empty_like(a)
+        _lib.check(_lib.load().kda_log_decay_bwd(_ptr(a), _ptr(dg), _ptr(da), a.numel(), GDN_LOG_ALPHA_MIN,
+                                                 _DTYPE_CODE[a.dtype], _stream(a.device)), "kda_log_decay_bwd")
+        return da
+
+
+def _log_alpha(alpha: torch.Tensor) -> torch.Tensor:
+    if alpha.device.type == "cuda" and alpha.dtype in _DTYPE_CODE:
+        return LogDecayFunction.apply(alpha)
+    return torch.clamp(torch.log(alpha.float()), min=GDN_LOG_ALPHA_MIN)
+
+
 def chunk_gdn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, alpha: torch.Tensor, beta: torch.Tensor,
               initial_state: Optional[torch.Tensor] = None, chunk_size: int = CHUNK
               ) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -362,7 +392,7 @@ def chunk_gdn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, alpha: torch.Te
     Autograd through the log (and the broadcast) gives d alpha = sum_d dg / alpha."""
     if alpha.dim() != 3 or tuple(alpha.shape) != tuple(q.shape[:3]):
         raise ValueError(f"alpha must be (B, T, H) = {tuple(q.shape[:3])}; got {tuple(alpha.shape)}")
-    g = torch.clamp(torch.log(alpha.float()), min=GDN_LOG_ALPHA_MIN)
+    g = _log_alpha(alpha)
     if not (q.dim() == 4 and head_decay_supported(q.shape[-1], q.dtype)):
         g = g.unsqueeze(-1).expand(q.shape).contiguous()
     return chunk_kda(q, k, v, g, beta, initial_state, chunk_size)

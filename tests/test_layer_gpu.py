@@ -491,3 +491,28 @@ def test_layer_one_node_matches_modules(H, D, L, frozen, contiguous):
     for n, g in one.items():
         assert g.dtype == mods[n].dtype and g.shape == mods[n].shape, n
     _check(errs, 1e-2, f"one node H={H} D={D} L={L}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 255, 1000])
+def test_log_decay(n, dtype):
+    """The scalar decay's logarithm and its adjoint against torch's clamp(log) on
+    the same values, alpha = 0, the clamp's edge and alpha = 1 among them, and a
+    strided alpha: g to one fp32 rounding of the logarithm, d alpha to alpha's
+    own rounding."""
+    from mlx_vit_amd.kda import GDN_LOG_ALPHA_MIN, _log_alpha
+    gen = torch.Generator().manual_seed(n)
+    a = torch.rand(2 * n, generator=gen)
+    a[:8] = torch.tensor([0.0, 1.0, 0.5, 1e-38, 1e-30, 0.999, 1e-35, 1e-34])[:min(8, 2 * n)]
+    al = a.to(dtype).to(DEV)[::2].requires_grad_()
+    ref = al.detach().clone().requires_grad_()
+    dg = torch.randn(n, generator=gen).to(DEV)
+    g = _log_alpha(al)
+    (da,) = torch.autograd.grad(g, al, dg)
+    gr = torch.clamp(torch.log(ref.float()), min=GDN_LOG_ALPHA_MIN)
+    (dr,) = torch.autograd.grad(gr, ref, dg)
+    torch.cuda.synchronize()
+    assert torch.allclose(g, gr, rtol=2.0 ** -22, atol=2.0 ** -23)
+    fin = torch.isfinite(dr.float())
+    assert torch.equal(fin, torch.isfinite(da.float()))
+    assert torch.allclose(da.float()[fin], dr.float()[fin], rtol=2.0 ** (-8 if dtype == torch.bfloat16 else -22), atol=0.0)
