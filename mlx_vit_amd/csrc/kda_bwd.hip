@@ -1,10 +1,11 @@
 // kda_bwd.hip -- backward kernels of the KDA chunkwise WY recurrence (gfx950).
 //
 // The backward stores no per-step state.  The forward's chunk-boundary states
-// are recomputed (prep + kda_recur_kernel MODE 1), the reverse state carry
-// (kda_dh_kernel, kda_recur.hip) stores dS at each chunk end and dV', then:
+// are recomputed (the prep and the states recurrence), the reverse state carry
+// stores dS at each chunk end and dV' (kda_recur.hip, kda_recur_f32.hip), then:
 //
-//   kda_bwd_local3_kernel (bf16 operands) / kda_bwd_local_kernel (fp32 operands)
+//   kda_bwd_local3_kernel (bf16 operands, D <= 64) / kda_bwd_localw_kernel
+//                     (kda_bwdw.hip: fp32 operands and D = 128)
 //                     one workgroup per chunk, fully parallel: every remaining
 //                     adjoint of the chunk -- output / state products, the
 //                     transposed WY solve (nope_gdn_mlx.py:2637-2641, as block
@@ -22,23 +23,6 @@ namespace kda {
 // local adjoints
 // ----------------------------------------------------------------------------
 
-// rows of a (B, T, H, D) tensor as an A operand; rows at or past `valid` read as zero
-template <typename TI>
-__device__ __forceinline__ Fr8 frag8_rows(const TI* base, size_t rstride, int row0, int k0, int valid) {
-    const int l = lane_id(), r = l & 15, g = l >> 4;
-    Fr8 f;
-    if (row0 + r < valid) {
-        const TI* p = base + (size_t)(row0 + r) * rstride + k0 + 4 * g;
-        const float4 x = ld4<TI>(p), y = ld4<TI>(p + 16);
-        f.v[0] = x.x; f.v[1] = x.y; f.v[2] = x.z; f.v[3] = x.w;
-        f.v[4] = y.x; f.v[5] = y.y; f.v[6] = y.z; f.v[7] = y.w;
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f.v[e] = 0.f;
-    }
-    return f;
-}
-
 // sum over the 16 lanes that share a lane group (same l/16)
 __device__ __forceinline__ float sum16(float x) {
     x += __shfl_xor(x, 1, 64);
@@ -54,355 +38,8 @@ __device__ __forceinline__ float sum4g(float x) {
     return x;
 }
 
-template <int D, typename TI, typename TG, int PREC>
-__global__ __launch_bounds__(256) void kda_bwd_local_kernel(const LocalArgs a) {
-    constexpr int NT = D / BS;
-    __shared__ ChunkLds<D> s;
-    __shared__ float sp[C][C + 4];           // Akk, then dP = diag(beta) dL
-    __shared__ float sda[C][C + 4];          // dAqk
-    __shared__ float sdr[C][2 * D + 4];      // dR = (I + L)^-T [dW | dU]
-    __shared__ float tii[NB][BS][BS + 4];
-    __shared__ float sdb[NB + NT][C];        // dbeta partials: [j] from dL tiles of column block j, [NB + nt] from channel tile nt
-
-    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, r16 = l & 15, g4 = l >> 4;
-    const int ch = blockIdx.x, bh = ch / a.nc, n = ch - bh * a.nc;
-    const int b = bh / a.H, h = bh - b * a.H;
-    const int t0 = n * C, valid = min(C, a.T - t0);
-    const size_t rs = (size_t)a.H * D;
-    const size_t base = ((size_t)b * a.T + t0) * rs + (size_t)h * D;
-    const size_t bbase = ((size_t)b * a.T + t0) * a.H + h;
-    const TI* q = static_cast<const TI*>(a.q);
-    const TI* k = static_cast<const TI*>(a.k);
-    const TI* v = static_cast<const TI*>(a.v);
-    const TG* g = static_cast<const TG*>(a.g);
-    const TI* beta = static_cast<const TI*>(a.beta);
-    const TI* dout = static_cast<const TI*>(a.dout);
-    const size_t cCD = (size_t)ch * C * D, cCC = (size_t)ch * C * C;
-    const TI* hS = static_cast<const TI*>(a.h) + (size_t)ch * D * D;
-    const TI* dhS = static_cast<const TI*>(a.dh) + (size_t)ch * D * D;
-    const TI* Vp = static_cast<const TI*>(a.Vp) + cCD;
-    const TI* dVp = static_cast<const TI*>(a.dVp) + cCD;
-    const TI* Wc = static_cast<const TI*>(a.W) + cCD;
-    const TI* Uc = static_cast<const TI*>(a.U) + cCD;
-
-    // ---------------- phase 0: chunk factors, raw per-lane values ----------------
-    for (int idx = tid; idx < C * C; idx += 256) sp[idx / C][idx % C] = a.Akk[cCC + idx];
-    for (int idx = tid; idx < NB * BS * BS; idx += 256) {
-        const int i = idx / (BS * BS), e = idx - i * BS * BS;
-        tii[i][e / BS][e % BS] = a.Tii[(size_t)ch * NB * BS * BS + idx];
-    }
-    for (int idx = tid; idx < (NB + NT) * C; idx += 256) sdb[idx / C][idx % C] = 0.f;
-    int flag = chunk_load<D, TI, TG>(s, q, k, g, beta, base, rs, bbase, a.H, valid);
-    chunk_cumsum<D>(s);
-    const int unsafe = chunk_factors<D, PREC>(s, flag);
-    if (unsafe) chunk_band<D, 256>(s, __syncthreads_or(flag));
-
-    // wave w owns channel tile nt = w: rows t = 16 m + 4 g4 + e, channel d
-    const int nt = w;
-    const bool own = nt < NT;
-    const int d = own ? nt * BS + r16 : 0;
-    float kx[NB][4], qx[NB][4], el[NB][4], er[NB][4], eb[NB][4], erb[NB];
-    if (own) {
-        const float G = s.g[C - 1][d];
-#pragma unroll
-        for (int m = 0; m < NB; ++m) {
-            const float gr = s.g[BS * m][d];
-            erb[m] = s.er[m][d];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int t = BS * m + 4 * g4 + e;
-                const float gt = s.g[t][d];
-                kx[m][e] = s.kr[t][d];
-                qx[m][e] = s.ql[t][d];
-                el[m][e] = kexp<PREC>(gt - gr);
-                er[m][e] = unsafe ? 0.f : kexp<PREC>(gr - gt);
-                eb[m][e] = kexp<PREC>(G - gt);
-            }
-        }
-    }
-    __syncthreads();
-    if (!unsafe) chunk_transform<D, PREC>(s, true);
-    __syncthreads();
-    // PHASE 1
-
-    f32x4 dqa[NB], dka[NB], dga[NB], dWt[NB];
-#pragma unroll
-    for (int m = 0; m < NB; ++m) { dqa[m] = zero4(); dka[m] = zero4(); dga[m] = zero4(); dWt[m] = zero4(); }
-    float dgcol = 0.f;
-
-    // ---------------- phase 1: products over dv ----------------
-    if (own) {
-#pragma unroll
-        for (int m = 0; m < NB; ++m) {
-            f32x4 dQp = zero4(), dKb = zero4(), dW = zero4();
-#pragma unroll
-            for (int ks = 0; ks < D / 32; ++ks) {
-                const Fr8 Bh = frag8(hS, D, BS * nt, 32 * ks);
-                const Fr8 Bdh = frag8(dhS, D, BS * nt, 32 * ks);
-                dQp = mma8<PREC>(frag8_rows<TI>(dout + base, rs, BS * m, 32 * ks, valid), Bh, dQp);
-                dKb = mma8<PREC>(frag8(Vp, D, BS * m, 32 * ks), Bdh, dKb);
-                dW = mma8<PREC>(neg(frag8(dVp, D, BS * m, 32 * ks)), Bh, dW);
-            }
-            dWt[m] = dW;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float egt = erb[m] * el[m][e];                 // e^{gamma_t}
-                dqa[m][e] = dQp[e] * egt;
-                dka[m][e] = dKb[e] * eb[m][e];
-                const float kbv = kx[m][e] * eb[m][e];
-                dga[m][e] = dQp[e] * qx[m][e] * egt - dKb[e] * kbv;
-                dgcol += dKb[e] * kbv;
-            }
-        }
-        // state-decay term of dG: e^G sum_col dh[d][col] h[d][col]
-        float part = 0.f;
-        for (int c = g4 * (D / 4); c < (g4 + 1) * (D / 4); ++c)
-            part += ld1<TI>(dhS + (size_t)d * D + c) * ld1<TI>(hS + (size_t)d * D + c);
-        dgcol = sum4g(dgcol) + kexp<PREC>(s.g[C - 1][d]) * sum4g(part);
-    }
-    // dAqk = tril(dO V'^T), 10 lower tiles over the 4 waves
-    for (int tix = w; tix < 10; tix += 4) {
-        int i, j;
-        tile_ij(tix, i, j);
-        f32x4 acc = zero4();
-#pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks)
-            acc = mma8<PREC>(frag8_rows<TI>(dout + base, rs, BS * i, 32 * ks, valid), frag8(Vp, D, BS * j, 32 * ks), acc);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int t = BS * i + 4 * g4 + e, sx = BS * j + r16;
-            sda[t][sx] = (sx <= t) ? acc[e] : 0.f;
-        }
-    }
-    __syncthreads();
-
-    // PHASE 2
-    // ---------------- phase 2: transposed WY solve ----------------
-    if (own) {
-        f32x4 dRk[NB], dRv[NB];
-#pragma unroll
-        for (int i = NB - 1; i >= 0; --i) {
-            f32x4 Yk = dWt[i], Yv;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) Yv[e] = ld1<TI>(dVp + (size_t)(BS * i + 4 * g4 + e) * D + d);
-#pragma unroll
-            for (int j = i + 1; j < NB; ++j) {
-                // A[a][b] = -L[16j + b][16i + a] = -beta_{16j+b} Akk[16j+b][16i+a]
-                Fr4 A;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int rb = BS * j + 4 * g4 + e;
-                    A.v[e] = -s.beta[rb] * sp[rb][BS * i + r16];
-                }
-                Yk = mma4<3>(A, acc2frag4(dRk[j]), Yk);
-                Yv = mma4<3>(A, acc2frag4(dRv[j]), Yv);
-            }
-            const Fr4 Tt = frag4T(&tii[i][0][0], BS + 4, 0, 0);     // A[a][b] = T_ii[b][a]
-            dRk[i] = mma4<3>(Tt, acc2frag4(Yk), zero4());
-            dRv[i] = mma4<3>(Tt, acc2frag4(Yv), zero4());
-        }
-        TI* dv = static_cast<TI*>(a.dv);
-#pragma unroll
-        for (int m = 0; m < NB; ++m) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int t = BS * m + 4 * g4 + e;
-                const float bt = s.beta[t];
-                const float egt = erb[m] * el[m][e];
-                const float vv = (t < valid) ? ld1<TI>(v + base + (size_t)t * rs + d) : 0.f;
-                if (t < valid) st1<TI>(dv + base + (size_t)t * rs + d, bt * dRv[m][e]);
-                dka[m][e] += bt * egt * dRk[m][e];
-                dga[m][e] += dRk[m][e] * bt * egt * kx[m][e];
-                const float db = sum16(dRv[m][e] * vv + dRk[m][e] * egt * kx[m][e]);
-                if (r16 == 0) sdb[NB + nt][t] = db;
-                sdr[t][d] = dRk[m][e];
-                sdr[t][D + d] = dRv[m][e];
-            }
-        }
-    }
-    __syncthreads();
-
-    // PHASE 3
-    // ---------------- phase 3: dL = -tril(dR X^T, -1); dbeta; dP ----------------
-    for (int tix = w; tix < 10; tix += 4) {
-        int i, j;
-        tile_ij(tix, i, j);
-        f32x4 acc = zero4();
-#pragma unroll
-        for (int ks = 0; ks < 2 * D / 32; ++ks) {
-            const Fr8 A = frag8(&sdr[0][0], 2 * D + 4, BS * i, 32 * ks);
-            const Fr8 B = (32 * ks < D) ? frag8(Wc, D, BS * j, 32 * ks) : frag8(Uc, D, BS * j, 32 * ks - D);
-            acc = mma8<3>(A, B, acc);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int t = BS * i + 4 * g4 + e, sx = BS * j + r16;
-            const float dL = (sx < t) ? -acc[e] : 0.f;
-            const float db = sum16(dL * sp[t][sx]);
-            if (r16 == 0) sdb[j][t] = db;
-            sp[t][sx] = s.beta[t] * dL;
-        }
-    }
-    __syncthreads();
-
-    // PHASE 4
-    // ---------------- phase 4: decay-masked K K^T / Q K^T adjoints ----------------
-    if (own) {
-        if (!unsafe) {
-            // row and column sides of a pair must agree to fp32 (see below): exact split products
-            constexpr int PX = PREC >= 3 ? 4 : PREC;
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                f32x4 dKl = zero4(), dQl = zero4();
-#pragma unroll
-                for (int j = 0; j <= i; ++j) {
-                    const float fs = (j < i) ? s.f[pair_idx(i, j)][d] : 1.f;
-                    Fr4 B;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) B.v[e] = s.kr[BS * j + 4 * g4 + e][d] * fs;
-                    dKl = mma4<PX>(frag4(&sp[0][0], C + 4, BS * i, BS * j), B, dKl);
-                    Fr4 Aq = frag4(&sda[0][0], C + 4, BS * i, BS * j);
-                    if (j == i) {   // the diagonal pairs (t, t) are added apart, below
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (4 * g4 + e == r16) Aq.v[e] = 0.f;
-                    }
-                    dQl = mma4<PX>(Aq, B, dQl);
-                }
-                Fr4 Bk, Bq;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    Bk.v[e] = s.kl[BS * i + 4 * g4 + e][d];
-                    Bq.v[e] = s.ql[BS * i + 4 * g4 + e][d];
-                }
-                // The row-t and column-s contributions of each pair (t, s) to dgamma
-                // cancel in the reverse cumsum below; weight each side by the very
-                // operand values the other side's MFMA used (split to PREC), so that
-                // the cancellation is exact to fp32 and the error stays independent
-                // of the block's decay span.
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    dka[i][e] += dKl[e] * el[i][e];
-                    dqa[i][e] += dQl[e] * el[i][e];
-                    dga[i][e] += dKl[e] * mfma_operand<PREC>(Bk.v[e]) + dQl[e] * mfma_operand<PREC>(Bq.v[e]);
-                }
-#pragma unroll
-                for (int j = 0; j <= i; ++j) {
-                    f32x4 dKr = mma4<PX>(frag4T(&sp[0][0], C + 4, BS * j, BS * i), Bk, zero4());
-                    Fr4 Aq = frag4T(&sda[0][0], C + 4, BS * j, BS * i);
-                    if (j == i) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (4 * g4 + e == r16) Aq.v[e] = 0.f;
-                    }
-                    dKr = mma4<PX>(Aq, Bq, dKr);
-                    const float fs = (j < i) ? s.f[pair_idx(i, j)][d] : 1.f;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float fac = fs * er[j][e];
-                        dka[j][e] += dKr[e] * fac;
-                        // the row side's B operand for this s and block pair
-                        dga[j][e] -= dKr[e] * mfma_operand<PREC>(s.kr[BS * j + 4 * g4 + e][d] * fs);
-                    }
-                }
-            }
-        } else {
-            // pairwise path: raw k in s.kr, raw q in s.ql, gamma in s.g
-#pragma unroll
-            for (int m = 0; m < NB; ++m) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int t = BS * m + 4 * g4 + e;
-                    const float gt = s.g[t][d];
-                    float ak = 0.f, aq = 0.f, ag = 0.f;
-                    // row t (dP[t][sx] strict, dA[t][sx]) and column t (dP[sx][t],
-                    // dA[sx][t]) as two loops over the decay band
-                    for (int sx = s.blo[t]; sx < t; ++sx) {
-                        const float ks = s.kr[sx][d] * kexp<PREC>(gt - s.g[sx][d]);
-                        const float pp = sp[t][sx], pa = sda[t][sx];
-                        ak += pp * ks;
-                        aq += pa * ks;
-                        ag += (pp * kx[m][e] + pa * qx[m][e]) * ks;
-                    }
-                    for (int sx = t + 1; sx <= s.bhi[t]; ++sx) {
-                        const float ex = kexp<PREC>(s.g[sx][d] - gt);
-                        const float pp = sp[sx][t], pa = sda[sx][t];
-                        const float c = (pp * s.kr[sx][d] + pa * s.ql[sx][d]) * ex;
-                        ak += c;
-                        ag -= c * kx[m][e];
-                    }
-                    dka[m][e] += ak;
-                    dqa[m][e] += aq;
-                    dga[m][e] += ag;
-                }
-            }
-        }
-        // The diagonal pairs (t, t) of A_qk (weight 1): dq_t += dA_tt k_t and
-        // dk_t += dA_tt q_t, and nothing in dgamma_t, whose row and column terms
-        // of such a pair are equal and opposite (summed into the two sides they
-        // would dominate both, and the fp32 rounding of those sums would survive
-        // the cancellation into dg).
-#pragma unroll
-        for (int m = 0; m < NB; ++m)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int t = BS * m + 4 * g4 + e;
-                dqa[m][e] += sda[t][t] * kx[m][e];
-                dka[m][e] += sda[t][t] * qx[m][e];
-            }
-
-        // PHASE 5
-        // ---------------- phase 5: dG, reverse cumsum, stores ----------------
-        if (g4 == 3) dga[NB - 1][3] += dgcol;        // row C-1
-        // suffix sums over rows t = 16 m + 4 g4 + e of this lane's channel
-        float lsum[NB][4], tot[NB];
-#pragma unroll
-        for (int m = 0; m < NB; ++m) {
-            float run = 0.f;
-#pragma unroll
-            for (int e = 3; e >= 0; --e) { run += dga[m][e]; lsum[m][e] = run; }
-            tot[m] = run;
-        }
-        float after_m = 0.f;   // sum over row tiles > m
-#pragma unroll
-        for (int m = NB - 1; m >= 0; --m) {
-            const float t0v = __shfl(tot[m], r16, 64);
-            const float t1v = __shfl(tot[m], r16 + 16, 64);
-            const float t2v = __shfl(tot[m], r16 + 32, 64);
-            const float t3v = __shfl(tot[m], r16 + 48, 64);
-            const float later = (g4 < 1 ? t1v : 0.f) + (g4 < 2 ? t2v : 0.f) + (g4 < 3 ? t3v : 0.f);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) lsum[m][e] += later + after_m;
-            after_m += t0v + t1v + t2v + t3v;
-        }
-        TI* dq = static_cast<TI*>(a.dq);
-        TI* dk = static_cast<TI*>(a.dk);
-        TG* dg = static_cast<TG*>(a.dg);
-#pragma unroll
-        for (int m = 0; m < NB; ++m)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int t = BS * m + 4 * g4 + e;
-                if (t < valid) {
-                    const size_t o = base + (size_t)t * rs + d;
-                    st1<TI>(dq + o, dqa[m][e]);
-                    st1<TI>(dk + o, dka[m][e]);
-                    st1<TG>(dg + o, lsum[m][e]);
-                }
-            }
-    }
-    if (tid < valid) {
-        float db = 0.f;
-#pragma unroll
-        for (int j = 0; j < NB + NT; ++j) db += sdb[j][tid];
-        st1<TI>(static_cast<TI*>(a.dbeta) + bbase + (size_t)tid * a.H, db);
-    }
-    // PHASE 6
-}
-
 // ----------------------------------------------------------------------------
-// LDS plan of the bf16 local-adjoint kernel (kda_bwd_local3_kernel below;
-// kda_bwd_local_kernel above serves fp32 inputs).
+// LDS plan of the bf16 local-adjoint kernel (kda_bwd_local3_kernel below).
 //
 // Every global operand of the chunk arrives in one batch of 16-byte loads and
 // lives in LDS; LDS regions are reused once their phase is over:
@@ -1499,15 +1136,11 @@ __global__ __launch_bounds__(512) void kda_bwd_local3_kernel(const LocalArgs a) 
 // ----------------------------------------------------------------------------
 template <int D, typename TI, typename TG>
 static hipError_t launch_local_t(const LocalArgs& a, int nchunks, hipStream_t st) {
-    if constexpr (std::is_same<TI, float>::value)
-        hipLaunchKernelGGL((kda_bwd_local_kernel<D, TI, TG, 3>), dim3(nchunks), dim3(256), 0, st, a);
-    else {
-        // prefetch distance: one chunk per CU (one local-adjoint workgroup fills a CU)
-        int dev = 0;
-        LocalArgs b = a;
-        b.pf_ahead = (hipGetDevice(&dev) == hipSuccess) ? device_cu_count(dev) : 0;
-        hipLaunchKernelGGL((kda_bwd_local3_kernel<D, TI, TG, 1>), dim3(nchunks), dim3(512), 0, st, b);
-    }
+    // prefetch distance: one chunk per CU (one local-adjoint workgroup fills a CU)
+    int dev = 0;
+    LocalArgs b = a;
+    b.pf_ahead = (hipGetDevice(&dev) == hipSuccess) ? device_cu_count(dev) : 0;
+    hipLaunchKernelGGL((kda_bwd_local3_kernel<D, TI, TG, 1>), dim3(nchunks), dim3(512), 0, st, b);
     return hipGetLastError();
 }
 
@@ -1521,17 +1154,18 @@ hipError_t launch_local(const LocalArgs& a, int D, int in_bf16, int g_kind, int 
         return hipErrorInvalidValue;
     }
     const int g_bf16 = g_kind == 1;
-#define KDA_LOCAL_CASE(DD)                                                                         \
-    if (D == DD) {                                                                                 \
-        if (in_bf16) return g_bf16 ? launch_local_t<DD, uint16_t, uint16_t>(a, nchunks, st)        \
-                                   : launch_local_t<DD, uint16_t, float>(a, nchunks, st);          \
-        return g_bf16 ? launch_local_t<DD, float, uint16_t>(a, nchunks, st)                        \
-                      : launch_local_t<DD, float, float>(a, nchunks, st);                          \
-    }
+    // fp32 operands at every D: one wave per channel tile with the anchored operands
+    // in registers (two workgroups a CU at D <= 64); with the chunk's fp32 tiles
+    // in LDS, one workgroup a CU, 2 x 1568 x 6 x 64 took 98 us (200 us at the
+    // layer's initial decay) against 59 (84).  bf16 at D <= 64: the tiles fit LDS
+    // and the 8-wave kernel of this file serves them.
+    if (!in_bf16 || D == 128) return launch_local_wide(a, D, in_bf16, g_bf16, nchunks, st);
+#define KDA_LOCAL_CASE(DD)                                                                   \
+    if (D == DD) return g_bf16 ? launch_local_t<DD, uint16_t, uint16_t>(a, nchunks, st)      \
+                               : launch_local_t<DD, uint16_t, float>(a, nchunks, st);
     KDA_LOCAL_CASE(32)
     KDA_LOCAL_CASE(64)
 #undef KDA_LOCAL_CASE
-    if (D == 128) return launch_local_wide(a, D, in_bf16, g_bf16, nchunks, st);
     return hipErrorInvalidValue;
 }
 

@@ -1,12 +1,15 @@
-// kda_bwdw.hip -- the local-adjoint kernel of the KDA backward at D = 128.
+// kda_bwdw.hip -- the local-adjoint kernel of the KDA backward at D = 128 and, for
+// fp32 operands, at D = 32 and 64.
 //
-// kda_bwd_localw_kernel: one 512-thread workgroup per chunk; wave w owns
+// kda_bwd_localw_kernel: one workgroup of D / 16 waves per chunk; wave w owns
 // channel tile w (16 channels) of every per-(t, d) adjoint.  Same chunk
-// algebra as the D = 64 kernels (nope_gdn_mlx.py:2579-2720, the transposed WY
+// algebra as kda_bwd.hip (nope_gdn_mlx.py:2579-2720, the transposed WY
 // solve 1209-1286, the M backward kernels 2080-2295, the in-chunk reverse
-// cumsum 2573-2577), with an LDS plan that fits D = 128:
+// cumsum 2573-2577), with an LDS plan that fits D = 128, and at D <= 64 in fp32
+// two workgroups a CU:
 //   - the chunk's operands that are read as fragments (dO, V', dV', h, dh, W,
-//     U) come straight from global memory (L2): nothing of them is staged;
+//     U) come straight from global memory (L2): nothing of them is staged
+//     (bf16 stages what it can, below);
 //   - A_kk and the inverted diagonal blocks of I + L come from the prep's
 //     workspace, V' from the state recompute's;
 //   - the anchored decay operands of phase 4 (k e^{gamma_t - gamma_r},
@@ -15,7 +18,12 @@
 //   - dR = (I + L)^-T [dW | dU] passes through LDS one half (dW columns, then
 //     dU columns) at a time.
 // LDS: gamma and its factor tables, dP / dA (C x C fp32 each), half of dR, the
-// diagonal inverses, the dbeta partials: about 118 KB.
+// diagonal inverses, the dbeta partials: fp32 118 KB at D = 128, 79 KB at 64.
+// What bounds it: the vector instructions that split fp32 operands into bf16
+// parts (fp32), memory latency with two waves a SIMD (bf16).  Layer's initial
+// decay, fp32: 2 x 1568 x 8 x 128 559 -> 216 us, 8 x 1568 x 12 x 64 1127 ->
+// 457 us, 4 x 1568 x 6 x 32 275 -> 74 us since a strong block's diagonal tiles
+// are the only ones taken pair by pair and no operand tile is kept in LDS.
 #include "kda_internal.h"
 
 namespace kda {
@@ -62,42 +70,23 @@ __device__ __forceinline__ float sum4gw(float x) {
     return x;
 }
 
-// Layout of a wave's private LDS for its diagonal tiles: the raw k and q rows of
-// its 16 channels ([64][DT_K] bf16 each), then over them two planes of sums
-// ([64][DT_P] fp32); strides that put the four blocks' rows on distinct banks
-constexpr int DT_K = 18, DT_P = 17, DT_BYTES = 2 * C * DT_P * 4;
-static_assert(2 * C * DT_K * 2 <= DT_BYTES, "k and q fit under the planes");
+typedef __attribute__((address_space(3))) float lds_f32;
 
 // The four diagonal tiles of a wave's channel tile, pair by pair with the exact
 // weight e^{gamma_t - gamma_s} (s < t): lane (r16, g4) takes block g4 of channel
-// d = its r16's, all 120 pairs of it, the block's rows in registers.  wp: the
-// wave's private area (above); gamma s.g (row stride ldg, own channels only),
-// dP sp and dA sda (row stride lda).  The sums (rows of dk, dq) go to the two
-// planes and those of dgamma over the gamma column itself, which nothing reads
-// afterwards: everything is the wave's own, so no barrier.  Each pair's dgamma
-// term is one value, added to row t and taken from row s.
-// Not inlined: its registers stay out of the kernel's common path.
-typedef __attribute__((address_space(3))) float lds_f32;
-typedef __attribute__((address_space(3))) uint16_t lds_u16;
-typedef __attribute__((address_space(3))) unsigned char lds_u8;
-
+// d = its r16's, all 120 pairs of it, each once, the block's rows (gamma, k, q) in
+// registers.  dP sp and dA sda (row stride lda) from LDS.  ak, aq, ag: the
+// sums of dk, dq and dgamma of those rows.  Each pair's dgamma term is one
+// value, added to row t and taken from row s.
 template <int PREC>
-__device__ __noinline__ void wide_diag_tiles(lds_f32* g, int ldg, lds_u8* wp, const lds_f32* sp, const lds_f32* sda,
-                                             int lda, int g4, int r16) {
-    const lds_u16* sk = reinterpret_cast<const lds_u16*>(wp) + BS * g4 * DT_K + r16;
-    const lds_u16* sq = sk + C * DT_K;
-    g += BS * g4 * ldg;
-    float gt[BS], kt[BS], qt[BS], ak[BS], aq[BS], ag[BS];
-#pragma unroll
-    for (int t = 0; t < BS; ++t) {
-        gt[t] = g[t * ldg];
-        kt[t] = bf2f(sk[t * DT_K]);
-        qt[t] = bf2f(sq[t * DT_K]);
-        ak[t] = aq[t] = ag[t] = 0.f;
-    }
+__device__ __forceinline__ void diag_pairs(const lds_f32* sp, const lds_f32* sda, int lda, int g4, const float (&gt)[BS],
+                                           const float (&kt)[BS], const float (&qt)[BS], float (&ak)[BS],
+                                           float (&aq)[BS], float (&ag)[BS]) {
     const lds_f32* pr = sp + BS * g4 * lda + BS * g4;
     const lds_f32* ar = sda + BS * g4 * lda + BS * g4;
     typedef __attribute__((address_space(3))) const f32x4 lds_f32x4;
+#pragma unroll
+    for (int t = 0; t < BS; ++t) ak[t] = aq[t] = ag[t] = 0.f;
 #pragma unroll
     for (int t = 1; t < BS; ++t) {
 #pragma unroll
@@ -124,21 +113,34 @@ __device__ __noinline__ void wide_diag_tiles(lds_f32* g, int ldg, lds_u8* wp, co
         for (int s = 0; s <= t; ++s) asm volatile("" : "+v"(ak[s]), "+v"(ag[s]));
         asm volatile("" : "+v"(aq[t])::"memory");
     }
-    lds_f32* res = reinterpret_cast<lds_f32*>(wp) + BS * g4 * DT_P + r16;
-    wave_sync();   // every lane has read its k and q: the planes take their place
+}
+
+// x[4 j + e] of lane group g <-> x[4 g + e] of lane group j: from the rows 4 g4 + e
+// of every block (index 4 m + e) to all rows of block g4, and back
+__device__ __forceinline__ void group_transpose(float (&x)[BS]) {
+    auto swap32 = [](float& p, float& q) __attribute__((always_inline)) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(p), __float_as_uint(q), false, false);
+        p = __uint_as_float(r[0]);
+        q = __uint_as_float(r[1]);
+    };
+    auto swap16 = [](float& p, float& q) __attribute__((always_inline)) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(p), __float_as_uint(q), false, false);
+        p = __uint_as_float(r[0]);
+        q = __uint_as_float(r[1]);
+    };
 #pragma unroll
-    for (int t = 0; t < BS; ++t) {
-        res[t * DT_P] = ak[t];
-        res[(C + t) * DT_P] = aq[t];
-        g[t * ldg] = ag[t];
+    for (int e = 0; e < 4; ++e) {
+        swap32(x[e], x[8 + e]);
+        swap32(x[4 + e], x[12 + e]);
+        swap16(x[e], x[4 + e]);
+        swap16(x[8 + e], x[12 + e]);
     }
-    wave_sync();
 }
 
 }  // namespace
 
 template <int D, typename TI, typename TG, int PREC>
-__global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a) {
+__global__ __launch_bounds__(4 * D, D == 32 ? 1 : 2) void kda_bwd_localw_kernel(const LocalArgs a) {
     constexpr int NT = D / BS, NTH = 4 * D, NW = NTH / 64;
     static_assert(NW == NT && NB == 4, "one wave per channel tile, one thread per (channel, row block)");
     __shared__ WideLds<D> s;
@@ -201,8 +203,12 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
     for (int i = 0; i < (AKV + NTH - 1) / NTH; ++i)
         if (AKV % NTH == 0 || tid + NTH * i < AKV)
             akv[i] = reinterpret_cast<const float4*>(a.Akk + cCC)[tid + NTH * i];
-    float4 tiv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (tid < TIV) tiv = reinterpret_cast<const float4*>(a.Tii + (size_t)ch * NB * BS * BS)[tid];
+    float4 tiv[(TIV + NTH - 1) / NTH];
+#pragma unroll
+    for (int i = 0; i < (TIV + NTH - 1) / NTH; ++i) {
+        tiv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (tid + NTH * i < TIV) tiv[i] = reinterpret_cast<const float4*>(a.Tii + (size_t)ch * NB * BS * BS)[tid + NTH * i];
+    }
     const int cd = tid % D, cb = tid / D;
     // rows past T (and channels past dio) are read from the last valid row
     // (channel) -- no branch around a load, so the sixteen loads are in flight
@@ -230,10 +236,12 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
             const int e = 4 * (tid + NTH * i);
             *reinterpret_cast<float4*>(&sp[e / C][e % C]) = akv[i];
         }
-    if (tid < TIV) {
-        const int e = 4 * tid, i = e / (BS * BS), r = (e / BS) % BS, c = e % BS;
-        *reinterpret_cast<float4*>(&tii[i][r][c]) = tiv;
-    }
+#pragma unroll
+    for (int i = 0; i < (TIV + NTH - 1) / NTH; ++i)
+        if (tid + NTH * i < TIV) {
+            const int e = 4 * (tid + NTH * i), b16 = e / (BS * BS), r = (e / BS) % BS, c = e % BS;
+            *reinterpret_cast<float4*>(&tii[b16][r][c]) = tiv[i];
+        }
     for (int idx = tid; idx < (NB + NT) * C; idx += NTH) sdb[idx / C][idx % C] = 0.f;
     if (tid < C) s.beta[tid] = (tid < valid) ? ld1<TI>(beta + bbase + (size_t)tid * a.H) : 0.f;
     if constexpr (STG) {
@@ -288,7 +296,7 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
     // addresses are formed here: a pick among the argument block's fields inside
     // the instantiated phases put the block in scratch memory (224 -> 278 us).
     const char *pfp = nullptr, *pfi = nullptr;
-    if (a.pf_ahead > 0 && ch + a.pf_ahead < (int)gridDim.x) {
+    if (NW == 8 && a.pf_ahead > 0 && ch + a.pf_ahead < (int)gridDim.x) {
         const int pc = ch + a.pf_ahead, pbh = pc / a.nc, pn = pc - pbh * a.nc;
         const int pb = pbh / a.H, ph = pbh - pb * a.H, pvalid = min(C, a.T - pn * C);
         const size_t pbase = ((size_t)pb * a.T + (size_t)pn * C) * rs + (size_t)ph * dio;
@@ -305,7 +313,7 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
     // The phases after the cumsum are instantiated twice, apart from here on: with
     // the copies parting only at phase 4 the strong copy's diagonal tiles spilled
     // the common one's registers.  SSv2 shape (8 x 1568 x 8 x 96): 224 -> 211 us
-    // within the guard, 417 -> 258 us at the layer's initial decay.  (Two
+    // within the guard, 417 -> 253 us at the layer's initial decay.  (Two
     // kernels by a flag from the prep: 201 and 273 us, but fp32 551 -> 622.)
     auto tail = [&](auto mode_c) __attribute__((always_inline)) {
     constexpr int MODE = decltype(mode_c)::value;
@@ -658,41 +666,42 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
             }
         }
         if constexpr (STRONG) {
-            // The diagonal tiles pair by pair, in the wave's private part of the
-            // (then free) staging area; each lane then adds its own rows' sums.
-            unsigned char* const wp = stg + w * DT_BYTES;
-            static_assert(!STRONG || NW * DT_BYTES <= STG_BYTES, "the waves' private areas fit the staging area");
-            TI* const sk = reinterpret_cast<TI*>(wp) + r16;
+            // The diagonal tiles pair by pair, the lane groups' rows exchanged by lane
+            // swaps (through LDS instead, the pairs in a function of their own: 264
+            // against 253 us at the SSv2 shape)
+            float gt[BS], kt[BS], qt[BS], ak[BS], aq[BS], ag[BS];
 #pragma unroll
             for (int m = 0; m < NB; ++m)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int t = BS * m + 4 * g4 + e;
-                    st1<TI>(sk + t * DT_K, kx[m][e]);
-                    st1<TI>(sk + (C + t) * DT_K, qx[m][e]);
+                    kt[4 * m + e] = kx[m][e];
+                    qt[4 * m + e] = qx[m][e];
                 }
-            wave_sync();
-            wide_diag_tiles<PREC>((lds_f32*)&s.g[0][d], D + 4, (lds_u8*)wp, (const lds_f32*)&sp[0][0],
-                                  (const lds_f32*)&sda[0][0], C + 4, g4, r16);
-            const float* res = reinterpret_cast<const float*>(wp) + r16;
+            group_transpose(kt);
+            group_transpose(qt);
+#pragma unroll
+            for (int t = 0; t < BS; ++t) gt[t] = s.g[BS * g4 + t][d];
+            diag_pairs<PREC>((const lds_f32*)&sp[0][0], (const lds_f32*)&sda[0][0], C + 4, g4, gt, kt, qt, ak, aq,
+                             ag);
+            group_transpose(ak);
+            group_transpose(aq);
+            group_transpose(ag);
 #pragma unroll
             for (int m = 0; m < NB; ++m)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const int t = BS * m + 4 * g4 + e;
-                    dka[m][e] += res[t * DT_P];
-                    dqa[m][e] += res[(C + t) * DT_P];
-                    dga[m][e] += s.g[t][d];
+                    dka[m][e] += ak[4 * m + e];
+                    dqa[m][e] += aq[4 * m + e];
+                    dga[m][e] += ag[4 * m + e];
                 }
         }
     };
     // MODE 0: every block within the guard (the condition always holds: the
     // branch keeps phase 4's loads and factors from being scheduled into its
-    // neighbours, 120 -> 30 spill accesses).  MODE 1: bf16 strong blocks, unless
-    // g > 0 or a NaN; everything else (fp32 operands have no room to stage k and
-    // q) takes the pair-by-pair path below
-    if (MODE == 0 ? valid > 0 : (STG && !unsafe)) {
-        anchored(std::integral_constant<bool, MODE == 1 && STG>{});
+    // neighbours, 120 -> 30 spill accesses).  MODE 1: strong blocks; with g > 0 or
+    // a NaN somewhere every pair takes the pair-by-pair path below
+    if (MODE == 0 ? valid > 0 : !unsafe) {
+        anchored(std::integral_constant<bool, MODE == 1>{});
     } else if constexpr (MODE == 1) {
         // pair by pair with the exact weight e^{gamma_t - gamma_s}: raw k and q of
         // the other rows from global memory, gamma from LDS
@@ -791,24 +800,27 @@ __global__ __launch_bounds__(4 * D) void kda_bwd_localw_kernel(const LocalArgs a
 
 // bf16 operands: bf16 MFMA products (PREC 1); fp32: split-bf16 products
 // accurate to fp32 (PREC 3)
+template <int D, typename TI>
+static hipError_t launch_wide_t(const LocalArgs& a, int g_bf16, int nchunks, hipStream_t st) {
+    constexpr int PREC = sizeof(TI) == 2 ? 1 : 3;
+    if (g_bf16)
+        hipLaunchKernelGGL((kda_bwd_localw_kernel<D, TI, uint16_t, PREC>), dim3(nchunks), dim3(4 * D), 0, st, a);
+    else
+        hipLaunchKernelGGL((kda_bwd_localw_kernel<D, TI, float, PREC>), dim3(nchunks), dim3(4 * D), 0, st, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_local_wide(const LocalArgs& args, int D, int in_bf16, int g_bf16, int nchunks, hipStream_t st) {
-    if (D != 128) return hipErrorInvalidValue;
     // prefetch distance: one chunk per CU (one workgroup fills a CU)
     int dev = 0;
     LocalArgs a = args;
     a.pf_ahead = (hipGetDevice(&dev) == hipSuccess) ? device_cu_count(dev) : 0;
-    if (in_bf16) {
-        if (g_bf16)
-            hipLaunchKernelGGL((kda_bwd_localw_kernel<128, uint16_t, uint16_t, 1>), dim3(nchunks), dim3(512), 0, st, a);
-        else
-            hipLaunchKernelGGL((kda_bwd_localw_kernel<128, uint16_t, float, 1>), dim3(nchunks), dim3(512), 0, st, a);
-    } else {
-        if (g_bf16)
-            hipLaunchKernelGGL((kda_bwd_localw_kernel<128, float, uint16_t, 3>), dim3(nchunks), dim3(512), 0, st, a);
-        else
-            hipLaunchKernelGGL((kda_bwd_localw_kernel<128, float, float, 3>), dim3(nchunks), dim3(512), 0, st, a);
-    }
-    return hipGetLastError();
+    if (D == 128) return in_bf16 ? launch_wide_t<128, uint16_t>(a, g_bf16, nchunks, st)
+                                 : launch_wide_t<128, float>(a, g_bf16, nchunks, st);
+    if (in_bf16) return hipErrorInvalidValue;
+    if (D == 64) return launch_wide_t<64, float>(a, g_bf16, nchunks, st);
+    if (D == 32) return launch_wide_t<32, float>(a, g_bf16, nchunks, st);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace kda

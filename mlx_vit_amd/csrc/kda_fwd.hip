@@ -10,7 +10,7 @@
 //                     Replaces nope_gdn_mlx.py:549-597 (preamble, M / M_oq
 //                     kernels 1301-1469, IA build) and lifts the triangular solve
 //                     (1098-1196) out of the sequential chunk loop.
-// The sequential half of the forward, kda_recur_kernel, is in kda_recur.hip.
+// The sequential half of the forward is in kda_recur.hip (bf16) and kda_recur_f32.hip.
 #include "kda_internal.h"
 
 namespace kda {

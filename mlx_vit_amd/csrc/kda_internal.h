@@ -156,7 +156,7 @@ hipError_t launch_dh_seg_maps(const DhArgs& a, hipStream_t st);
 hipError_t launch_states_dh(const RecurArgs& ra, const DhArgs& da, hipStream_t st);
 hipError_t launch_dh_seg(const DhArgs& a, hipStream_t st);
 hipError_t launch_local(const LocalArgs& a, int D, int in_bf16, int g_kind, int nchunks, hipStream_t st);
-// the local adjoints at D = 128 (kda_bwdw.hip): reads A_kk, the diagonal-block
+// the local adjoints at D = 128 and of fp32 operands (kda_bwdw.hip): reads A_kk, the diagonal-block
 // inverses and V' from the workspace
 hipError_t launch_local_wide(const LocalArgs& a, int D, int in_bf16, int g_bf16, int nchunks, hipStream_t st);
 hipError_t launch_solve(const float* M, const float* b, float* y, int BH, int Cm, int N, int upper,

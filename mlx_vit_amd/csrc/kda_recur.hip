@@ -541,7 +541,7 @@ __global__ __launch_bounds__(256) void kda_dh_kernel(const DhArgs a) {
 // The backward's state recompute and reverse carry at bf16 D = 128 in one
 // launch.  They are independent (the reverse carry does not read the states)
 // and one workgroup of either fills a CU's LDS, so workgroups 0 .. 2 BH - 1
-// recompute the states (two per (b, h), as kda_recur_kernel) and the next 2 BH
+// recompute the states (two per (b, h), as on its own) and the next 2 BH
 // run the reverse carry (two per (b, h), as kda_dh_kernel), side by side on
 // 4 BH CUs instead of one kernel after the other.
 __global__ __launch_bounds__(256) void kda_states_dh_kernel(const RecurArgs ra, const DhArgs da) {

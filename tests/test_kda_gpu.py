@@ -293,6 +293,28 @@ def test_mixed_span_blocks_d128(scales):
     _assert_all(_bwd_errors(x, torch.bfloat16), TOL[torch.bfloat16], f"bwd mixed spans D128 {scales}")
 
 
+@pytest.mark.parametrize("T", [65, 191, 256])
+@pytest.mark.parametrize("D,g_dtype", [(32, torch.float32), (32, torch.bfloat16), (64, torch.bfloat16),
+                                       (96, torch.float32), (128, torch.float32)])
+def test_bwd_fp32_mixed_blocks(T, D, g_dtype):
+    """fp32 operands at every head size: one chunk within the span guard, one with
+    some blocks beyond it (their diagonal tiles by lane-group exchange), one with
+    g > 0, the last chunk of one row, one row short, or whole; g bf16 and fp32.
+    TOL: fp32 products accurate to 2^-24 a term over sums of up to 128 terms; a bf16
+    dg (g's type) is off by its own rounding besides, at most 2^-8 an element."""
+    x = _inputs(2, T, 3, D, torch.float32, seed=36 + T + D, with_state=True, grad=True, g_scale=0.2)
+    g = x["g"].float()
+    g[:, :16] *= 60.0
+    g[:, 48:64] *= 100.0
+    if T > 140:
+        g[:, 130:134, 1] = 0.03
+    x["g"] = g.to(g_dtype)
+    errs = _bwd_errors(x, torch.float32)
+    if g_dtype == torch.bfloat16:
+        assert errs.pop("dg") <= 2.0 ** -8
+    _assert_all(errs, TOL[torch.float32], f"bwd fp32 blocks T={T} D={D} g {g_dtype}")
+
+
 @pytest.mark.parametrize("D", [96, 64])
 def test_layer_init_decay(D):
     """The SSv2 layer's decay at initialisation, g = -A_h softplus(N(0, 0.5^2))
