@@ -17,7 +17,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 BUILD_DIR = os.path.join(HERE, "_build")
 LIB_PATH = os.path.join(HERE, "libkda_hip.so")
-SOURCES = ["kda_fwd.hip", "kda_recur.hip", "kda_bwd.hip", "kda_layer.hip", "kda_api.hip", "kda_noalloc.hip", "kda_seg.hip", "kda_bwdw.hip", "kda_pad.hip", "kda_short.hip",
+SOURCES = ["kda_fwd.hip", "kda_prepw.hip", "kda_recur.hip", "kda_bwd.hip", "kda_layer.hip", "kda_api.hip", "kda_noalloc.hip", "kda_seg.hip", "kda_bwdw.hip", "kda_pad.hip", "kda_short.hip",
            "kda_wgrad.hip", "kda_recur_f32.hip"]
 ARCH = os.environ.get("KDA_OFFLOAD_ARCH", "gfx950")
 
@@ -30,9 +30,10 @@ COMMON_FLAGS = [
 ]
 
 
-# Per-source additions.  The prep kernel is scheduled with LLVM's
+# Per-source additions.  The prep kernel of kda_fwd.hip is scheduled with LLVM's
 # iterative-ILP strategy, measured faster there (it is VALU-bound); the other
-# kernels measured slower with it and keep the default.
+# kernels measured slower with it (kda_prepw.hip's 333 -> 377 us) and keep the
+# default.
 SOURCE_FLAGS = {"kda_fwd.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]}
 
 

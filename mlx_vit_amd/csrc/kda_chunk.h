@@ -274,8 +274,9 @@ __device__ __forceinline__ int chunk_factors2(ChunkSmem<D, ST>& s, int flag, int
 // of the tile; entries above the diagonal are not masked.  With ksel >= 0 only
 // the 32 channels of k-step ksel contribute (a partial product, so that two
 // waves can share a tile).
-template <int D, typename ST, int PREC, bool WITH_Q>
-__device__ __forceinline__ void subanchor_tile(const ChunkSmem<D, ST>& s, int i, f32x4& P, f32x4& Q, int ksel = -1) {
+// S: any layout with the members kr, ql (rows of ST) and g.
+template <int D, typename ST, int PREC, bool WITH_Q, typename S>
+__device__ __forceinline__ void subanchor_tile(const S& s, int i, f32x4& P, f32x4& Q, int ksel = -1) {
     const int l = lane_id(), r16 = l & 15, g4 = l >> 4, q = r16 >> 2;
     const int row = BS * i + r16;
     P = zero4();
@@ -336,8 +337,8 @@ __device__ __forceinline__ void subanchor_tile(const ChunkSmem<D, ST>& s, int i,
 
 // gamma_t of row t, channel d, from a (any chunk): a_t plus the totals of the
 // blocks before t's
-template <int D, typename ST>
-__device__ __forceinline__ float chunk_gamma(const ChunkSmem<D, ST>& s, int t, int d) {
+template <typename S>
+__device__ __forceinline__ float chunk_gamma(const S& s, int t, int d) {
     float x = s.g[t][d];
     if (t >= BS) x += s.g[BS - 1][d];
     if (t >= 2 * BS) x += s.g[2 * BS - 1][d];
@@ -358,21 +359,22 @@ __device__ __forceinline__ float chunk_gamma(const ChunkSmem<D, ST>& s, int t, i
 // With fc != nullptr the block's transpose is also written as split (PREC 3)
 // MFMA A fragments, fc[64 w + lane] = fragment of lane (g, r) holding
 // T_ww[4g + e][r], so that other waves load it with one 16-byte read per lane.
+// block_inverse_reg: one such block, its rows at Akk (stride LDA) and its betas; xq
+// receives the lane's inverse[4 p .. 4 p + 3][c].
 template <int LDA>
-__device__ __forceinline__ void diag_inverse_reg(const float* __restrict__ akk, const float* __restrict__ beta,
-                                                 float (*tii)[BS][BS + 4], Frag4* fc = nullptr) {
+__device__ __forceinline__ void block_inverse_reg(const float* akk, const float* beta, float (&xq)[4]) {
     static_assert(BS == 16, "four quarters of four");
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l >> 2, p = l & 3;
-    const float* Ab = akk + (size_t)(BS * w) * LDA + BS * w + 4 * p;
+    const int l = threadIdx.x & 63, c = l >> 2, p = l & 3;
+    const float* Ab = akk + 4 * p;
     float4 R[BS];   // R[t] = Akk[t][4 p .. 4 p + 3] of the block (zero at s >= t in akk)
     float bt[BS];
 #pragma unroll
     for (int t = 1; t < BS; ++t) {
-        bt[t] = beta[BS * w + t];
+        bt[t] = beta[t];
         R[t] = *reinterpret_cast<const float4*>(Ab + t * LDA);
     }
     __builtin_amdgcn_sched_barrier(0);
-    float xq[4] = {0.f, 0.f, 0.f, 0.f};   // x_{4p} .. x_{4p+3}
+    xq[0] = xq[1] = xq[2] = xq[3] = 0.f;   // x_{4p} .. x_{4p+3}
     if (p == 0) xq[0] = (c == 0) ? 1.f : 0.f;
 #pragma unroll
     for (int t = 1; t < BS; ++t) {
@@ -383,6 +385,13 @@ __device__ __forceinline__ void diag_inverse_reg(const float* __restrict__ akk, 
         const float xt = ((t == c) ? 1.f : 0.f) - bt[t] * part;
         if ((t >> 2) == p) xq[t & 3] = xt;
     }
+}
+template <int LDA>
+__device__ __forceinline__ void diag_inverse_reg(const float* __restrict__ akk, const float* __restrict__ beta,
+                                                 float (*tii)[BS][BS + 4], Frag4* fc = nullptr) {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, c = l >> 2, p = l & 3;
+    float xq[4];
+    block_inverse_reg<LDA>(akk + (size_t)(BS * w) * LDA + BS * w, beta + BS * w, xq);
 #pragma unroll
     for (int e = 0; e < 4; ++e) tii[w][4 * p + e][c] = xq[e];
     if (fc) fc[64 * w + 16 * p + c] = frag4_from_f32<3>(xq);

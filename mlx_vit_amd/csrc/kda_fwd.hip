@@ -49,7 +49,7 @@ template <int D, typename ST, typename TG, int PREC, int NTH>
 __global__ __launch_bounds__(NTH) void kda_prep_kernel(const PrepArgs a) {
     using G = PrepGeom<D, ST>;
     constexpr int NW = NTH / 64;   // waves
-    static_assert(NW == 4 || NW == 8 || NW == 16, "four, eight or sixteen waves");
+    static_assert(NW == 4 || NW == 8, "four or eight waves");
     constexpr int LDK = G::LDK, LDA = G::LDA, LDT = G::LDT, NT = D / BS, NCT = 2 * NT;
     constexpr int TPW = (NCT + NW - 1) / NW;
     constexpr int EPV = 16 / (int)sizeof(ST);
@@ -616,10 +616,8 @@ __global__ __launch_bounds__(NTH) void kda_prep_kernel(const PrepArgs a) {
 template <int D, typename ST, typename TG>
 static hipError_t launch_prep_t(const PrepArgs& a, int nchunks, hipStream_t st) {
     constexpr int PREC = std::is_same<ST, float>::value ? 3 : 1;
-    // eight waves per chunk where the registers allow four waves per SIMD;
-    // bf16 at D = 128 (133 KB of LDS: one workgroup per CU, 123 VGPRs) sixteen,
-    // four per SIMD on one chunk: config 3's prep 396 -> 368 us, bit-identical
-    constexpr int NTH = (D >= 128 && std::is_same<ST, uint16_t>::value) ? 1024 : (D >= 64) ? KDA_PREP_NTH : 256;
+    // eight waves per chunk where the registers allow four waves per SIMD
+    constexpr int NTH = (D >= 64) ? KDA_PREP_NTH : 256;
     hipLaunchKernelGGL((kda_prep_kernel<D, ST, TG, PREC, NTH>), dim3(nchunks), dim3(NTH), 0, st, a);
     return hipGetLastError();
 }
@@ -634,6 +632,9 @@ hipError_t launch_prep(const PrepArgs& a, int D, int in_bf16, int g_kind, int nc
         return hipErrorInvalidValue;
     }
     const int g_bf16 = g_kind == 1;
+    // bf16 at D = 128: two workgroups a CU by keeping less in LDS (kda_prepw.hip);
+    // fp32 tiles of that size fill the CU either way
+    if (in_bf16 && D == 128) return launch_prep_wide(a, g_bf16, nchunks, st);
 #define KDA_PREP_CASE(DD)                                                                          \
     if (D == DD) {                                                                                 \
         if (in_bf16) return g_bf16 ? launch_prep_t<DD, uint16_t, uint16_t>(a, nchunks, st)         \
@@ -643,8 +644,9 @@ hipError_t launch_prep(const PrepArgs& a, int D, int in_bf16, int g_kind, int nc
     }
     KDA_PREP_CASE(32)
     KDA_PREP_CASE(64)
-    KDA_PREP_CASE(128)
 #undef KDA_PREP_CASE
+    if (D == 128) return g_bf16 ? launch_prep_t<128, float, uint16_t>(a, nchunks, st)
+                                : launch_prep_t<128, float, float>(a, nchunks, st);
     return hipErrorInvalidValue;
 }
 

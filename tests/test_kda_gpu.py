@@ -315,6 +315,25 @@ def test_bwd_fp32_mixed_blocks(T, D, g_dtype):
     _assert_all(errs, TOL[torch.float32], f"bwd fp32 blocks T={T} D={D} g {g_dtype}")
 
 
+@pytest.mark.parametrize("T", [65, 191, 256])
+@pytest.mark.parametrize("D,g_dtype", [(96, torch.bfloat16), (96, torch.float32), (128, torch.bfloat16),
+                                       (128, torch.float32)])
+def test_bf16_d128_chunk_kinds(T, D, g_dtype):
+    """bf16 above D = 64: a chunk with one block beyond the 16-row span guard and
+    one beyond the 4-row guard too, a chunk within both, one with g > 0 somewhere,
+    the last of one row, one row short, or whole; every output of the training
+    pair.  TOL: bf16 operands and results, 2^-8 each."""
+    x = _inputs(2, T, 3, D, torch.bfloat16, seed=37 + T + D, with_state=True, grad=True, g_scale=0.2)
+    g = x["g"].float()
+    g[:, :16] *= 60.0
+    g[:, 48:64] -= 25.0
+    if T > 140:
+        g[:, 130:134, 1] = 0.03
+    x["g"] = g.to(g_dtype)
+    _assert_all(_fwd_errors(x, torch.bfloat16), TOL[torch.bfloat16], f"fwd chunk kinds T={T} D={D} g {g_dtype}")
+    _assert_all(_bwd_errors(x, torch.bfloat16), TOL[torch.bfloat16], f"bwd chunk kinds T={T} D={D} g {g_dtype}")
+
+
 @pytest.mark.parametrize("D", [96, 64])
 def test_layer_init_decay(D):
     """The SSv2 layer's decay at initialisation, g = -A_h softplus(N(0, 0.5^2))
