@@ -623,30 +623,23 @@ static hipError_t launch_prep_t(const PrepArgs& a, int nchunks, hipStream_t st) 
 }
 
 // g_kind: 0 fp32 g, 1 bf16 g, 2 one fp32 decay per (b, t, h) (bf16 inputs at
-// D <= 64 only)
+// D <= 64 only).  bf16 at D = 64 and 128 goes to kda_prepw.hip, which keeps less of
+// a chunk in LDS (figures there); fp32 tiles leave no room for a second
+// workgroup either way, and a 32-channel chunk fits three times as it is.
 hipError_t launch_prep(const PrepArgs& a, int D, int in_bf16, int g_kind, int nchunks, hipStream_t st) {
-    if (g_kind == 2) {
-        if (!in_bf16) return hipErrorInvalidValue;
-        if (D == 32) return launch_prep_t<32, uint16_t, GHead>(a, nchunks, st);
-        if (D == 64) return launch_prep_t<64, uint16_t, GHead>(a, nchunks, st);
-        return hipErrorInvalidValue;
-    }
-    const int g_bf16 = g_kind == 1;
-    // bf16 at D = 128: two workgroups a CU by keeping less in LDS (kda_prepw.hip);
-    // fp32 tiles of that size fill the CU either way
-    if (in_bf16 && D == 128) return launch_prep_wide(a, g_bf16, nchunks, st);
-#define KDA_PREP_CASE(DD)                                                                          \
-    if (D == DD) {                                                                                 \
-        if (in_bf16) return g_bf16 ? launch_prep_t<DD, uint16_t, uint16_t>(a, nchunks, st)         \
-                                   : launch_prep_t<DD, uint16_t, float>(a, nchunks, st);           \
-        return g_bf16 ? launch_prep_t<DD, float, uint16_t>(a, nchunks, st)                         \
-                      : launch_prep_t<DD, float, float>(a, nchunks, st);                           \
-    }
+    if (in_bf16 && (D == 64 || D == 128)) return launch_prep_wide(a, D, g_kind, nchunks, st);
+    if (in_bf16 && D == 32)
+        return g_kind == 2   ? launch_prep_t<32, uint16_t, GHead>(a, nchunks, st)
+               : g_kind == 1 ? launch_prep_t<32, uint16_t, uint16_t>(a, nchunks, st)
+                             : launch_prep_t<32, uint16_t, float>(a, nchunks, st);
+    if (in_bf16 || g_kind == 2) return hipErrorInvalidValue;
+#define KDA_PREP_CASE(DD)                                                          \
+    if (D == DD) return g_kind == 1 ? launch_prep_t<DD, float, uint16_t>(a, nchunks, st) \
+                                    : launch_prep_t<DD, float, float>(a, nchunks, st);
     KDA_PREP_CASE(32)
     KDA_PREP_CASE(64)
+    KDA_PREP_CASE(128)
 #undef KDA_PREP_CASE
-    if (D == 128) return g_bf16 ? launch_prep_t<128, float, uint16_t>(a, nchunks, st)
-                                : launch_prep_t<128, float, float>(a, nchunks, st);
     return hipErrorInvalidValue;
 }
 

@@ -141,8 +141,8 @@ int device_cu_count(int dev);
 // g_kind: 0 fp32 g [B, T, H, D], 1 bf16 g, 2 one fp32 decay per (b, t, h),
 // g and dg [B, T, H] (GHead; bf16 inputs at D <= 64 only)
 hipError_t launch_prep(const PrepArgs& a, int D, int in_bf16, int g_kind, int nchunks, hipStream_t st);
-// bf16 operands at D = 128 (kda_prepw.hip)
-hipError_t launch_prep_wide(const PrepArgs& a, int g_bf16, int nchunks, hipStream_t st);
+// bf16 operands at D = 64 and 128 (kda_prepw.hip)
+hipError_t launch_prep_wide(const PrepArgs& a, int D, int g_kind, int nchunks, hipStream_t st);
 // bf16; mode 0: O and the final state (and y when a.y is set); 1: the chunk-start
 // states h (D <= 64)
 hipError_t launch_recur(const RecurArgs& a, int D, int mode, hipStream_t st);

@@ -1,10 +1,12 @@
-// kda_prepw.hip -- the forward prep at D = 128, bf16 operands.
+// kda_prepw.hip -- the forward prep of bf16 operands at D = 64 and 128.
 //
 // Same chunk algebra and outputs as kda_prep_kernel (kda_fwd.hip; nope_gdn_mlx.py:
-// 2400-2472, 1319-1334, 1141-1207), in 80 KB of LDS so that two 8-wave workgroups
-// share a CU: one chunk's loads and stores run beside another's products and
-// solve.  With a chunk's every array in LDS (133 KB, one 16-wave workgroup a CU)
-// each barrier left the CU idle.  What is kept out of LDS:
+// 2400-2472, 1319-1334, 1141-1207), in 80 KB of LDS at D = 128 so that two 8-wave
+// workgroups share a CU: one chunk's loads and stores run beside another's
+// products and solve.  With a chunk's every array in LDS (133 KB, one 16-wave
+// workgroup a CU) each barrier left the CU idle.  At D = 64 two share it as
+// before (the registers' limit), with two phases and their LDS passes fewer.
+// What is kept out of LDS:
 //   - the in-block cumsums a of g: a thread loads q, k and g of the same (token,
 //     8 channels), so the operands k e^{a}, q e^{a}, k e^{b} form in registers;
 //     only the block totals pass through LDS.  Chunks with strong blocks lay
@@ -12,35 +14,38 @@
 //   - v: in registers until the products have read K_r, then in its place;
 //   - A_kk: the off-diagonal tiles go from the accumulators to the split
 //     operands of the solve, the diagonal ones to the rows their inverses take.
-// 8192 chunks (32768 x 16 x 128): 411 -> 333 us, 1.14 GB read and written, 2.8 ->
-// 3.4 TB/s against 5.2 for a copy; 8 x 1568 x 8 x 96 at the layer's initial decay
-// 103 -> 81 us.  Left: the vector instructions of the operand conversions, at
-// the 128 registers two workgroups allow.
+// Before -> after: 32768 x 16 x 128 411 -> 333 us (1.14 GB read and written, 2.8 ->
+// 3.4 TB/s against 5.2 for a copy); 8 x 1568 x 8 x 96 at the layer's initial decay
+// 103 -> 81 us; 8 x 1568 x 12 x 64 55 -> 48 us, at that decay 68 -> 62 us.  Left:
+// the vector instructions of the operand conversions, at the 128 registers two
+// workgroups allow (three at D = 64, 80 registers: 80 us).
 #include "kda_internal.h"
 
 namespace kda {
 
 namespace {
 
-constexpr int PW_D = 128, PW_NTH = 512, PW_LDK = PW_D + 8, PW_LDT = C + 8, PW_SPR = 2 * BS + 8, PW_SPB = BS * PW_SPR;
+constexpr int PW_NTH = 512, PW_LDT = C + 8, PW_SPR = 2 * BS + 8, PW_SPB = BS * PW_SPR;
 
+template <int D>
 struct PrepWLds {
-    uint16_t ql[C][PW_LDK];   // raw q (strong chunks), then q e^{a}; U at the end
-    uint16_t kr[C][PW_LDK];   // raw k (strong chunks), then k e^{b}, then v
+    static constexpr int LDK = D + 8;
+    uint16_t ql[C][LDK];   // raw q (strong chunks), then q e^{a}; U at the end
+    uint16_t kr[C][LDK];   // raw k (strong chunks), then k e^{b}, then v
     union {
         struct {
-            uint16_t kl[C][PW_LDK];    // k e^{a}; W at the end
+            uint16_t kl[C][LDK];    // k e^{a}; W at the end
             uint16_t aqk[C][PW_LDT];   // A_qk on its way out
             uint16_t spl[6][PW_SPB];   // split -beta A_kk of the blocks below the diagonal
         };
-        float g[C][PW_D + 4];   // a, strong chunks only, before kl is written
+        float g[C][D + 4];   // a, strong chunks only, before kl is written
     };
-    float fac[14][PW_D];          // factor tables, rows FAC_*
+    float fac[14][D];          // factor tables, rows FAC_*
     float tii[NB][BS][BS + 4];    // block totals of g; A_kk's diagonal tiles; their inverses, then split
     float beta[C];
     int fl[PW_NTH / 64];          // decay flags per wave
 };
-static_assert(sizeof(PrepWLds) <= 80 * 1024, "two workgroups a CU");
+static_assert(sizeof(PrepWLds<128>) <= 80 * 1024, "two workgroups a CU");
 
 // the value of lane 15 of the lane's row of 16
 __device__ __forceinline__ float row16_last(float x) {
@@ -49,13 +54,14 @@ __device__ __forceinline__ float row16_last(float x) {
 
 }  // namespace
 
-template <typename TG>
+template <int D, typename TG>
 __global__ __launch_bounds__(PW_NTH, 4) void kda_prepw_kernel(const PrepArgs a) {
     using ST = uint16_t;
-    constexpr int D = PW_D, NTH = PW_NTH, NW = NTH / 64, NT = D / BS, LDK = PW_LDK, LDT = PW_LDT, PREC = 1;
-    constexpr int SPR = PW_SPR;
-    static_assert(NW == 2 * NB && NT == NW, "two waves a row block; one K and one V column tile a wave");
-    __shared__ __align__(16) PrepWLds s;
+    constexpr int NTH = PW_NTH, NW = NTH / 64, NT = D / BS, LDK = D + 8, LDT = PW_LDT, PREC = 1, SPR = PW_SPR;
+    constexpr bool GH = std::is_same<TG, GHead>::value;   // one fp32 decay per (b, t, h)
+    using TGE = typename std::conditional<GH, float, TG>::type;
+    static_assert(NW == 2 * NB && (2 * NT) % NW == 0, "two waves a row block; whole column tiles of [K | V] a wave");
+    __shared__ __align__(16) PrepWLds<D> s;
 
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, r16 = l & 15, g4 = l >> 4;
     __builtin_assume(w >= 0 && w < NW);
@@ -63,7 +69,7 @@ __global__ __launch_bounds__(PW_NTH, 4) void kda_prepw_kernel(const PrepArgs a) 
     const int b = bh / a.H, h = bh - b * a.H;
     const int t0 = n * C, valid = min(C, a.T - t0);
     // dio: the channels of a q, k, v, g row (a multiple of 8; the rest read as zero)
-    const int dio = (a.dio > 0) ? a.dio : D;
+    const int dio = (D == 128 && a.dio > 0) ? a.dio : D;
     const size_t rs = (size_t)a.H * dio;
     const size_t base = ((size_t)b * a.T + t0) * rs + (size_t)h * dio;
     const size_t bbase = ((size_t)b * a.T + t0) * a.H + h;
@@ -87,21 +93,24 @@ __global__ __launch_bounds__(PW_NTH, 4) void kda_prepw_kernel(const PrepArgs a) 
     // wave w: rows of block w / 2, lane row r16 of it, the 8-channel groups
     // 4 (w % 2) + g4 and 8 more; rows past T and channels past dio are read from the
     // last valid ones and zeroed after
-    constexpr int CP = 2, GE = 16 / (int)sizeof(TG), GV = 8 / GE;
+    constexpr int CP = D / 64, GE = 16 / (int)sizeof(TGE), GV = GH ? 1 : 8 / GE;
     const int blk = w >> 1, row = BS * blk + r16, c0 = 8 * (4 * (w & 1) + g4);
     uint4 qr[CP], kr[CP], gr[CP][GV];
+    float gh = 0.f;
     {
         const size_t ro = base + (size_t)min(row, valid - 1) * rs;
         const ST* qp = static_cast<const ST*>(a.q) + ro;
         const ST* kp = static_cast<const ST*>(a.k) + ro;
-        const TG* gp = static_cast<const TG*>(a.g) + ro;
+        const TGE* gp = static_cast<const TGE*>(a.g) + ro;
+        if constexpr (GH) gh = static_cast<const float*>(a.g)[bbase + (size_t)min(row, valid - 1) * a.H];
 #pragma unroll
         for (int cp = 0; cp < CP; ++cp) {
             const int cc = min(c0 + 64 * cp, dio - 8);
             qr[cp] = *reinterpret_cast<const uint4*>(qp + cc);
             kr[cp] = *reinterpret_cast<const uint4*>(kp + cc);
+            if constexpr (!GH)
 #pragma unroll
-            for (int u = 0; u < GV; ++u) gr[cp][u] = *reinterpret_cast<const uint4*>(gp + cc + GE * u);
+                for (int u = 0; u < GV; ++u) gr[cp][u] = *reinterpret_cast<const uint4*>(gp + cc + GE * u);
         }
     }
     const float braw = ld1<ST>(static_cast<const ST*>(a.beta) + bbase + (size_t)min(tid, valid - 1) * a.H);
@@ -120,8 +129,9 @@ __global__ __launch_bounds__(PW_NTH, 4) void kda_prepw_kernel(const PrepArgs a) 
         if (!ok) qr[cp] = kr[cp] = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const Vec16<TG> xv{gr[cp][e / GE]};
-            const float x = ok ? xv.get(e % GE) : 0.f;
+            float x = gh;
+            if constexpr (!GH) x = Vec16<TGE>{gr[cp][e / GE]}.get(e % GE);
+            x = ok ? x : 0.f;
             if (!(x <= 0.f)) fpos = 1;
             at[cp][e] = row16_scan(x);
             const float prev = __int_as_float(
@@ -446,14 +456,16 @@ __global__ __launch_bounds__(PW_NTH, 4) void kda_prepw_kernel(const PrepArgs a) 
                 Frag4 A[PBT];
                 float sv[PBT];
 #pragma unroll
-                for (int i = 0; i < PBT; ++i) {   // token block i, channel block w
-                    A[i] = ldfrag4<1, ST>(X, LDK, BS * i, BS * w);
-                    sv[i] = o ? (i ? s.fac[FAC_EP + i - 1][BS * w + r16] : 1.f)
-                              : (i < NB - 1 ? s.fac[FAC_EQ + i][BS * w + r16] : 1.f);
+                for (int it = 0; it < PBT; ++it) {   // token block i, channel block j
+                    const int tt = w + NW * it, i = tt / NT, j = tt % NT;
+                    A[it] = ldfrag4<1, ST>(X, LDK, BS * i, BS * j);
+                    sv[it] = o ? (i ? s.fac[FAC_EP + i - 1][BS * j + r16] : 1.f)
+                              : (i < NB - 1 ? s.fac[FAC_EQ + i][BS * j + r16] : 1.f);
                 }
 #pragma unroll
-                for (int i = 0; i < PBT; ++i) {
-                    const short hi = (short)f2bf(sv[i]), lo = (short)f2bf(sv[i] - bf2f((uint16_t)hi));
+                for (int it = 0; it < PBT; ++it) {
+                    const int tt = w + NW * it, i = tt / NT, j = tt % NT;
+                    const short hi = (short)f2bf(sv[it]), lo = (short)f2bf(sv[it] - bf2f((uint16_t)hi));
                     short4v bh4, bl4;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
@@ -462,9 +474,9 @@ __global__ __launch_bounds__(PW_NTH, 4) void kda_prepw_kernel(const PrepArgs a) 
                         bl4[e] = dg ? lo : (short)0;
                     }
                     const f32x4 c =
-                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(cat4(A[i].h, A[i].h), cat4(bh4, bl4), zero4(), 0, 0, 0);
+                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(cat4(A[it].h, A[it].h), cat4(bh4, bl4), zero4(), 0, 0, 0);
                     const float c4[4] = {c[0], c[1], c[2], c[3]};
-                    *reinterpret_cast<uint2*>(out + cCD + (size_t)(BS * w + r16) * C + BS * i + 4 * g4) = pk4(c4);
+                    *reinterpret_cast<uint2*>(out + cCD + (size_t)(BS * j + r16) * C + BS * i + 4 * g4) = pk4(c4);
                 }
             }
         }
@@ -478,33 +490,40 @@ __global__ __launch_bounds__(PW_NTH, 4) void kda_prepw_kernel(const PrepArgs a) 
     else
         middle(std::false_type{});
 
-    // ---------------- block forward substitution: column tile w of K_t and of beta V ----------------
-    const int d = BS * w + r16;
-    f32x4 X[2][NB];
-    Frag4 XB[2][NB - 1];   // X's split B fragments, formed once for the later blocks
+    // ---------------- block forward substitution: the wave's column tiles of [K_t | beta V] ----------------
+    constexpr int TPW = 2 * NT / NW;
+    f32x4 X[TPW][NB];
+    Frag4 XB[TPW][NB - 1];   // X's split B fragments, formed once for the later blocks
+    bool isK[TPW];
+    int d0[TPW];
+#pragma unroll
+    for (int u = 0; u < TPW; ++u) {
+        const int ct = w + NW * u;
+        isK[u] = ct < NT;
+        d0[u] = BS * (isK[u] ? ct : ct - NT);
+    }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-        f32x4 Y[2];
+        f32x4 Y[TPW];
         const float4 b4 = *reinterpret_cast<const float4*>(&s.beta[BS * i + 4 * g4]);
         const float bv[4] = {b4.x, b4.y, b4.z, b4.w};
-        const float fe = i ? s.fac[FAC_EP + i - 1][d] : 1.f;
-        float ck[4], cv[4];
-        ld_col4(&s.kl[0][0], LDK, BS * w, BS * i, ck);
-        ld_col4(&s.kr[0][0], LDK, BS * w, BS * i, cv);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            Y[0][e] = bv[e] * fe * ck[e];
-            Y[1][e] = bv[e] * cv[e];
+        for (int u = 0; u < TPW; ++u) {
+            float cx[4];
+            ld_col4(isK[u] ? &s.kl[0][0] : &s.kr[0][0], LDK, d0[u], BS * i, cx);
+            const float fe = (i && isK[u]) ? s.fac[FAC_EP + (i ? i - 1 : 0)][d0[u] + r16] : 1.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Y[u][e] = bv[e] * fe * cx[e];
         }
 #pragma unroll
         for (int j = 0; j < i; ++j) {
             const Frag4 A = get_split(&s.spl[pair_idx(i, j)][0]);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) Y[u] = mma4f<3>(A, XB[u][j], Y[u]);
+            for (int u = 0; u < TPW; ++u) Y[u] = mma4f<3>(A, XB[u][j], Y[u]);
         }
         const Frag4 Tf = get_split(reinterpret_cast<const uint16_t*>(&s.tii[i][0][0]));
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < TPW; ++u) {
             X[u][i] = mma4f<3>(Tf, accfrag4<3>(Y[u]), zero4());
             if (i < NB - 1) XB[u][i] = accfrag4<3>(X[u][i]);
         }
@@ -513,27 +532,31 @@ __global__ __launch_bounds__(PW_NTH, 4) void kda_prepw_kernel(const PrepArgs a) 
     // W -> kl, U -> ql (both read by now), stored coalesced; WT straight from the
     // accumulators
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
+    for (int u = 0; u < TPW; ++u)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            st1<ST>(&s.kl[BS * i + 4 * g4 + e][d], X[0][i][e]);
-            st1<ST>(&s.ql[BS * i + 4 * g4 + e][d], X[1][i][e]);
+        for (int i = 0; i < NB; ++i) {
+            ST* o = isK[u] ? &s.kl[0][0] : &s.ql[0][0];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) st1<ST>(o + (BS * i + 4 * g4 + e) * LDK + d0[u] + r16, X[u][i][e]);
+            if (isK[u] && oWT) {
+                const float x[4] = {X[u][i][0], X[u][i][1], X[u][i][2], X[u][i][3]};
+                *reinterpret_cast<uint2*>(oWT + cCD + (size_t)(d0[u] + r16) * C + BS * i + 4 * g4) = pk4(x);
+            }
         }
-        if (oWT) {
-            const float x[4] = {X[0][i][0], X[0][i][1], X[0][i][2], X[0][i][3]};
-            *reinterpret_cast<uint2*>(oWT + cCD + (size_t)d * C + BS * i + 4 * g4) = pk4(x);
-        }
-    }
     __syncthreads();
     tile_out<ST, C, D, NTH>(&s.kl[0][0], LDK, oW + cCD, D, C);
     tile_out<ST, C, D, NTH>(&s.ql[0][0], LDK, oU + cCD, D, C);
 }
 
-hipError_t launch_prep_wide(const PrepArgs& a, int g_bf16, int nchunks, hipStream_t st) {
-    if (g_bf16)
-        hipLaunchKernelGGL(kda_prepw_kernel<uint16_t>, dim3(nchunks), dim3(PW_NTH), 0, st, a);
-    else
-        hipLaunchKernelGGL(kda_prepw_kernel<float>, dim3(nchunks), dim3(PW_NTH), 0, st, a);
+hipError_t launch_prep_wide(const PrepArgs& a, int D, int g_kind, int nchunks, hipStream_t st) {
+#define KDA_PREPW_CASE(DD, TG) hipLaunchKernelGGL((kda_prepw_kernel<DD, TG>), dim3(nchunks), dim3(PW_NTH), 0, st, a)
+    if (D == 128 && g_kind == 1) KDA_PREPW_CASE(128, uint16_t);
+    else if (D == 128 && g_kind == 0) KDA_PREPW_CASE(128, float);
+    else if (D == 64 && g_kind == 1) KDA_PREPW_CASE(64, uint16_t);
+    else if (D == 64 && g_kind == 0) KDA_PREPW_CASE(64, float);
+    else if (D == 64 && g_kind == 2) KDA_PREPW_CASE(64, GHead);
+    else return hipErrorInvalidValue;
+#undef KDA_PREPW_CASE
     return hipGetLastError();
 }
 

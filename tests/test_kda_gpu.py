@@ -316,10 +316,10 @@ def test_bwd_fp32_mixed_blocks(T, D, g_dtype):
 
 
 @pytest.mark.parametrize("T", [65, 191, 256])
-@pytest.mark.parametrize("D,g_dtype", [(96, torch.bfloat16), (96, torch.float32), (128, torch.bfloat16),
-                                       (128, torch.float32)])
-def test_bf16_d128_chunk_kinds(T, D, g_dtype):
-    """bf16 above D = 64: a chunk with one block beyond the 16-row span guard and
+@pytest.mark.parametrize("D,g_dtype", [(64, torch.bfloat16), (64, torch.float32), (96, torch.bfloat16),
+                                       (96, torch.float32), (128, torch.bfloat16), (128, torch.float32)])
+def test_bf16_chunk_kinds(T, D, g_dtype):
+    """bf16 from D = 64 on: a chunk with one block beyond the 16-row span guard and
     one beyond the 4-row guard too, a chunk within both, one with g > 0 somewhere,
     the last of one row, one row short, or whole; every output of the training
     pair.  TOL: bf16 operands and results, 2^-8 each."""
