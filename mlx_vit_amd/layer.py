@@ -6,7 +6,9 @@ and maps the result back to ``hidden``:
 
 * projections ``q_proj/k_proj/v_proj``, the low-rank decay ``f_proj_2(f_proj_1(x))``,
   the write gate ``b_proj`` and the low-rank output gate ``g_proj_2(g_proj_1(x))``
-  stay GEMMs (hipBLASLt through torch); q, k and v share one GEMM;
+  stay GEMMs (hipBLASLt through torch); q, k and v share one GEMM.  In bf16
+  (``layer_fused.py``) the layer is one autograd node: its weights stacked by
+  one pack kernel, its weight gradients formed by one launch;
 * the element-wise producer -- short causal conv + SiLU + L2 norm + scale,
   ``g = -exp(A_log) softplus(f + dt_bias)``, ``beta = sigmoid(b)``
   (nope_gdn_mlx.py:796-821) -- is one HIP kernel, ``kda_layer_producer_fwd``,
