@@ -237,7 +237,7 @@ def load_traffic(kernel_name):
 PROFILE_ROLES = {
     # rocprof kernel symbol fragment -> profile names in dispatch order within a
     # fwd+bwd step (the training pair: one prep launch, in its training mode)
-    "kda_prep_kernel": ["kda_prep_kernel(train)"],
+    "kda_prep": ["kda_prep_kernel(train)"],
     "kda_recur": ["kda_recur_kernel(fwd)", "kda_recur_kernel(states)"],
     "kda_dh": ["kda_dh_kernel"],
     "kda_bwd_local": ["kda_bwd_local_kernel"],
