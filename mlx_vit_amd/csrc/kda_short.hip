@@ -36,8 +36,9 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
 }
 
 constexpr float LOG2E = 1.44269504088896340736f;
-// A token's decay below this is taken as this: e^-110 is zero in fp32, so no
-// weight changes, and the cumsums of the tokens after it keep their precision.
+// A token's g below this, less the sum of its channel's positive g, is taken as
+// that floor: a weight across the token is then at most e^-110, zero in fp32,
+// with either value, and the cumsums of the tokens after it keep their precision.
 constexpr float G_MIN = -110.f;
 
 // The wave's TT x D tile of a [B, T, H, D] tensor as 16-byte vectors, rows past
@@ -267,10 +268,15 @@ __device__ __forceinline__ void cumsum_g(const GT* __restrict__ g, size_t grow, 
         const float* gp = reinterpret_cast<const float*>(g);
         if (lane_id() < T) gh = gp[(grow + lane_id()) * H + h];
     }
+    float floor = G_MIN;
 #pragma unroll
     for (int t = 0; t < TT; ++t) {
-        const float gt = std::is_same<GT, GHead>::value ? uniform(gh, t) : lds[t * (D + 4) + ch];
-        c += gt < G_MIN ? G_MIN : gt;   // keeps a NaN
+        a[t] = std::is_same<GT, GHead>::value ? uniform(gh, t) : lds[t * (D + 4) + ch];
+        floor -= fmaxf(a[t], 0.f);
+    }
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+        c += a[t] < floor ? floor : a[t];   // keeps a NaN
         a[t] = c * LOG2E;
     }
 }

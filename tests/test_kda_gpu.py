@@ -944,3 +944,35 @@ def test_short_sequences(T, D, dtype, g_kind, decay):
             else:
                 errs[n] = R.rel_l2(a.cpu(), refb[n])
         _assert_all(errs, tol, f"short T={T} D={D} {dtype} g={g_kind} {decay} s0={s0 is not None} dsf={ds is not None}")
+
+
+@pytest.mark.parametrize("dtype,g_kind", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
+                                          (torch.bfloat16, "head")])
+@pytest.mark.parametrize("T,D", [(7, 64), (16, 64), (8, 32), (9, 32)])
+def test_short_sequences_growth_after_strong_decay(T, D, dtype, g_kind):
+    """A decay beyond fp32's range (g = -150) that later positive g partly undo (+50,
+    +30): the tokens before it and the states reach the ones after it with weight
+    e^-70, not zero.  The tokens from the strong one on write nothing (beta = 0) and
+    only the last ones have a cotangent, so the outputs compared consist of such
+    weights alone.  Exponents of up to 216 in log2 units, four fp32 roundings of
+    2^-17 each: 1e-4; bf16 outputs by their own rounding besides, 2^-8."""
+    kda = _kda()
+    B, H = (87, 3) if T > 8 and D == 64 and dtype == torch.bfloat16 else (2, 3)
+    x = R.make_inputs(B, T, H, D, dtype=dtype, seed=T + D, with_state=True, with_grad=True)
+    x["g"] = torch.full((B, T, H, D), -0.125)
+    x["g"][:, 2], x["g"][:, 4], x["g"][:, 5] = -150.0, 50.0, 30.0
+    x["beta"][:, 2:] = 0
+    x["do"][:, :5] = 0
+    ga = x["g"][..., 0].contiguous() if g_kind == "head" else x["g"].to(g_kind)
+    dsf = torch.randn(B, H, D, D, generator=torch.Generator().manual_seed(T))
+    args = [t.to(DEV) for t in (x["q"], x["k"], x["v"], ga, x["beta"], x["s0"])]
+    o, sf, ws = kda.kda_forward_train(*args)
+    got = kda.kda_backward_train(*args, x["do"].to(DEV), dsf.to(DEV), ws)
+    torch.cuda.synchronize()
+    ref = cref.forward(x["q"], x["k"], x["v"], x["g"], x["beta"], x["s0"])
+    refb = cref.backward(x["q"], x["k"], x["v"], x["g"], x["beta"], x["s0"], x["do"], dsf)
+    if g_kind == "head":
+        refb["dg"] = refb["dg"].sum(-1)
+    errs = {"o": R.rel_l2(o[:, 5:].cpu(), ref["o"][:, 5:]), "s_final": R.rel_l2(sf.cpu(), ref["s_final"]),
+            "dv": R.rel_l2(got[2][:, :2].cpu(), refb["dv"][:, :2]), "ds0": R.rel_l2(got[5].cpu(), refb["ds0"])}
+    _assert_all(errs, 1e-4 if dtype == torch.float32 else 2.0 ** -8, f"short growth T={T} D={D} {dtype} g={g_kind}")
