@@ -41,7 +41,8 @@ def fused_params(layer, x: torch.Tensor, state: Optional[torch.Tensor]) -> Optio
     from .layer import GatedDeltaLayer, RMSNormGated, ShortCausalConv1d
     if x.dtype != torch.bfloat16 or x.device.type != "cuda" or x.numel() == 0 or type(x) not in _PLAIN_TENSORS:
         return None
-    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling():
+    # a trace records the launches of an autograd node, none of those made outside one
+    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing():
         return None
     if (_nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks
             or _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks):

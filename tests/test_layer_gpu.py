@@ -516,3 +516,31 @@ def test_log_decay(n, dtype):
     fin = torch.isfinite(dr.float())
     assert torch.equal(fin, torch.isfinite(da.float()))
     assert torch.allclose(da.float()[fin], dr.float()[fin], rtol=2.0 ** (-8 if dtype == torch.bfloat16 else -22), atol=0.0)
+
+
+def _bf16_layer(H, D, seed=7):
+    from mlx_vit_amd import GatedDeltaLayer
+    from mlx_vit_amd.model import to_bf16
+    torch.manual_seed(seed)
+    return to_bf16(GatedDeltaLayer(H * D, H, D)).to(DEV)
+
+
+def _bf16_randn(seed, *shape):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16).to(DEV)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.filterwarnings("ignore")
+def test_layer_jit_trace(grad):
+    """A traced bf16 layer computes what the layer does, on other inputs than
+    those it was traced with (the same kernels: the same bits)."""
+    layer = _bf16_layer(3, 64).requires_grad_(grad)
+    x, y = _bf16_randn(1, 2, 100, 192), _bf16_randn(2, 2, 100, 192)
+    with torch.set_grad_enabled(grad):
+        traced = torch.jit.trace(layer, (x,), check_trace=False)
+        got = traced(y)
+        handle = layer.b_proj.register_forward_hook(lambda *a: None)   # module by module, as traced
+        ref = layer(y)
+        handle.remove()
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
