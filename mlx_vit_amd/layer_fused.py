@@ -19,6 +19,7 @@ from typing import List, Optional, Tuple
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 from torch.nn.modules import module as _nn_module
 
 from . import _lib
@@ -43,6 +44,9 @@ def fused_params(layer, x: torch.Tensor, state: Optional[torch.Tensor]) -> Optio
         return None
     # a trace records the launches of an autograd node, none of those made outside one
     if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return None
+    # forward-mode tangents: the autograd nodes refuse them, the kernels would drop them
+    if forward_ad._current_level >= 0:
         return None
     if (_nn_module._global_forward_hooks or _nn_module._global_forward_pre_hooks
             or _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks):

@@ -544,3 +544,20 @@ def test_layer_jit_trace(grad):
         handle.remove()
     for a, b in zip(got, ref):
         assert torch.equal(a, b)
+
+
+def test_layer_refuses_forward_mode():
+    """The kernels have no forward-mode derivative: a tangent on x, or on a weight,
+    is refused, with or without gradients, and never dropped."""
+    from torch.autograd import forward_ad
+    layer = _bf16_layer(3, 64)
+    x = _bf16_randn(1, 2, 20, 192)
+    for trained in (True, False):
+        layer.requires_grad_(trained)
+        with forward_ad.dual_level(), pytest.raises(NotImplementedError):
+            layer(forward_ad.make_dual(x, torch.ones_like(x)))
+        with forward_ad.dual_level(), pytest.raises(NotImplementedError):
+            w = layer.q_proj.weight.detach()
+            dual = forward_ad.make_dual(w, torch.ones_like(w))
+            torch.func.functional_call(layer, {"q_proj.weight": dual}, (x,))
+        layer(x)
