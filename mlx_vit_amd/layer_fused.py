@@ -23,7 +23,7 @@ from torch.autograd import forward_ad
 from torch.nn.modules import module as _nn_module
 
 from . import _lib
-from .kda import _DTYPE_CODE, _stream, kda_backward_train, kda_forward, kda_forward_train
+from .kda import _DTYPE_CODE, _stream, kda_backward, kda_backward_train, kda_forward, kda_forward_train
 
 _PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
 
@@ -181,9 +181,13 @@ class FusedLayerFunction(torch.autograd.Function):
         conv_w, conv_b, nw, dt_bias, A_log = _views(fp, HD, D)
         dy = torch.mm(dout2, wo).view(B, L, HD)
         do, dz, dnw = gated_rmsnorm_backward(o, z, nw, eps, dy)
-        dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws, chunk,
-                                                        _need_ds0=ctx.needs_input_grad[1])
-        ctx.ws = None
+        need_ds0 = ctx.needs_input_grad[1]
+        if ctx.ws is not None:
+            dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws, chunk,
+                                                            _need_ds0=need_ds0)
+            ctx.ws = None
+        else:   # another backward of a retained graph
+            dq, dk, dv, dg, dbeta, ds0 = kda_backward(q, k, v, g, beta, s0, do, ds_final, chunk, _need_ds0=need_ds0)
         dP = torch.empty((M, NP), dtype=x2.dtype, device=dev)
         P3, dP3 = P.view(B, L, NP), dP.view(B, L, NP)
         _, dxf, _, dcw, dcb, ddt, dA = producer_backward(

@@ -561,3 +561,27 @@ def test_layer_refuses_forward_mode():
             dual = forward_ad.make_dual(w, torch.ones_like(w))
             torch.func.functional_call(layer, {"q_proj.weight": dual}, (x,))
         layer(x)
+
+
+@pytest.mark.parametrize("H,D,L", [(3, 64, 100), (2, 64, 8), (8, 96, 70)])
+def test_layer_second_backward(H, D, L):
+    """Two backwards over one retained graph: the first uses the training forward's
+    workspace, the second forms the factors again, the same bits; and the output's
+    and the state's gradients taken apart add up to the joint ones."""
+    layer = _bf16_layer(H, D)
+    x = _bf16_randn(1, 2, L, H * D).requires_grad_()
+    s0 = (0.1 * _bf16_randn(2, 2, H, D, D).float()).requires_grad_()
+    dout, ds = _bf16_randn(3, 2, L, H * D), _bf16_randn(4, 2, H, D, D).float()
+    leaves = [x, s0, *layer.parameters()]
+    out, s = layer(x, s0)
+
+    def grads(outs, cots):
+        return torch.autograd.grad(outs, leaves, cots, retain_graph=True, allow_unused=True)
+
+    first, second = grads([out, s], [dout, ds]), grads([out, s], [dout, ds])
+    parts = list(zip(grads([out], [dout]), grads([s], [ds])))
+    torch.cuda.synchronize()
+    for a, b in zip(first, second):
+        assert torch.equal(a, b)
+    _check({str(i): _rel(a.float() + (0 if b is None else b.float()), t)
+            for i, ((a, b), t) in enumerate(zip(parts, first))}, TOL[torch.bfloat16], f"second backward {H} {D} {L}")
