@@ -226,17 +226,30 @@ def _i64(rows) -> ctypes.Array:
     return (ctypes.c_int64 * len(flat))(*flat)
 
 
+def _dma_rows(t: torch.Tensor) -> torch.Tensor:
+    """t (rows, n) bf16 as ``kda_weight_grad`` reads it, 16 bytes at a time: a 16-byte
+    aligned base and row stride, rows that hold n rounded up to 8; copied when not."""
+    rows, n = t.shape
+    n8 = -(-n // 8) * 8
+    if t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(0) >= n8:
+        return t
+    out = torch.empty((rows, n8), dtype=t.dtype, device=t.device)[:, :n]
+    return out.copy_(t)
+
+
 def weight_grads(problems, rows: int):
     """Weight gradients of linear maps over the same ``rows`` rows, in one
     launch: for each (dy, x, bias) with dy (rows, n) and x (rows, k) bf16, rows
     at even strides, dw = dy^T x (n, k) and, with ``bias``, db = sum of dy's rows
     (n,).  Returns [(dw, db or None), ...]."""
-    out, fields = [], []
+    out, fields, keep = [], [], []   # keep: copies live until the launch
     dev = problems[0][0].device
     for dy, x, bias in problems:
         for name, t in (("dy", dy), ("x", x)):
             if t.dim() != 2 or t.shape[0] != rows or t.dtype != torch.bfloat16 or t.stride(1) != 1 or t.device != dev:
                 raise ValueError(f"{name} must be a ({rows}, n) bfloat16 matrix with unit column stride on {dev}")
+        dy, x = _dma_rows(dy), _dma_rows(x)
+        keep.append((dy, x))
         n, k = dy.shape[1], x.shape[1]
         dw = torch.empty((n, k), dtype=torch.bfloat16, device=dev)
         db = torch.empty((n,), dtype=torch.bfloat16, device=dev) if bias else None

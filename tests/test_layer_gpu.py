@@ -585,3 +585,37 @@ def test_layer_second_backward(H, D, L):
         assert torch.equal(a, b)
     _check({str(i): _rel(a.float() + (0 if b is None else b.float()), t)
             for i, ((a, b), t) in enumerate(zip(parts, first))}, TOL[torch.bfloat16], f"second backward {H} {D} {L}")
+
+
+@pytest.mark.parametrize("offset", [1, 4])
+def test_layer_unaligned_inputs(offset):
+    """x and the output's cotangent at a storage offset that is no multiple of 16
+    bytes: the same bits as from aligned copies, gradients included."""
+    layer = _bf16_layer(3, 64)
+
+    def shifted(t):
+        return torch.empty(t.numel() + offset, dtype=t.dtype, device=DEV)[offset:].view_as(t).copy_(t)
+
+    def run(x, dout):
+        x = x.requires_grad_()
+        out, s = layer(x)
+        return [out, s, *torch.autograd.grad(out, [x, *layer.parameters()], dout)]
+
+    x, dout = _bf16_randn(1, 2, 50, 192), _bf16_randn(2, 2, 50, 192)
+    ref, got = run(x, dout), run(shifted(x.detach()), shifted(dout))
+    assert shifted(dout).data_ptr() % 16 != 0 and shifted(dout).is_contiguous()
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n,k,ld,offset", [(12, 8, 13, 0), (8, 16, 24, 3), (20, 24, 24, 8)])
+def test_weight_grads_any_rows(n, k, ld, offset):
+    """Rows that the kernel cannot read 16 bytes at a time -- odd strides, bases and
+    widths -- are copied: the same bits as from aligned operands."""
+    from mlx_vit_amd.layer import weight_grads
+    rows, wide = 40, max(ld, n) + offset
+    dy = _bf16_randn(n, rows, wide)[:, offset:offset + n]
+    x = _bf16_randn(k, rows, k + ld)[:, 1:1 + k]
+    ref = torch.empty(rows, -(-n // 8) * 8, dtype=torch.bfloat16, device=DEV)[:, :n].copy_(dy)
+    (dw, db), (rw, rb) = weight_grads([(dy, x, True)], rows) + weight_grads([(ref, x.contiguous(), True)], rows)
+    assert torch.equal(dw, rw) and torch.equal(db, rb)
