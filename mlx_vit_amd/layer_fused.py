@@ -19,6 +19,7 @@ from typing import List, Optional, Tuple
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _nn_module
 
@@ -139,7 +140,8 @@ def _forward(x, state, spec, params, train: bool):
     else:
         o, s_final = kda_forward(q, k, v, g, beta, state, chunk)
     y = gated_rmsnorm_forward(o, z, nw, eps)
-    out = torch.mm(y.view(M, HD), wo.t()).view(B, L, hidden)
+    # no view of the product: a node's output that is one refuses in-place operations
+    out = F.linear(y, wo)
     return out, s_final, (x2, P, xf, z, q, k, v, g, beta, state, o, y, wcat, fp, wf2, wg2, wo), ws
 
 

@@ -619,3 +619,21 @@ def test_weight_grads_any_rows(n, k, ld, offset):
     ref = torch.empty(rows, -(-n // 8) * 8, dtype=torch.bfloat16, device=DEV)[:, :n].copy_(dy)
     (dw, db), (rw, rb) = weight_grads([(dy, x, True)], rows) + weight_grads([(ref, x.contiguous(), True)], rows)
     assert torch.equal(dw, rw) and torch.equal(db, rb)
+
+
+def test_layer_output_in_place():
+    """The layer's outputs take in-place operations: under autograd, and a result
+    formed without gradients that later enters a graph."""
+    layer = _bf16_layer(3, 64)
+    x, dout = _bf16_randn(1, 2, 20, 192), _bf16_randn(2, 2, 20, 192)
+    out, s = layer(x)
+    ref = torch.autograd.grad([2 * out, s], list(layer.parameters()), [dout, torch.ones_like(s)])
+    out, s = layer(x)
+    with torch.no_grad():
+        plain, _ = layer(x)
+    out *= 2
+    s += 1
+    for a, b in zip(torch.autograd.grad([out, s], list(layer.parameters()), [dout, torch.ones_like(s)]), ref):
+        assert torch.equal(a, b)
+    plain += torch.ones(1, dtype=plain.dtype, device=DEV, requires_grad=True)
+    assert plain.requires_grad and torch.equal(plain, 1 + out / 2)
