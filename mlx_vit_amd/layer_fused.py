@@ -177,12 +177,14 @@ class FusedLayerFunction(torch.autograd.Function):
         N = 3 * HD + rank + D + H
         f1, g1 = slice(3 * HD, 3 * HD + rank), slice(3 * HD + rank, 3 * HD + rank + D)
         dev = x2.device
-        if dout is None:
-            dout = torch.zeros((B, L, hidden), dtype=x2.dtype, device=dev)
-        dout2 = dout.to(x2.dtype).contiguous().view(M, hidden)
         conv_w, conv_b, nw, dt_bias, A_log = _views(fp, HD, D)
-        dy = torch.mm(dout2, wo).view(B, L, HD)
-        do, dz, dnw = gated_rmsnorm_backward(o, z, nw, eps, dy)
+        used = dout is not None   # else: only the new state was, and the maps behind the output get no gradient
+        if used:
+            dout2 = dout.to(x2.dtype).contiguous().view(M, hidden)
+            dy = torch.mm(dout2, wo).view(B, L, HD)
+            do, dz, dnw = gated_rmsnorm_backward(o, z, nw, eps, dy)
+        else:
+            do = torch.zeros_like(o)
         need_ds0 = ctx.needs_input_grad[1]
         if ctx.ws is not None:
             dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws, chunk,
@@ -195,21 +197,32 @@ class FusedLayerFunction(torch.autograd.Function):
         _, dxf, _, dcw, dcb, ddt, dA = producer_backward(
             P3[..., :3 * HD], xf, P3[..., N - H:N], conv_w, conv_b, dt_bias, A_log, dq, dk, dv, dg, dbeta, H, D, scale,
             mult, _dqkv=dP3[..., :3 * HD], _dxb=dP3[..., N - H:N])
-        dxf2, dz2 = dxf.view(M, HD), dz.view(M, HD)
+        dxf2 = dxf.view(M, HD)
         torch.mm(dxf2, wf2, out=dP[:, f1])
-        torch.mm(dz2, wg2, out=dP[:, g1])
+        if used:
+            dz2 = dz.view(M, HD)
+            torch.mm(dz2, wg2, out=dP[:, g1])
+        else:
+            dP[:, g1].zero_()
         need = ctx.needs_input_grad
         dx = torch.mm(dP[:, :N], wcat[:N]).view(B, L, hidden) if need[0] else None
         grads: List[Optional[torch.Tensor]] = [None] * 19
         if any(need[3:13]):
-            (dwcat, _), (dwo, _), (dwf2, _), (dwg2, dbg2) = weight_grads(
-                [(dP[:, :N], x2, False), (dout2, y.view(M, HD), False), (dxf2, P[:, f1], False),
-                 (dz2, P[:, g1], True)], M)
-            grads[:10] = [*dwcat.split([HD, HD, HD, rank, D, H]), dwf2, dwg2, dwo, dbg2]
+            problems = [(dP[:, :N], x2, False), (dxf2, P[:, f1], False)]
+            if used:
+                problems += [(dz2, P[:, g1], True), (dout2, y.view(M, HD), False)]
+            dw = weight_grads(problems, M)
+            grads[:7] = [*dw[0][0].split([HD, HD, HD, rank, D, H]), dw[1][0]]
+            if used:
+                grads[7:10] = [dw[2][0], dw[3][0], dw[2][1]]
+            else:
+                grads[4] = None
         if any(need[13:]):
-            sources = [*dcw, *dcb, dnw, ddt, dA]
+            sources = [*dcw, *dcb, dnw if used else None, ddt, dA]
             jobs = []
             for i, (t, (dt, shape)) in enumerate(zip(sources, ctx.small)):
+                if t is None:
+                    continue
                 if dt == torch.float32:
                     grads[10 + i] = t.view(shape)
                 else:
