@@ -27,6 +27,10 @@ from . import _lib
 from .kda import _DTYPE_CODE, _stream, kda_backward, kda_backward_train, kda_forward, kda_forward_train
 
 _PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
+# positions in ``fused_params``' order: those whose gradient comes through the
+# recurrence (all but g_proj_1, g_proj_2, o_proj, the gate's bias and the norm
+# weight)
+_BEFORE_RECURRENCE = (0, 1, 2, 3, 5, 6, 10, 11, 12, 13, 14, 15, 17, 18)
 
 
 def _plain_module(m: nn.Module, cls: type) -> bool:
@@ -44,7 +48,7 @@ def fused_params(layer, x: torch.Tensor, state: Optional[torch.Tensor]) -> Optio
     if x.dtype != torch.bfloat16 or x.device.type != "cuda" or x.numel() == 0 or type(x) not in _PLAIN_TENSORS:
         return None
     # a trace records the launches of an autograd node, none of those made outside one
-    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing():
+    if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch._C._is_tracing():
         return None
     # forward-mode tangents: the autograd nodes refuse them, the kernels would drop them
     if forward_ad._current_level >= 0:
@@ -155,11 +159,24 @@ def fused_layer(x, state, spec, params):
 
 
 class FusedLayerFunction(torch.autograd.Function):
-    """``fused_layer`` with a gradient for every input."""
+    """``fused_layer`` with a gradient for every input.  A part of the backward runs
+    only where a gradient needs it (frozen parameters, as autograd would skip
+    its modules); with nothing before the output norm trained the forward keeps
+    no factors, and the new state does not require grad."""
 
     @staticmethod
     def forward(ctx, x, state, spec, *params):
-        out, s_final, saved, ctx.ws = _forward(x, state, spec, params, True)
+        need = ctx.needs_input_grad
+        # what reaches the recurrence: x, every map and gate of its operands, the state
+        ctx.need_prod = need[0] or any(need[3 + i] for i in _BEFORE_RECURRENCE)
+        ctx.need_rec = ctx.need_prod or need[1]
+        out, s_final, saved, ctx.ws = _forward(x, state, spec, params, ctx.need_rec)
+        ctx.need_norm = ctx.need_rec or need[19] or any(need[3 + i] for i in (4, 7, 9))   # or the gate's maps
+        if not ctx.need_rec:
+            ctx.mark_non_differentiable(s_final)
+            x2, P, xf, z, q, k, v, g, beta, s0, o, *rest = saved
+            saved = (x2 if need[7] else None, P if need[10] or need[12] else None, None, z if ctx.need_norm else None,
+                     None, None, None, None, None, None, o if ctx.need_norm else None, *rest)
         ctx.save_for_backward(*saved)
         ctx.spec, ctx.shape = spec, (*x.shape, params[3].shape[0])
         ctx.small = [(p.dtype, p.shape) for p in params[10:]]
@@ -176,58 +193,87 @@ class FusedLayerFunction(torch.autograd.Function):
         M, HD, NP = B * L, H * D, wcat.shape[0]
         N = 3 * HD + rank + D + H
         f1, g1 = slice(3 * HD, 3 * HD + rank), slice(3 * HD + rank, 3 * HD + rank + D)
-        dev = x2.device
+        dev, dt = wo.device, wo.dtype
+        need_x, need_ds0, need = ctx.needs_input_grad[0], ctx.needs_input_grad[1], ctx.needs_input_grad[3:]
         conv_w, conv_b, nw, dt_bias, A_log = _views(fp, HD, D)
+        grads: List[Optional[torch.Tensor]] = [None] * 19
+        small: List[Optional[torch.Tensor]] = [None] * 9   # the gradients of params[10:], fp32
         used = dout is not None   # else: only the new state was, and the maps behind the output get no gradient
         if used:
-            dout2 = dout.to(x2.dtype).contiguous().view(M, hidden)
-            dy = torch.mm(dout2, wo).view(B, L, HD)
-            do, dz, dnw = gated_rmsnorm_backward(o, z, nw, eps, dy)
-        else:
+            dout2 = dout.to(dt).contiguous().view(M, hidden)
+            if ctx.need_norm:
+                dy = torch.mm(dout2, wo).view(B, L, HD)
+                do, dz, small[6] = gated_rmsnorm_backward(o, z, nw, eps, dy)
+                dz2 = dz.view(M, HD)
+        elif ctx.need_rec:
             do = torch.zeros_like(o)
-        need_ds0 = ctx.needs_input_grad[1]
-        if ctx.ws is not None:
-            dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws, chunk,
-                                                            _need_ds0=need_ds0)
-            ctx.ws = None
-        else:   # another backward of a retained graph
-            dq, dk, dv, dg, dbeta, ds0 = kda_backward(q, k, v, g, beta, s0, do, ds_final, chunk, _need_ds0=need_ds0)
-        dP = torch.empty((M, NP), dtype=x2.dtype, device=dev)
-        P3, dP3 = P.view(B, L, NP), dP.view(B, L, NP)
-        _, dxf, _, dcw, dcb, ddt, dA = producer_backward(
-            P3[..., :3 * HD], xf, P3[..., N - H:N], conv_w, conv_b, dt_bias, A_log, dq, dk, dv, dg, dbeta, H, D, scale,
-            mult, _dqkv=dP3[..., :3 * HD], _dxb=dP3[..., N - H:N])
-        dxf2 = dxf.view(M, HD)
-        torch.mm(dxf2, wf2, out=dP[:, f1])
-        if used:
-            dz2 = dz.view(M, HD)
-            torch.mm(dz2, wg2, out=dP[:, g1])
-        else:
-            dP[:, g1].zero_()
-        need = ctx.needs_input_grad
-        dx = torch.mm(dP[:, :N], wcat[:N]).view(B, L, hidden) if need[0] else None
-        grads: List[Optional[torch.Tensor]] = [None] * 19
-        if any(need[3:13]):
-            problems = [(dP[:, :N], x2, False), (dxf2, P[:, f1], False)]
+        dx = ds0 = None
+        if ctx.need_rec:
+            if ctx.ws is not None:
+                dq, dk, dv, dg, dbeta, ds0 = kda_backward_train(q, k, v, g, beta, s0, do, ds_final, ctx.ws, chunk,
+                                                                _need_ds0=need_ds0)
+                ctx.ws = None
+            else:   # another backward of a retained graph
+                dq, dk, dv, dg, dbeta, ds0 = kda_backward(q, k, v, g, beta, s0, do, ds_final, chunk,
+                                                          _need_ds0=need_ds0)
+        if ctx.need_prod or need[4]:
+            dP = torch.empty((M, NP), dtype=dt, device=dev)
+        if ctx.need_prod:
+            P3, dP3 = P.view(B, L, NP), dP.view(B, L, NP)
+            _, dxf, _, dcw, dcb, ddt, dA = producer_backward(
+                P3[..., :3 * HD], xf, P3[..., N - H:N], conv_w, conv_b, dt_bias, A_log, dq, dk, dv, dg, dbeta, H, D,
+                scale, mult, _dqkv=dP3[..., :3 * HD], _dxb=dP3[..., N - H:N])
+            small[:6], small[7:] = [*dcw, *dcb], [ddt, dA]
+            dxf2 = dxf.view(M, HD)
+            if need_x or need[3]:
+                torch.mm(dxf2, wf2, out=dP[:, f1])
+        if need_x or need[4]:
             if used:
-                problems += [(dz2, P[:, g1], True), (dout2, y.view(M, HD), False)]
-            dw = weight_grads(problems, M)
-            grads[:7] = [*dw[0][0].split([HD, HD, HD, rank, D, H]), dw[1][0]]
-            if used:
-                grads[7:10] = [dw[2][0], dw[3][0], dw[2][1]]
+                torch.mm(dz2, wg2, out=dP[:, g1])
             else:
-                grads[4] = None
-        if any(need[13:]):
-            sources = [*dcw, *dcb, dnw if used else None, ddt, dA]
-            jobs = []
-            for i, (t, (dt, shape)) in enumerate(zip(sources, ctx.small)):
-                if t is None:
-                    continue
-                if dt == torch.float32:
-                    grads[10 + i] = t.view(shape)
-                else:
-                    grads[10 + i] = torch.empty(shape, dtype=dt, device=dev)
-                    jobs.append((t, grads[10 + i].data_ptr(), _DTYPE_CODE[dt]))
-            if jobs:
-                _pack(jobs)
-        return (dx, ds0, None, *(t if n else None for t, n in zip(grads, need[3:])))
+                dP[:, g1].zero_()
+        if need_x:
+            dx = torch.mm(dP[:, :N], wcat[:N]).view(B, L, hidden)
+
+        # the weight gradients: one problem for each run of adjacent maps of x that need one
+        sizes = [HD, HD, HD, rank, D, H]
+        runs: List[List[int]] = []   # first column and end of P, first map and end
+        at = 0
+        for i, j, want in ((0, 3, any(need[:3])), (3, 4, need[3]), (4, 5, need[4] and used), (5, 6, need[5])):
+            end = at + (3 * HD if j == 3 else sizes[i])
+            if want and runs and runs[-1][3] == i:
+                runs[-1][1], runs[-1][3] = end, j
+            elif want:
+                runs.append([at, end, i, j])
+            at = end
+        problems = [(dP[:, a:b], x2, False) for a, b, _, _ in runs]
+        into = []
+        if need[6]:
+            into.append(6)
+            problems.append((dxf2, P[:, f1], False))
+        if used and (need[7] or need[9]):
+            into.append(7)
+            problems.append((dz2, P[:, g1], True))
+        if used and need[8]:
+            into.append(8)
+            problems.append((dout2, y.view(M, HD), False))
+        if problems:
+            dw = weight_grads(problems, M)
+            for (_, _, i, j), (d, _) in zip(runs, dw):
+                grads[i:j] = d.split(sizes[i:j])
+            for m, (d, db) in zip(into, dw[len(runs):]):
+                grads[m] = d
+                if db is not None:
+                    grads[9] = db
+        jobs = []
+        for i, (t, (dtype, shape)) in enumerate(zip(small, ctx.small)):
+            if t is None or not need[10 + i]:
+                continue
+            if dtype == torch.float32:
+                grads[10 + i] = t.view(shape)
+            else:
+                grads[10 + i] = torch.empty(shape, dtype=dtype, device=dev)
+                jobs.append((t, grads[10 + i].data_ptr(), _DTYPE_CODE[dtype]))
+        if jobs:
+            _pack(jobs)
+        return (dx, ds0, None, *(t if n else None for t, n in zip(grads, need)))

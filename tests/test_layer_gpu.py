@@ -637,3 +637,71 @@ def test_layer_output_in_place():
         assert torch.equal(a, b)
     plain += torch.ones(1, dtype=plain.dtype, device=DEV, requires_grad=True)
     assert plain.requires_grad and torch.equal(plain, 1 + out / 2)
+
+
+def _records(fn):
+    """(fn(), the ids of the library's kernels that it launched)."""
+    from mlx_vit_amd import _lib
+    import ctypes
+    lib = _lib.load()
+    lib.kda_profile_enable(1)
+    try:
+        out = fn()
+        torch.cuda.synchronize()
+    finally:
+        lib.kda_profile_enable(0)
+    ms, n, ids = ctypes.c_double(), ctypes.c_int(), set()
+    for i in range(_lib.PROF_NKERNELS):
+        _lib.check(lib.kda_profile_read(i, ctypes.byref(ms), ctypes.byref(n)), "kda_profile_read")
+        if n.value:
+            ids.add(i)
+    return out, ids
+
+
+_PREP_TRAIN, _LOCAL, _PRODUCER_BWD, _NORM_BWD = 6, 5, 8, 10
+_WHOLE = {_PREP_TRAIN, _LOCAL, _PRODUCER_BWD, _NORM_BWD}
+
+
+@pytest.mark.parametrize("trained,backward_kernels,problems", [
+    (("o_proj",), set(), [(192, 192)]),
+    (("o_norm",), {_NORM_BWD}, []),
+    (("g_proj_2.bias",), {_NORM_BWD}, [(192, 64)]),
+    (("g_proj_1", "o_proj"), {_NORM_BWD}, [(64, 192), (192, 192)]),
+    (("k_proj",), _WHOLE, [(576, 192)]),
+    (("q_proj", "f_proj_1"), _WHOLE, [(640, 192)]),
+    (("f_proj_1", "b_proj"), _WHOLE, [(64, 192), (3, 192)]),
+    (("f_proj_2", "v_conv1d"), _WHOLE, [(192, 64)]),
+    (("A_log", "dt_bias"), _WHOLE, []),
+    (("x",), _WHOLE, []),
+    (("state",), _WHOLE - {_PRODUCER_BWD}, []),
+])
+def test_layer_frozen_parameters(trained, backward_kernels, problems, monkeypatch):
+    """With some parameters frozen the layer launches what their gradients need and
+    no more -- recurrence, producer and norm backward, weight gradients by shape
+    -- and those gradients are the ones of the layer trained whole (the sums over
+    the tokens in another split: bf16 results by their own rounding)."""
+    from mlx_vit_amd import layer as layer_module
+    H, D, L = 3, 64, 100
+    layer = _bf16_layer(H, D)
+    x, s0 = _bf16_randn(1, 2, L, H * D), 0.1 * _bf16_randn(2, 2, H, D, D).float()
+    dout = _bf16_randn(3, 2, L, H * D)
+    shapes = []
+    weight_grads = layer_module.weight_grads
+    monkeypatch.setattr(layer_module, "weight_grads", lambda p, rows: (
+        shapes.extend((dy.shape[1], t.shape[1]) for dy, t, _ in p), weight_grads(p, rows))[1])
+
+    def run(pick):
+        named = [("x", x.detach()), ("state", s0.detach()), *layer.named_parameters()]
+        leaves = {n: t.requires_grad_(pick(n)) for n, t in named if t.is_leaf}
+        out, s = layer(leaves["x"], leaves["state"])
+        want = [n for n in leaves if pick(n)]
+        return out, s, dict(zip(want, torch.autograd.grad(out, [leaves[n] for n in want], dout)))
+
+    out, s, ref = run(lambda n: True)
+    shapes.clear()
+    (out_f, s_f, got), ids = _records(lambda: run(lambda n: n.startswith(trained)))
+    assert ids & _WHOLE == backward_kernels and sorted(shapes) == sorted(problems)
+    through = bool(backward_kernels & {_LOCAL})
+    assert out_f.requires_grad and s_f.requires_grad == through
+    assert torch.equal(out, out_f) and torch.equal(s, s_f)
+    _check({n: _rel(g, ref[n]) for n, g in got.items()}, TOL[torch.bfloat16], f"frozen all but {trained}")
