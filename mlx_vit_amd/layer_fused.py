@@ -24,7 +24,7 @@ from torch.autograd import forward_ad
 from torch.nn.modules import module as _nn_module
 
 from . import _lib
-from .kda import _DTYPE_CODE, _stream, kda_backward, kda_backward_train, kda_forward, kda_forward_train
+from .kda import _DTYPE_CODE, _stream, chunk_kda, kda_backward, kda_backward_train, kda_forward, kda_forward_train
 
 _PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
 # positions in ``fused_params``' order: those whose gradient comes through the
@@ -149,6 +149,21 @@ def _forward(x, state, spec, params, train: bool):
     return out, s_final, (x2, P, xf, z, q, k, v, g, beta, state, o, y, wcat, fp, wf2, wg2, wo), ws
 
 
+def _by_modules(x, state, spec, params):
+    """What ``GatedDeltaLayer.forward`` computes map by map, one autograd node each."""
+    from .layer import CONV_TAPS, GatedRMSNormFunction, ProducerFunction
+    H, D, scale, mult, eps, chunk = spec
+    wq, wk, wv, wf1, wg1, wb, wf2, wg2, wo, bg2, *small = params
+    conv_w = torch.stack([w.reshape(H * D, CONV_TAPS) for w in small[:3]])
+    nw, dt_bias, A_log = small[6:]
+    q, k, v, g, beta = ProducerFunction.apply(
+        F.linear(x, torch.cat([wq, wk, wv])), F.linear(F.linear(x, wf1), wf2), F.linear(x, wb), conv_w,
+        torch.stack(small[3:6]), dt_bias, A_log, H, D, scale, mult, torch.float32)
+    o, s_final = chunk_kda(q, k, v, g, beta, state, chunk)
+    gate = F.linear(F.linear(x, wg1), wg2, bg2)
+    return F.linear(GatedRMSNormFunction.apply(o, gate, nw, eps), wo), s_final
+
+
 def fused_layer(x, state, spec, params):
     """(out, new_state) of the layer for x (B, L, hidden).  ``spec`` = (H, D, scale,
     beta_mult, eps, chunk_size); ``params`` as ``fused_params`` orders them."""
@@ -177,17 +192,37 @@ class FusedLayerFunction(torch.autograd.Function):
             x2, P, xf, z, q, k, v, g, beta, s0, o, *rest = saved
             saved = (x2 if need[7] else None, P if need[10] or need[12] else None, None, z if ctx.need_norm else None,
                      None, None, None, None, None, None, o if ctx.need_norm else None, *rest)
-        ctx.save_for_backward(*saved)
+        ctx.save_for_backward(*saved, x, state)
+        ctx.params, ctx.versions = params, [p._version for p in params]
         ctx.spec, ctx.shape = spec, (*x.shape, params[3].shape[0])
         ctx.small = [(p.dtype, p.shape) for p in params[10:]]
         ctx.set_materialize_grads(False)
         return out, s_final
 
     @staticmethod
-    @torch.no_grad()
     def backward(ctx, dout, ds_final):
+        if torch.is_grad_enabled():
+            return FusedLayerFunction._backward_with_graph(ctx, dout, ds_final)
+        return FusedLayerFunction._backward(ctx, dout, ds_final)
+
+    @staticmethod
+    def _backward_with_graph(ctx, dout, ds_final):
+        """``create_graph``: through the separate nodes, whose gradients keep a graph
+        where theirs do (the linear maps; the kernels' adjoints have none)."""
+        x, state = ctx.saved_tensors[-2:]
+        if [p._version for p in ctx.params] != ctx.versions:
+            raise RuntimeError("a parameter of the layer was modified in place before its backward")
+        outs = zip(_by_modules(x, state, ctx.spec, ctx.params), (dout, ds_final))
+        outs, cots = zip(*[(t, c) for t, c in outs if c is not None])
+        inputs = (x, state, None, *ctx.params)
+        got = iter(torch.autograd.grad(outs, [t for t, n in zip(inputs, ctx.needs_input_grad) if n], cots,
+                                       create_graph=True, allow_unused=True))
+        return tuple(next(got) if n else None for n in ctx.needs_input_grad)
+
+    @staticmethod
+    def _backward(ctx, dout, ds_final):
         from .layer import gated_rmsnorm_backward, producer_backward, weight_grads
-        x2, P, xf, z, q, k, v, g, beta, s0, o, y, wcat, fp, wf2, wg2, wo = ctx.saved_tensors
+        x2, P, xf, z, q, k, v, g, beta, s0, o, y, wcat, fp, wf2, wg2, wo, _, _ = ctx.saved_tensors
         H, D, scale, mult, eps, chunk = ctx.spec
         B, L, hidden, rank = ctx.shape
         M, HD, NP = B * L, H * D, wcat.shape[0]

@@ -705,3 +705,37 @@ def test_layer_frozen_parameters(trained, backward_kernels, problems, monkeypatc
     assert out_f.requires_grad and s_f.requires_grad == through
     assert torch.equal(out, out_f) and torch.equal(s, s_f)
     _check({n: _rel(g, ref[n]) for n, g in got.items()}, TOL[torch.bfloat16], f"frozen all but {trained}")
+
+
+def test_layer_create_graph():
+    """Gradients taken with create_graph keep the graph that the separate modules
+    give them: the same first gradients, and the same derivatives of a function of
+    them (through the linear maps; the kernels' adjoints have none), to the bf16 bar
+    (the cotangent 2 out comes from the one node's forward, whose products are
+    stacked)."""
+    layer = _bf16_layer(3, 64)
+    x0, s0 = _bf16_randn(1, 2, 50, 192), 0.1 * _bf16_randn(2, 2, 3, 64, 64).float()
+    names = [n for n, _ in layer.named_parameters()]
+
+    def run():
+        x = x0.clone().requires_grad_()
+        leaves = [x, *layer.parameters()]
+        out, s = layer(x, s0)
+        first = torch.autograd.grad([out.square().sum(), s.square().sum()], leaves, create_graph=True)
+        assert all(t.requires_grad for t in first[:1])
+        penalty = sum(t.float().square().sum() for t in first)
+        return first, torch.autograd.grad(penalty, leaves, allow_unused=True)
+
+    first, second = run()
+    handle = layer.b_proj.register_forward_hook(lambda *a: None)   # module by module
+    first_m, second_m = run()
+    handle.remove()
+    assert [t is None for t in second] == [t is None for t in second_m]
+    errs = {n: _rel(a, b) for n, a, b in zip(["x"] + names, first, first_m)}
+    errs.update({"second:" + n: _rel(a, b) for n, a, b in zip(["x"] + names, second, second_m) if a is not None})
+    _check(errs, TOL[torch.bfloat16], "create_graph")
+    out, _ = layer(x0)
+    with torch.no_grad():
+        layer.q_proj.weight.mul_(1.0)
+    with pytest.raises(RuntimeError, match="modified in place"):
+        torch.autograd.grad(out.sum(), layer.q_proj.weight, create_graph=True)
