@@ -131,8 +131,12 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
         p.Q.load(gQp, D);
         p.A.load(gAqk, C);
     }
-    for (int n = 0; n < a.nc; ++n) {
-        const int nx = min(n + 1, a.nc - 1);   // the next chunk's loads (the last one's again at the end)
+    // more: another chunk follows, whose operands are loaded as this one's are used.
+    // The last chunk is a copy of its own: its loads again cost 64 x 64 tokens x 12
+    // x 64 73.6 us of forward against 65, a branch around them 4 us of 95 at 25 chunks
+    auto step = [&](int n, auto more_c) __attribute__((always_inline)) {
+        constexpr bool more = decltype(more_c)::value;
+        const int nx = n + 1;
         lds_barrier();                         // the state's planes
         Frag8 Bs[CTV][D / 32];
 #pragma unroll
@@ -154,7 +158,7 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
             vp[j] = p.U[j] - vp[j];
             L.v.put(v0 + 16 * j, BS * m, vp[j]);
         }
-        load_wu(nx);
+        if constexpr (more) load_wu(nx);
         if constexpr (MODE == 1) {
             float* h = static_cast<float*>(a.h) + (ch0 + n) * D * D + (BS * mt + 4 * g4) * D + c0 + r16;
             float* V = static_cast<float*>(a.Vp) + (ch0 + n) * C * D + (BS * m + 4 * g4) * D + c0 + v0 + r16;
@@ -177,7 +181,7 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
 #pragma unroll
                 for (int j = 0; j < CTV; ++j) O[j] = mma<3>(A, Bs[j][ks], O[j]);
             }
-            p.Q.load(gQp + (size_t)nx * C * D, D);
+            if constexpr (more) p.Q.load(gQp + (size_t)nx * C * D, D);
         }
         lds_barrier();                         // V' planes; every wave has read the state's
         Frag8 Bv[CT][C / 32];
@@ -198,7 +202,7 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
             }
 #pragma unroll
             for (int j = 0; j < CT; ++j) L.s.put(16 * j, BS * mt, S[j]);
-            load_k(nx);
+            if constexpr (more) load_k(nx);
         }
         if constexpr (MODE == 0) {
             // O = Qp S + A_qk V' (A_qk lower triangular)
@@ -210,7 +214,7 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
                 for (int j = 0; j < CTV; ++j)
                     O[j] = mma<3>(A, WC == 1 ? Bv[j][ks] : L.v.frag(v0 + 16 * j, 32 * ks), O[j]);
             }
-            p.A.load(gAqk + (size_t)nx * C * C, C);
+            if constexpr (more) p.A.load(gAqk + (size_t)nx * C * C, C);
             const int t0 = n * C + BS * m + 4 * g4;
             const size_t row = (size_t)b * a.T + t0;
             float* o = static_cast<float*>(a.o) + (row * a.H + hd) * D + c0 + v0 + r16;
@@ -239,7 +243,9 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
                     }
             }
         }
-    }
+    };
+    for (int n = 0; n < a.nc - 1; ++n) step(n, std::true_type{});
+    step(a.nc - 1, std::false_type{});
     if (MODE == 0 && has && a.s_final)
 #pragma unroll
         for (int j = 0; j < CT; ++j)
@@ -308,8 +314,9 @@ __device__ __forceinline__ void dh_f32_body(const DhArgs& a, F32Lds<D, CT>& L, i
     p.W.load(gW + (size_t)n * C * D, C);
     put_do(n);
     load_do(max(n - 1, 0));
-    for (; n >= 0; --n) {
-        const int nx = max(n - 1, 0);
+    auto step = [&](int n, auto more_c) __attribute__((always_inline)) {   // as in the forward
+        constexpr bool more = decltype(more_c)::value;
+        const int nx = n - 1;
         lds_barrier();                         // the planes of dS and dO
         if (has) {
             float* dh = static_cast<float*>(a.dh) + (ch0 + n) * D * D + (BS * mt + 4 * g4) * D + c0 + r16;
@@ -348,8 +355,10 @@ __device__ __forceinline__ void dh_f32_body(const DhArgs& a, F32Lds<D, CT>& L, i
         }
 #pragma unroll
         for (int j = 0; j < CTV; ++j) L.v.put(v0 + 16 * j, BS * m, -dv[j]);
-        p.A.load(gA + (size_t)nx * C * C, C);
-        p.K.load(gKb + (size_t)nx * C * D, D);
+        if constexpr (more) {
+            p.A.load(gA + (size_t)nx * C * C, C);
+            p.K.load(gKb + (size_t)nx * C * D, D);
+        }
         float* dV = static_cast<float*>(a.dVp) + (ch0 + n) * C * D + (BS * m + 4 * g4) * D + c0 + v0 + r16;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -364,12 +373,16 @@ __device__ __forceinline__ void dh_f32_body(const DhArgs& a, F32Lds<D, CT>& L, i
 #pragma unroll
                 for (int j = 0; j < CT; ++j) S[j] = mma<3>(A, Bo[j][ks], S[j]);
             }
-            p.Q.load(gQ + (size_t)nx * C * D, C);
-            p.eg = *reinterpret_cast<const f32x4*>(gEg + (size_t)nx * D);
+            if constexpr (more) {
+                p.Q.load(gQ + (size_t)nx * C * D, C);
+                p.eg = *reinterpret_cast<const f32x4*>(gEg + (size_t)nx * D);
+            }
         }
         lds_barrier();                         // -dV' planes; every wave has read those of dS and dO
-        put_do(nx);
-        load_do(max(nx - 1, 0));
+        if constexpr (more) {
+            put_do(nx);
+            load_do(max(nx - 1, 0));
+        }
         if (has) {
             Frag8 Bv[CT][C / 32];
 #pragma unroll
@@ -385,9 +398,11 @@ __device__ __forceinline__ void dh_f32_body(const DhArgs& a, F32Lds<D, CT>& L, i
             }
 #pragma unroll
             for (int j = 0; j < CT; ++j) L.s.put(16 * j, BS * mt, S[j]);
-            p.W.load(gW + (size_t)nx * C * D, C);
+            if constexpr (more) p.W.load(gW + (size_t)nx * C * D, C);
         }
-    }
+    };
+    for (; n > 0; --n) step(n, std::true_type{});
+    step(0, std::false_type{});
     if (has && a.ds0)
 #pragma unroll
         for (int j = 0; j < CT; ++j)
@@ -413,6 +428,12 @@ __global__ __launch_bounds__(F32Geom<D>::NTH) void kda_states_dh_f32_kernel(cons
 }
 
 constexpr int F32_CT = 2;   // column tiles per workgroup
+// Whether the forward at D = 64 takes one workgroup per (b, h) instead of two, which
+// read every operand twice: where two would be more than the CUs, and for single
+// chunks earlier.  One against two: 96 x 64 tokens 19.4 / 20.5 us, 128 x 64 19.7 /
+// 22.4, 192 x 64 21.1 / 26.3, 192 x 256 59.7 / 65.1; but 48 x 64 19.2 / 18.2, 128 x 256
+// 46.1 / 44.7, 12 x 1568 112 / 90.
+static bool whole_rows(int BH, int nc) { return BH >= (nc == 1 ? 96 : 129); }
 
 template <int D> hipError_t recur_f32_t(const RecurArgs& a, hipStream_t st) {
     constexpr int NT = D / BS, NTH = F32Geom<D>::NTH;
@@ -421,6 +442,8 @@ template <int D> hipError_t recur_f32_t(const RecurArgs& a, hipStream_t st) {
             hipLaunchKernelGGL((kda_recur_f32_kernel<D, NT, true>), dim3(a.BH), dim3(NTH), 0, st, a);
         else
             return hipErrorInvalidValue;
+    } else if (D == 64 && whole_rows(a.BH, a.nc)) {
+        if constexpr (D == 64) hipLaunchKernelGGL((kda_recur_f32_kernel<D, NT, false>), dim3(a.BH), dim3(NTH), 0, st, a);
     } else {
         hipLaunchKernelGGL((kda_recur_f32_kernel<D, F32_CT, false>), dim3(a.BH * (NT / F32_CT)), dim3(NTH), 0, st, a);
     }

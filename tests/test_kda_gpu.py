@@ -976,3 +976,15 @@ def test_short_sequences_growth_after_strong_decay(T, D, dtype, g_kind):
     errs = {"o": R.rel_l2(o[:, 5:].cpu(), ref["o"][:, 5:]), "s_final": R.rel_l2(sf.cpu(), ref["s_final"]),
             "dv": R.rel_l2(got[2][:, :2].cpu(), refb["dv"][:, :2]), "ds0": R.rel_l2(got[5].cpu(), refb["ds0"])}
     _assert_all(errs, 1e-4 if dtype == torch.float32 else 2.0 ** -8, f"short growth T={T} D={D} {dtype} g={g_kind}")
+
+
+@pytest.mark.parametrize("B,T,H,D", [(24, 33, 4, 64), (24, 64, 4, 64), (32, 65, 4, 64), (43, 65, 3, 64), (43, 129, 3, 64),
+                                     (3, 128, 2, 32), (2, 129, 2, 128)])
+def test_fp32_recurrences_few_chunks(B, T, H, D):
+    """The fp32 recurrences at one to three chunks, the last a copy of its own, on both
+    sides of the forward's bound for one workgroup per (b, h) (96 of them with one
+    chunk, 129 with more): forward and backward, states in and out."""
+    x = _inputs(B, T, H, D, torch.float32, seed=B + T, with_state=True, grad=True, g_scale=0.3)
+    dsf = torch.randn(B, H, D, D, generator=torch.Generator().manual_seed(T))
+    _assert_all(_fwd_errors(x, torch.float32), TOL[torch.float32], f"fwd fp32 {B} {T} {H} {D}")
+    _assert_all(_bwd_errors(x, torch.float32, dsf), TOL[torch.float32], f"bwd fp32 {B} {T} {H} {D}")
