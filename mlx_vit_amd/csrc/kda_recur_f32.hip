@@ -137,6 +137,19 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
     auto step = [&](int n, auto more_c) __attribute__((always_inline)) {
         constexpr bool more = decltype(more_c)::value;
         const int nx = n + 1;
+        // the norm's gate values of this chunk's rows (past T the last one's), used at
+        // the step's end: loaded there they made every step wait (2 x 1568 x 6 x 64 with
+        // the norm 208 -> 172 us)
+        const int t0 = n * C + BS * m + 4 * g4;
+        float z[4][CTV];
+        if constexpr (EPI)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float* zp = static_cast<const float*>(a.z) +
+                                  ((size_t)b * a.T + min(t0 + e, a.T - 1)) * a.ld_z + (size_t)hd * D + r16;
+#pragma unroll
+                for (int j = 0; j < CTV; ++j) z[e][j] = zp[16 * j];
+            }
         lds_barrier();                         // the state's planes
         Frag8 Bs[CTV][D / 32];
 #pragma unroll
@@ -215,7 +228,6 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
                     O[j] = mma<3>(A, WC == 1 ? Bv[j][ks] : L.v.frag(v0 + 16 * j, 32 * ks), O[j]);
             }
             if constexpr (more) p.A.load(gAqk + (size_t)nx * C * C, C);
-            const int t0 = n * C + BS * m + 4 * g4;
             const size_t row = (size_t)b * a.T + t0;
             float* o = static_cast<float*>(a.o) + (row * a.H + hd) * D + c0 + v0 + r16;
             const size_t rs = (size_t)a.H * D;
@@ -236,9 +248,8 @@ __device__ __forceinline__ void recur_f32_body(const RecurArgs& a, F32Lds<D, CT>
                         o[e * rs + 16 * j] = O[j][e];
                         if constexpr (EPI) {
                             const int c = 16 * j + r16;
-                            const float z = static_cast<const float*>(a.z)[(row + e) * a.ld_z + (size_t)hd * D + c];
                             static_cast<float*>(a.y)[(row + e) * a.ld_y + (size_t)hd * D + c] =
-                                O[j][e] * rn * a.nw[c] * sigm(z);
+                                O[j][e] * rn * a.nw[c] * sigm(z[e][j]);
                         }
                     }
             }

@@ -179,6 +179,8 @@ GATED_CASES = [
     (2, 200, 12, 64, torch.bfloat16, True, True, 0),     # four chunks (the LDS sets wrap)
     (2, 100, 3, 64, torch.float32, True, True, 4),
     (1, 77, 2, 32, torch.float32, False, False, 0),
+    (2, 129, 3, 32, torch.float32, True, True, 4),       # a last chunk of one row, a strided gate
+    (2, 65, 2, 64, torch.float32, False, False, 0),
 ]
 
 
