@@ -49,7 +49,7 @@ template <int D, typename ST, typename TG, int PREC, int NTH>
 __global__ __launch_bounds__(NTH) void kda_prep_kernel(const PrepArgs a) {
     using G = PrepGeom<D, ST>;
     constexpr int NW = NTH / 64;   // waves
-    static_assert(NW == 4 || NW == 8, "four or eight waves");
+    static_assert(NW == 4 || NW == 8 || NW == 16, "four, eight or sixteen waves");
     constexpr int LDK = G::LDK, LDA = G::LDA, LDT = G::LDT, NT = D / BS, NCT = 2 * NT;
     constexpr int TPW = (NCT + NW - 1) / NW;
     constexpr int EPV = 16 / (int)sizeof(ST);
@@ -616,17 +616,29 @@ __global__ __launch_bounds__(NTH) void kda_prep_kernel(const PrepArgs a) {
 template <int D, typename ST, typename TG>
 static hipError_t launch_prep_t(const PrepArgs& a, int nchunks, hipStream_t st) {
     constexpr int PREC = std::is_same<ST, float>::value ? 3 : 1;
-    // eight waves per chunk where the registers allow four waves per SIMD
-    constexpr int NTH = (D >= 64) ? KDA_PREP_NTH : 256;
+    // eight waves per chunk where the registers allow four waves per SIMD; bf16 at
+    // D = 128 (133 KB of LDS: one workgroup per CU, 123 VGPRs) sixteen, four per SIMD on
+    // one chunk
+    constexpr int NTH = (D >= 128 && std::is_same<ST, uint16_t>::value) ? 1024 : (D >= 64) ? KDA_PREP_NTH : 256;
     hipLaunchKernelGGL((kda_prep_kernel<D, ST, TG, PREC, NTH>), dim3(nchunks), dim3(NTH), 0, st, a);
     return hipGetLastError();
 }
 
+// bf16 at D = 128 up to this many chunks -- at most one a CU -- in sixteen waves each;
+// kda_prepw.hip's two workgroups a CU have nothing to share then.  Sixteen against
+// eight waves (training prep, us): 8 chunks 15.2 / 16.8, 64 18.0 / 19.7, 192 18.0 /
+// 19.0 and 22.0 / 22.8 at the layer's initial decay; the forward's prep crosses
+// over between 192 (18.6 / 19.3) and 224 (19.1 / 18.7); 320 29.2 / 25.8.
+constexpr int PREP16_CHUNKS = 192;
+
 // g_kind: 0 fp32 g, 1 bf16 g, 2 one fp32 decay per (b, t, h) (bf16 inputs at
-// D <= 64 only).  bf16 at D = 64 and 128 goes to kda_prepw.hip, which keeps less of
-// a chunk in LDS (figures there); fp32 tiles leave no room for a second
+// D <= 64 only).  bf16 at D = 64 and (from 193 chunks) 128 goes to kda_prepw.hip, which
+// keeps less of a chunk in LDS (figures there); fp32 tiles leave no room for a second
 // workgroup either way, and a 32-channel chunk fits three times as it is.
 hipError_t launch_prep(const PrepArgs& a, int D, int in_bf16, int g_kind, int nchunks, hipStream_t st) {
+    if (in_bf16 && D == 128 && nchunks <= PREP16_CHUNKS && g_kind != 2)
+        return g_kind == 1 ? launch_prep_t<128, uint16_t, uint16_t>(a, nchunks, st)
+                           : launch_prep_t<128, uint16_t, float>(a, nchunks, st);
     if (in_bf16 && (D == 64 || D == 128)) return launch_prep_wide(a, D, g_kind, nchunks, st);
     if (in_bf16 && D == 32)
         return g_kind == 2   ? launch_prep_t<32, uint16_t, GHead>(a, nchunks, st)

@@ -316,14 +316,19 @@ def test_bwd_fp32_mixed_blocks(T, D, g_dtype):
 
 
 @pytest.mark.parametrize("T", [65, 191, 256])
-@pytest.mark.parametrize("D,g_dtype", [(64, torch.bfloat16), (64, torch.float32), (96, torch.bfloat16),
-                                       (96, torch.float32), (128, torch.bfloat16), (128, torch.float32)])
-def test_bf16_chunk_kinds(T, D, g_dtype):
+@pytest.mark.parametrize("few,D,g_dtype", [(True, 64, torch.bfloat16), (True, 64, torch.float32),
+                                           (True, 96, torch.bfloat16), (True, 96, torch.float32),
+                                           (True, 128, torch.bfloat16), (True, 128, torch.float32),
+                                           (False, 96, torch.bfloat16), (False, 96, torch.float32),
+                                           (False, 128, torch.bfloat16), (False, 128, torch.float32)])
+def test_bf16_chunk_kinds(T, few, D, g_dtype):
     """bf16 from D = 64 on: a chunk with one block beyond the 16-row span guard and
     one beyond the 4-row guard too, a chunk within both, one with g > 0 somewhere,
     the last of one row, one row short, or whole; every output of the training
-    pair.  TOL: bf16 operands and results, 2^-8 each."""
-    x = _inputs(2, T, 3, D, torch.bfloat16, seed=37 + T + D, with_state=True, grad=True, g_scale=0.2)
+    pair.  Few chunks, and more than 192 (the bound of the sixteen-wave prep at
+    D = 128).  TOL: bf16 operands and results, 2^-8 each."""
+    B = 2 if few else 66 // (-(-T // 64)) + 1   # of 3 heads: at least 198 chunks
+    x = _inputs(B, T, 3, D, torch.bfloat16, seed=37 + T + D, with_state=True, grad=True, g_scale=0.2)
     g = x["g"].float()
     g[:, :16] *= 60.0
     g[:, 48:64] -= 25.0
