@@ -37,6 +37,7 @@ constexpr int MAXW = 8;      // H*D <= 2048
 constexpr int PR = 3;        // producer forward: rows per workgroup
 constexpr int BR = 4;        // producer backward: rows per strip
 constexpr int BNS = 8;       // producer backward: strips per workgroup
+constexpr int BGROUPS = 128; // producer backward: groups of short sequences at least
 constexpr int NR = 4;        // norm forward: rows per workgroup
 constexpr int NRB = 4;       // norm backward: rows per strip
 constexpr int NNS = 2;       // norm backward: strips per workgroup
@@ -468,8 +469,14 @@ __device__ __forceinline__ void prod_bwd_conv(const ProdArgs& a, const Lanes& L,
 // Sequences shorter than a segment: as many of them per workgroup as fill one,
 // so that the parameter-gradient partials (17 H*D floats a workgroup) stay a
 // small part of the traffic (1568 sequences of 8 tokens: 82 MB written and
-// read with one each)
-__host__ __device__ __forceinline__ int prod_seqs(int T) { return T * 2 > BR * BNS ? 1 : BR * BNS / (T > 0 ? T : 1); }
+// read with one each) -- but no fewer than BGROUPS workgroups for each of the
+// four roles, two a CU in all: a workgroup takes its sequences one after
+// another.  H*D = 768, without the bound / with it: 64 sequences of one token 83 /
+// 38 us, 512 of one 86 / 38, 1568 of one 92 / 54, 512 of eight 40 / 40; one sequence
+// a workgroup 38, 53, 123 and 64 us.
+__host__ __device__ __forceinline__ int prod_seqs(int B, int T) {
+    return T * 2 > BR * BNS ? 1 : max(1, min(BR * BNS / max(T, 1), B / BGROUPS));
+}
 
 
 // Workgroup = (batch row b, segment of BR*BNS tokens; or prod_seqs short
@@ -492,7 +499,7 @@ __global__ __launch_bounds__(512) void producer_bwd_kernel(const ProdArgs a) {
     const Lanes L(a.H, a.D);
     const int T = a.T;
     constexpr int SEG = BR * BNS;
-    const int nseg = (T + SEG - 1) / SEG, nb = prod_seqs(T);
+    const int nseg = (T + SEG - 1) / SEG, nb = prod_seqs(a.B, T);
     const int wg = xcd_remap(blockIdx.x, gridDim.x);
     const int b0 = wg / nseg * nb, b1 = min(a.B, b0 + nb), tlo = (wg % nseg) * SEG;
     const int thi = min(tlo + SEG, T);
@@ -771,7 +778,7 @@ int norm_waves(int H, int D) {
 }
 
 int producer_partials(int B, int T) {
-    const int nb = prod_seqs(T);
+    const int nb = prod_seqs(B, T);
     return (B + nb - 1) / nb * ((T + BR * BNS - 1) / (BR * BNS));
 }
 size_t producer_ws_floats(int B, int T, int H, int D) {

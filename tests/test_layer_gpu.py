@@ -67,6 +67,15 @@ PRODUCER_CASES = [
     (2, 300, 4, 64, torch.float32, True, 1.0),
     (4, 260, 3, 64, torch.bfloat16, True, 1.0),
     (2, 37, 8, 96, torch.float32, True, 1.0),      # the SSv2 layer's 8 heads x 96
+    # short sequences, several in one workgroup of the backward: 3 of 10 tokens
+    # with two over, 2 of 16, up to 32 of one; 17 tokens are a segment of their own
+    (386, 10, 1, 32, torch.float32, True, 1.0),
+    (385, 10, 2, 32, torch.bfloat16, True, 1.0),
+    (257, 16, 1, 32, torch.float32, False, 2.0),
+    (131, 17, 1, 32, torch.float32, True, 1.0),
+    (130, 1, 2, 64, torch.float32, True, 1.0),
+    (4100, 1, 1, 32, torch.bfloat16, True, 1.0),
+    (1031, 4, 1, 32, torch.float32, True, 1.0),
 ]
 
 
