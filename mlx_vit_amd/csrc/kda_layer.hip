@@ -34,7 +34,14 @@ namespace {
 constexpr int KC = 4;        // conv taps (ShortCausalConv1d(kernel_size=4))
 constexpr int CPW = 256;     // channels per wave
 constexpr int MAXW = 8;      // H*D <= 2048
-constexpr int PR = 3;        // producer forward: rows per workgroup
+// producer forward: rows per workgroup (PR).  A strip reads PR + 3 rows and forms PR:
+// three, or two where that is less together (1, 2, 4 or, in bf16, where forming
+// counts as much as reading, 10 tokens).  H*D = 768, three / two rows: bf16 4096
+// sequences of 2 tokens 36.1 / 31.5 us, 1568 of 4 32.1 / 27.6, of 10 57.4 / 54.8, of 5
+// 33.1 / 36.4, of 8 46.3 / 47.9; fp32 4096 of 10 249 / 253.
+constexpr int prod_rows(int T, bool bf16) {
+    return (T + 1) / 2 * (5 + 2 * bf16) <= (T + 2) / 3 * (6 + 3 * bf16) ? 2 : 3;
+}
 constexpr int BR = 4;        // producer backward: rows per strip
 constexpr int BNS = 8;       // producer backward: strips per workgroup
 constexpr int BGROUPS = 128; // producer backward: groups of short sequences at least
@@ -146,7 +153,7 @@ __device__ __forceinline__ void load_taps(const ProdArgs& a, const Lanes& L, flo
 // The conv input is a template parameter so that its pointer is a fixed field
 // of the kernel arguments (a runtime choice among xq / xk / xv makes the
 // compiler copy the argument block to scratch memory).
-template <typename ST, int I>
+template <typename ST, int I, int PR>
 __device__ __forceinline__ void conv_silu_rows(const ProdArgs& a, const Lanes& L, int t0, size_t rb,
                                                float (&out)[PR][4]) {
     const int T = a.T;
@@ -178,7 +185,7 @@ __device__ __forceinline__ void conv_silu_rows(const ProdArgs& a, const Lanes& L
 // and stored, held in registers across it (80 VGPRs).  HBM-bound: 12544 x 768
 // bf16 with fp32 g, 173 MB, 45.6 us on warm inputs (3.8 TB/s) against 47.8 and
 // 49.8 us at 2 and 4 rows (a strip reads PR + 3 rows of each conv input).
-template <typename ST, typename GT>
+template <typename ST, typename GT, int PR>
 __global__ __launch_bounds__(512) void producer_fwd_kernel(const ProdArgs a) {
     __shared__ float red[2][MAXW][PR];
     const Lanes L(a.H, a.D);
@@ -200,13 +207,13 @@ __global__ __launch_bounds__(512) void producer_fwd_kernel(const ProdArgs a) {
         }
     };
     float sq[PR][4], sk[PR][4];
-    conv_silu_rows<ST, 0>(a, L, t0, rb, sq);
+    conv_silu_rows<ST, 0, PR>(a, L, t0, rb, sq);
     row_norms(sq, 0);
-    conv_silu_rows<ST, 1>(a, L, t0, rb, sk);
+    conv_silu_rows<ST, 1, PR>(a, L, t0, rb, sk);
     row_norms(sk, 1);
     {
         float sv[PR][4];
-        conv_silu_rows<ST, 2>(a, L, t0, rb, sv);
+        conv_silu_rows<ST, 2, PR>(a, L, t0, rb, sv);
 #pragma unroll
         for (int j = 0; j < PR; ++j)
             if (t0 + j < T && L.live) Vec4<ST>::st(static_cast<ST*>(a.v) + (rb + t0 + j) * L.HD + L.cc, sv[j]);
@@ -791,15 +798,21 @@ size_t rmsnorm_ws_floats(int rows, int H, int D) {
     return ((size_t)P + 1 + colsum_splits(P, N)) * N;
 }
 
-hipError_t launch_producer_fwd(const ProdArgs& a, int in_bf16, int g_bf16, hipStream_t st) {
+template <int PR>
+static void producer_fwd_rows(const ProdArgs& a, int in_bf16, int g_bf16, hipStream_t st) {
     const dim3 grid(a.B * ((a.T + PR - 1) / PR)), block(64 * nwaves(a.H, a.D));
     if (in_bf16) {
-        if (g_bf16) producer_fwd_kernel<uint16_t, uint16_t><<<grid, block, 0, st>>>(a);
-        else producer_fwd_kernel<uint16_t, float><<<grid, block, 0, st>>>(a);
+        if (g_bf16) producer_fwd_kernel<uint16_t, uint16_t, PR><<<grid, block, 0, st>>>(a);
+        else producer_fwd_kernel<uint16_t, float, PR><<<grid, block, 0, st>>>(a);
     } else {
-        if (g_bf16) producer_fwd_kernel<float, uint16_t><<<grid, block, 0, st>>>(a);
-        else producer_fwd_kernel<float, float><<<grid, block, 0, st>>>(a);
+        if (g_bf16) producer_fwd_kernel<float, uint16_t, PR><<<grid, block, 0, st>>>(a);
+        else producer_fwd_kernel<float, float, PR><<<grid, block, 0, st>>>(a);
     }
+}
+
+hipError_t launch_producer_fwd(const ProdArgs& a, int in_bf16, int g_bf16, hipStream_t st) {
+    if (prod_rows(a.T, in_bf16) == 2) producer_fwd_rows<2>(a, in_bf16, g_bf16, st);
+    else producer_fwd_rows<3>(a, in_bf16, g_bf16, st);
     return hipGetLastError();
 }
 

@@ -76,6 +76,11 @@ PRODUCER_CASES = [
     (130, 1, 2, 64, torch.float32, True, 1.0),
     (4100, 1, 1, 32, torch.bfloat16, True, 1.0),
     (1031, 4, 1, 32, torch.float32, True, 1.0),
+    # strips of the forward: of two rows at 2 and 4 tokens (and 10, above, in bf16), of three at 6 and 7
+    (3, 2, 3, 64, torch.float32, True, 1.0),
+    (3, 4, 3, 64, torch.bfloat16, True, 1.0),
+    (2, 6, 3, 64, torch.float32, True, 1.0),
+    (2, 7, 3, 64, torch.bfloat16, True, 1.0),
 ]
 
 
