@@ -168,6 +168,8 @@ def fused_layer(x, state, spec, params):
     """(out, new_state) of the layer for x (B, L, hidden).  ``spec`` = (H, D, scale,
     beta_mult, eps, chunk_size); ``params`` as ``fused_params`` orders them."""
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, state, *params)):
+        if any(t is not None and t.is_inference() for t in (x, state, *params)):
+            return _by_modules(x, state, spec, params)   # a node cannot save inference tensors
         return FusedLayerFunction.apply(x, state, spec, *params)
     out, s_final, _, _ = _forward(x, state, spec, params, False)
     return out, s_final

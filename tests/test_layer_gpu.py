@@ -755,3 +755,18 @@ def test_layer_create_graph():
         layer.q_proj.weight.mul_(1.0)
     with pytest.raises(RuntimeError, match="modified in place"):
         torch.autograd.grad(out.sum(), layer.q_proj.weight, create_graph=True)
+
+
+def test_layer_inference_tensor_input():
+    """x made under inference_mode with a gradient wanted for the state only: nothing
+    of x has to be saved, and the layer takes it, as the separate modules do."""
+    layer = _bf16_layer(3, 64).requires_grad_(False)
+    plain = _bf16_randn(1, 2, 50, 192)
+    with torch.inference_mode():
+        x = plain.clone()
+    grads = []
+    for t in (x, plain):
+        s0 = (0.1 * _bf16_randn(2, 2, 3, 64, 64).float()).requires_grad_()
+        out, s = layer(t, s0)
+        grads += [out.detach(), *torch.autograd.grad([out.float().sum(), s.sum()], s0)]
+    _check({"out": _rel(grads[0], grads[2]), "ds0": _rel(grads[1], grads[3])}, TOL[torch.bfloat16], "inference x")
