@@ -106,8 +106,9 @@ def _views(fp: torch.Tensor, HD: int, D: int):
             fp[15 * HD + D:16 * HD + D], fp[16 * HD + D:])
 
 
-def _forward(x, state, spec, params, train: bool):
-    """(out, new_state, what the backward reads, the training pair's workspace)."""
+def _forward(x, state, spec, params, train: bool, keep: bool):
+    """(out, new_state, what the backward reads, the training pair's workspace).
+    Without ``keep`` each tensor is given up after its last use."""
     from .layer import gated_rmsnorm_forward, producer_forward
     H, D, scale, mult, eps, chunk = spec
     wq, wk, wv, wf1, wg1, wb, wf2, wg2, wo, bg2 = params[:10]
@@ -138,12 +139,18 @@ def _forward(x, state, spec, params, train: bool):
     z = torch.addmm(bg2, P[:, 3 * HD + rank:3 * HD + rank + D], wg2.t()).view(B, L, HD)
     q, k, v, g, beta = producer_forward(P3[..., :3 * HD], xf, P3[..., N - H:N], conv_w, conv_b, dt_bias, A_log,
                                         H, D, scale, mult, torch.float32)
+    if not keep:
+        x2 = P = P3 = xf = wcat = None
     ws = None
     if train:
         o, s_final, ws = kda_forward_train(q, k, v, g, beta, state, chunk)
     else:
         o, s_final = kda_forward(q, k, v, g, beta, state, chunk)
+    if not keep:
+        q = k = v = g = beta = None
     y = gated_rmsnorm_forward(o, z, nw, eps)
+    if not keep:
+        o = z = None
     # no view of the product: a node's output that is one refuses in-place operations
     out = F.linear(y, wo)
     return out, s_final, (x2, P, xf, z, q, k, v, g, beta, state, o, y, wcat, fp, wf2, wg2, wo), ws
@@ -171,8 +178,7 @@ def fused_layer(x, state, spec, params):
         if any(t is not None and t.is_inference() for t in (x, state, *params)):
             return _by_modules(x, state, spec, params)   # a node cannot save inference tensors
         return FusedLayerFunction.apply(x, state, spec, *params)
-    out, s_final, _, _ = _forward(x, state, spec, params, False)
-    return out, s_final
+    return _forward(x, state, spec, params, False, False)[:2]
 
 
 class FusedLayerFunction(torch.autograd.Function):
@@ -187,7 +193,7 @@ class FusedLayerFunction(torch.autograd.Function):
         # what reaches the recurrence: x, every map and gate of its operands, the state
         ctx.need_prod = need[0] or any(need[3 + i] for i in _BEFORE_RECURRENCE)
         ctx.need_rec = ctx.need_prod or need[1]
-        out, s_final, saved, ctx.ws = _forward(x, state, spec, params, ctx.need_rec)
+        out, s_final, saved, ctx.ws = _forward(x, state, spec, params, ctx.need_rec, True)
         ctx.need_norm = ctx.need_rec or need[19] or any(need[3 + i] for i in (4, 7, 9))   # or the gate's maps
         if not ctx.need_rec:
             ctx.mark_non_differentiable(s_final)
@@ -242,6 +248,7 @@ class FusedLayerFunction(torch.autograd.Function):
                 dy = torch.mm(dout2, wo).view(B, L, HD)
                 do, dz, small[6] = gated_rmsnorm_backward(o, z, nw, eps, dy)
                 dz2 = dz.view(M, HD)
+                del dy, dz
         elif ctx.need_rec:
             do = torch.zeros_like(o)
         dx = ds0 = None
@@ -253,6 +260,7 @@ class FusedLayerFunction(torch.autograd.Function):
             else:   # another backward of a retained graph
                 dq, dk, dv, dg, dbeta, ds0 = kda_backward(q, k, v, g, beta, s0, do, ds_final, chunk,
                                                           _need_ds0=need_ds0)
+            do = None
         if ctx.need_prod or need[4]:
             dP = torch.empty((M, NP), dtype=dt, device=dev)
         if ctx.need_prod:
@@ -261,6 +269,7 @@ class FusedLayerFunction(torch.autograd.Function):
                 P3[..., :3 * HD], xf, P3[..., N - H:N], conv_w, conv_b, dt_bias, A_log, dq, dk, dv, dg, dbeta, H, D,
                 scale, mult, _dqkv=dP3[..., :3 * HD], _dxb=dP3[..., N - H:N])
             small[:6], small[7:] = [*dcw, *dcb], [ddt, dA]
+            dq = dk = dv = dg = None
             dxf2 = dxf.view(M, HD)
             if need_x or need[3]:
                 torch.mm(dxf2, wf2, out=dP[:, f1])

@@ -770,3 +770,28 @@ def test_layer_inference_tensor_input():
         out, s = layer(t, s0)
         grads += [out.detach(), *torch.autograd.grad([out.float().sum(), s.sum()], s0)]
     _check({"out": _rel(grads[0], grads[2]), "ds0": _rel(grads[1], grads[3])}, TOL[torch.bfloat16], "inference x")
+
+
+def test_layer_inference_memory():
+    """Without gradients the layer as one node holds no more memory at a time than
+    module by module (its stacked weight has the gates' rows besides q, k and v's)."""
+    H, D, B, L = 4, 64, 4, 4096
+    layer = _bf16_layer(H, D)
+    x = _bf16_randn(1, B, L, H * D)
+
+    def peak():
+        with torch.no_grad():
+            layer(x)   # the allocator's first use of these sizes
+            torch.cuda.synchronize()
+            torch.cuda.reset_peak_memory_stats()
+            base = torch.cuda.memory_allocated()
+            out = layer(x)
+            torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - base
+
+    one = peak()
+    handle = layer.b_proj.register_forward_hook(lambda *a: None)
+    modules = peak()
+    handle.remove()
+    print("inference memory", one, modules, flush=True)
+    assert one <= modules + 2 * H * D * (2 * D + H + 8) + 4096
