@@ -195,6 +195,14 @@ GATED_CASES = [
     (1, 77, 2, 32, torch.float32, False, False, 0),
     (2, 129, 3, 32, torch.float32, True, True, 4),       # a last chunk of one row, a strided gate
     (2, 65, 2, 64, torch.float32, False, False, 0),
+    # short sequences, one wave each with its epilogue: rows for 8 and 16 tokens
+    (2, 8, 3, 64, torch.bfloat16, True, True, 8),
+    (87, 9, 3, 64, torch.bfloat16, True, False, 8),      # (above 256 of them at 9 to 16 tokens)
+    (87, 16, 3, 64, torch.bfloat16, False, True, 0),
+    (2, 7, 3, 32, torch.float32, True, True, 4),
+    (2, 16, 3, 32, torch.float32, False, True, 0),
+    (3, 8, 2, 64, torch.float32, False, False, 0),
+    (2, 13, 2, 64, torch.float32, True, True, 4),
 ]
 
 
