@@ -227,14 +227,10 @@ def _i64(rows) -> ctypes.Array:
 
 
 def _dma_rows(t: torch.Tensor) -> torch.Tensor:
-    """t (rows, n) bf16 as ``kda_weight_grad`` reads it, 16 bytes at a time: a 16-byte
-    aligned base and row stride, rows that hold n rounded up to 8; copied when not."""
+    """A copy of t (rows, n) bf16 that ``kda_weight_grad`` can read 16 bytes at a time:
+    aligned, its rows n rounded up to 8."""
     rows, n = t.shape
-    n8 = -(-n // 8) * 8
-    if t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(0) >= n8:
-        return t
-    out = torch.empty((rows, n8), dtype=t.dtype, device=t.device)[:, :n]
-    return out.copy_(t)
+    return torch.empty((rows, -(-n // 8) * 8), dtype=t.dtype, device=t.device)[:, :n].copy_(t)
 
 
 def weight_grads(problems, rows: int):
@@ -248,14 +244,16 @@ def weight_grads(problems, rows: int):
         for name, t in (("dy", dy), ("x", x)):
             if t.dim() != 2 or t.shape[0] != rows or t.dtype != torch.bfloat16 or t.stride(1) != 1 or t.device != dev:
                 raise ValueError(f"{name} must be a ({rows}, n) bfloat16 matrix with unit column stride on {dev}")
-        dy, x = _dma_rows(dy), _dma_rows(x)
-        keep.append((dy, x))
         n, k = dy.shape[1], x.shape[1]
+        pdy, px, ld_dy, ld_x = dy.data_ptr(), x.data_ptr(), dy.stride(0), x.stride(0)
+        if (pdy | px) & 15 or (ld_dy | ld_x) & 7 or ld_dy < (n + 7 & ~7) or ld_x < k:
+            dy, x = _dma_rows(dy), _dma_rows(x)
+            keep += [dy, x]
+            pdy, px, ld_dy, ld_x = dy.data_ptr(), x.data_ptr(), dy.stride(0), x.stride(0)
         dw = torch.empty((n, k), dtype=torch.bfloat16, device=dev)
         db = torch.empty((n,), dtype=torch.bfloat16, device=dev) if bias else None
         out.append((dw, db))
-        fields.append((dy.data_ptr(), x.data_ptr(), dw.data_ptr(), 0 if db is None else db.data_ptr(),
-                       dy.stride(0), x.stride(0), n, k))
+        fields.append((pdy, px, dw.data_ptr(), 0 if db is None else db.data_ptr(), ld_dy, ld_x, n, k))
     lib = _lib.load()
     arr = _i64(fields)
     nws = lib.kda_weight_grad_workspace_size(arr, len(fields), rows)

@@ -175,8 +175,8 @@ def fused_layer(x, state, spec, params):
     """(out, new_state) of the layer for x (B, L, hidden).  ``spec`` = (H, D, scale,
     beta_mult, eps, chunk_size); ``params`` as ``fused_params`` orders them."""
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, state, *params)):
-        if any(t is not None and t.is_inference() for t in (x, state, *params)):
-            return _by_modules(x, state, spec, params)   # a node cannot save inference tensors
+        if x.is_inference():
+            return _by_modules(x, state, spec, params)   # a node cannot save it
         return FusedLayerFunction.apply(x, state, spec, *params)
     return _forward(x, state, spec, params, False, False)[:2]
 
@@ -283,28 +283,33 @@ class FusedLayerFunction(torch.autograd.Function):
 
         # the weight gradients: one problem for each run of adjacent maps of x that need one
         sizes = [HD, HD, HD, rank, D, H]
-        runs: List[List[int]] = []   # first column and end of P, first map and end
-        at = 0
-        for i, j, want in ((0, 3, any(need[:3])), (3, 4, need[3]), (4, 5, need[4] and used), (5, 6, need[5])):
-            end = at + (3 * HD if j == 3 else sizes[i])
-            if want and runs and runs[-1][3] == i:
-                runs[-1][1], runs[-1][3] = end, j
-            elif want:
-                runs.append([at, end, i, j])
-            at = end
-        problems = [(dP[:, a:b], x2, False) for a, b, _, _ in runs]
-        into = []
-        if need[6]:
-            into.append(6)
-            problems.append((dxf2, P[:, f1], False))
-        if used and (need[7] or need[9]):
-            into.append(7)
-            problems.append((dz2, P[:, g1], True))
-        if used and need[8]:
-            into.append(8)
-            problems.append((dout2, y.view(M, HD), False))
-        if problems:
-            dw = weight_grads(problems, M)
+        if used and all(need[:10]):
+            (dwcat, _), (grads[6], _), (grads[7], grads[9]), (grads[8], _) = weight_grads(
+                [(dP[:, :N], x2, False), (dxf2, P[:, f1], False), (dz2, P[:, g1], True),
+                 (dout2, y.view(M, HD), False)], M)
+            grads[:6] = dwcat.split(sizes)
+        elif any(need[:10]):
+            runs: List[List[int]] = []   # first column and end of P, first map and end
+            at = 0
+            for i, j, want in ((0, 3, any(need[:3])), (3, 4, need[3]), (4, 5, need[4] and used), (5, 6, need[5])):
+                end = at + (3 * HD if j == 3 else sizes[i])
+                if want and runs and runs[-1][3] == i:
+                    runs[-1][1], runs[-1][3] = end, j
+                elif want:
+                    runs.append([at, end, i, j])
+                at = end
+            problems = [(dP[:, a:b], x2, False) for a, b, _, _ in runs]
+            into = []
+            if need[6]:
+                into.append(6)
+                problems.append((dxf2, P[:, f1], False))
+            if used and (need[7] or need[9]):
+                into.append(7)
+                problems.append((dz2, P[:, g1], True))
+            if used and need[8]:
+                into.append(8)
+                problems.append((dout2, y.view(M, HD), False))
+            dw = weight_grads(problems, M) if problems else []
             for (_, _, i, j), (d, _) in zip(runs, dw):
                 grads[i:j] = d.split(sizes[i:j])
             for m, (d, db) in zip(into, dw[len(runs):]):
