@@ -526,7 +526,7 @@ __global__ __launch_bounds__(4 * D, D == 32 ? 1 : 2) void kda_bwd_localw_kernel(
     if constexpr (STG) tw.store(swu, LDQ);
     __syncthreads();
 
-    // the L2 prefetch (pfp below): after this chunk's last global load, so that
+    // the L2 prefetch (pfp above): after this chunk's last global load, so that
     // no wait of this chunk covers it; waited for at the end
     if (pfp) dma4(pfp, lds_addr(pfbuf));
     if (pfi) dma4(pfi, lds_addr(pfbuf));

@@ -20,9 +20,9 @@
 //     reads them;
 //   - two barriers a step, which leave the loads and stores in flight;
 //   - the backward's two recurrences are independent and share one launch.
-// B2 H6 T1568 D64: forward 117 -> 70 us, state recompute and reverse carry 75 +
-// 129 -> 64 us together; B2 H8 T1568 D128: forward 660 -> 161 us, the other two
-// 151 + 209 -> 135 us.
+// B2 H6 T1568 D64: forward 117 -> 64 us, state recompute and reverse carry 75 +
+// 129 -> 61 us together; B2 H8 T1568 D128: forward 660 -> 141 us, the other two
+// 151 + 209 -> 129 us.
 #include "kda_internal.h"
 
 namespace kda {
