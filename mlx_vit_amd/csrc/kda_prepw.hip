@@ -6,6 +6,8 @@
 // products and solve.  With a chunk's every array in LDS (133 KB, one 16-wave
 // workgroup a CU) each barrier left the CU idle.  At D = 64 two share it as
 // before (the registers' limit), with two phases and their LDS passes fewer.
+// (At D = 128 up to 192 chunks, at most one a CU, stay with the sixteen-wave
+// kernel: PREP16_CHUNKS in kda_fwd.hip.)
 // What is kept out of LDS:
 //   - the in-block cumsums a of g: a thread loads q, k and g of the same (token,
 //     8 channels), so the operands k e^{a}, q e^{a}, k e^{b} form in registers;
